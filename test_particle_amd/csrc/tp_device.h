@@ -903,16 +903,17 @@ __device__ __forceinline__ void get_emf64(const FieldDev &f, double x, double y,
          * parallelism for the FP64 FMA chains), summed in mode order */
         double bx = 0.0, by = 0.0, bz = 0.0;
         const int n4 = f.nmodes & ~3;
+        const tp_cos_pi_consts ck = tp_cos_pi_init();
         /* the table is read-only for the whole kernel: read it through the
          * constant address space so uniform reads become scalar loads */
         typedef const double __attribute__((address_space(4))) *ctab;
         const ctab tab = (ctab)f.modes;
         for (int n = 0; n < n4; n += 4) {
             const ctab m = tab + 7 * n;
-            double c0 = tp_cos_pi(fma(m[2], z, fma(m[1], y, fma(m[0], x, m[6]))));
-            double c1 = tp_cos_pi(fma(m[9], z, fma(m[8], y, fma(m[7], x, m[13]))));
-            double c2 = tp_cos_pi(fma(m[16], z, fma(m[15], y, fma(m[14], x, m[20]))));
-            double c3 = tp_cos_pi(fma(m[23], z, fma(m[22], y, fma(m[21], x, m[27]))));
+            double c0 = tp_cos_pi_with(fma(m[2], z, fma(m[1], y, fma(m[0], x, m[6]))), &ck);
+            double c1 = tp_cos_pi_with(fma(m[9], z, fma(m[8], y, fma(m[7], x, m[13]))), &ck);
+            double c2 = tp_cos_pi_with(fma(m[16], z, fma(m[15], y, fma(m[14], x, m[20]))), &ck);
+            double c3 = tp_cos_pi_with(fma(m[23], z, fma(m[22], y, fma(m[21], x, m[27]))), &ck);
             bx = fma(m[3], c0, bx); by = fma(m[4], c0, by); bz = fma(m[5], c0, bz);
             bx = fma(m[10], c1, bx); by = fma(m[11], c1, by); bz = fma(m[12], c1, bz);
             bx = fma(m[17], c2, bx); by = fma(m[18], c2, by); bz = fma(m[19], c2, bz);
@@ -920,7 +921,7 @@ __device__ __forceinline__ void get_emf64(const FieldDev &f, double x, double y,
         }
         for (int n = n4; n < f.nmodes; n++) {
             const ctab m = tab + 7 * n;
-            double cs = tp_cos_pi(fma(m[2], z, fma(m[1], y, fma(m[0], x, m[6]))));
+            double cs = tp_cos_pi_with(fma(m[2], z, fma(m[1], y, fma(m[0], x, m[6]))), &ck);
             bx = fma(m[3], cs, bx);
             by = fma(m[4], cs, by);
             bz = fma(m[5], cs, bz);

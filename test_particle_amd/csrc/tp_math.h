@@ -28,12 +28,44 @@
 #define TP_MATH_H
 
 #include <math.h>
+#include <stdint.h>
+#include <string.h>
 
 #if defined(__HIPCC__)
 #define TP_HD __host__ __device__ __forceinline__
 #else
 #define TP_HD static inline
 #endif
+
+/* A polynomial coefficient.  On the GPU it is kept in scalar registers (the
+ * empty asm hides its value): otherwise the compiler copies each one into
+ * vector registers in front of a two-operand FMA that overwrites it. */
+TP_HD double tp_const(double c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+s"(c));
+#endif
+    return c;
+}
+
+/* v with its sign flipped if the lowest bit of t is set */
+TP_HD double tp_flip_by_low_bit(double v, double t)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 b = __builtin_bit_cast(u32x2, v);
+    /* adding 2^31 to the high word flips its top bit (one v_lshl_add_u32) */
+    b.y += __builtin_bit_cast(u32x2, t).x << 31;
+    return __builtin_bit_cast(double, b);
+#else
+    uint64_t b, c;
+    memcpy(&b, &v, sizeof(b));
+    memcpy(&c, &t, sizeof(c));
+    b ^= c << 63;
+    memcpy(&v, &b, sizeof(v));
+    return v;
+#endif
+}
 
 #define TP_2_OVER_PI 0x1.45f306dc9c883p-1
 #define TP_PIO2_1    0x1.921fb54442d18p+0
@@ -111,33 +143,66 @@ TP_HD double tp_cos(double x)
 }
 
 /*
- * cos(x) alone, for sums over many modes: reduction by pi instead of pi/2
- * (k = rint(x/pi), r = x - k pi in [-pi/2, pi/2], three-part constant, the
- * first product exact by the same fma argument as above), then one even
- * Taylor polynomial to r^22 (truncation < 4e-20 on that interval) and the
- * sign (-1)^k.  About 40 % fewer operations than tp_sincos.
+ * cos(x) alone, for sums over many modes: reduction by pi instead of pi/2,
+ * then one even Taylor polynomial to r^22 (truncation < 4e-20 on
+ * [-pi/2, pi/2]) and the sign (-1)^k.  Rounding x/pi by adding 1.5 2^52
+ * leaves k = rint(x/pi) in the low bits of the sum, so the sign is its lowest
+ * bit moved to the sign position: one integer operation, where comparing
+ * k/2 with its floor takes five.  r = x - k pi with pi in two parts, the
+ * first product exact by the same fma argument as above (|x| < 2^52); a
+ * third part would move r by less than 2^-57 even there.  17 operations; the
+ * comparison and the third part make it 22 and give the same bits (3e7
+ * arguments in each of |x| < 1.5, 30, 1e3, 1e5, 1e9).
  */
+typedef struct tp_cos_pi_consts {
+    double inv_pi, round, pi_hi, pi_lo, c[10];
+} tp_cos_pi_consts;
+
+/* the constants, to be formed once ahead of a loop over modes */
+TP_HD tp_cos_pi_consts tp_cos_pi_init(void)
+{
+    tp_cos_pi_consts q;
+    q.inv_pi = tp_const(0x1.45f306dc9c883p-2);
+    q.round = 0x1.8p52;
+    q.pi_hi = tp_const(0x1.921fb54442d18p+1);
+    q.pi_lo = tp_const(0x1.1a62633145c07p-53);
+    q.c[0] = tp_const(0x1.0ce396db7f853p-70);               /*  1/22! */
+    q.c[1] = tp_const(-0x1.e542ba4020225p-62);              /* -1/20! */
+    q.c[2] = tp_const(0x1.6827863b97d97p-53);               /*  1/18! */
+    q.c[3] = tp_const(-0x1.ae7f3e733b81fp-45);              /* -1/16! */
+    q.c[4] = tp_const(0x1.93974a8c07c9dp-37);               /*  1/14! */
+    q.c[5] = tp_const(-0x1.1eed8eff8d898p-29);              /* -1/12! */
+    q.c[6] = tp_const(0x1.27e4fb7789f5cp-22);               /*  1/10! */
+    q.c[7] = tp_const(-0x1.a01a01a01a01ap-16);              /* -1/8!  */
+    q.c[8] = tp_const(0x1.6c16c16c16c17p-10);               /*  1/6!  */
+    q.c[9] = tp_const(-0x1.5555555555555p-5);               /* -1/4!  */
+    return q;
+}
+
+TP_HD double tp_cos_pi_with(double x, const tp_cos_pi_consts *q)
+{
+    const double t = fma(x, q->inv_pi, q->round);
+    const double k = t - q->round;
+    double r = fma(-k, q->pi_hi, x);                        /* exact */
+    r = fma(-k, q->pi_lo, r);
+    const double z = r * r;
+    double p = fma(q->c[0], z, q->c[1]);
+    p = fma(p, z, q->c[2]);
+    p = fma(p, z, q->c[3]);
+    p = fma(p, z, q->c[4]);
+    p = fma(p, z, q->c[5]);
+    p = fma(p, z, q->c[6]);
+    p = fma(p, z, q->c[7]);
+    p = fma(p, z, q->c[8]);
+    p = fma(p, z, q->c[9]);
+    p = fma(p, z, 0.5);
+    return tp_flip_by_low_bit(fma(-z, p, 1.0), t);  /* 1 - z/2 + z^2/24 - ... */
+}
+
 TP_HD double tp_cos_pi(double x)
 {
-    double k = rint(x * 0x1.45f306dc9c883p-2);             /* 1/pi */
-    double r = fma(-k, 0x1.921fb54442d18p+1, x);            /* exact */
-    r = fma(-k, 0x1.1a62633145c07p-53, r);
-    r = fma(-k, -0x1.f1976b7ed8fbcp-109, r);
-    double z = r * r;
-    double p = 0x1.0ce396db7f853p-70;                       /*  1/22! */
-    p = fma(p, z, -0x1.e542ba4020225p-62);                  /* -1/20! */
-    p = fma(p, z, 0x1.6827863b97d97p-53);                   /*  1/18! */
-    p = fma(p, z, -0x1.ae7f3e733b81fp-45);                  /* -1/16! */
-    p = fma(p, z, 0x1.93974a8c07c9dp-37);                   /*  1/14! */
-    p = fma(p, z, -0x1.1eed8eff8d898p-29);                  /* -1/12! */
-    p = fma(p, z, 0x1.27e4fb7789f5cp-22);                   /*  1/10! */
-    p = fma(p, z, -0x1.a01a01a01a01ap-16);                  /* -1/8!  */
-    p = fma(p, z, 0x1.6c16c16c16c17p-10);                   /*  1/6!  */
-    p = fma(p, z, -0x1.5555555555555p-5);                   /* -1/4!  */
-    p = fma(p, z, 0.5);
-    double c = fma(-z, p, 1.0);                             /* 1 - z/2 + z^2/24 - ... */
-    double half = k * 0.5;
-    return (half == floor(half)) ? c : -c;
+    const tp_cos_pi_consts q = tp_cos_pi_init();
+    return tp_cos_pi_with(x, &q);
 }
 
 /*

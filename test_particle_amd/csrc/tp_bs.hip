@@ -12,8 +12,11 @@
  *    evaluation is the derivative at an accepted point) is a small state
  *    machine, so lanes at different rows and orders still evaluate the field
  *    together and the expensive field sum (1000 cosines for the multi-mode
- *    field) never diverges across a wavefront.  Only the cheap tableau and
- *    controller bookkeeping between evaluations is divergent.
+ *    field) never diverges across a wavefront; the mode sum runs on the
+ *    matrix cores over the active lanes' points only (modes_wave64).  Only
+ *    the tableau and controller bookkeeping between evaluations is divergent;
+ *    its parts are run once an iteration for all lanes that need them, from
+ *    registers.
  *  - The kernel is persistent: a fixed number of waves per compute unit pull
  *    particles from a global work queue.  Lanes whose particle reached its
  *    end time are refilled together: one atomic per wavefront hands out as
@@ -42,17 +45,21 @@
 #define BS_KFAC1 0.8
 #define BS_KFAC2 0.9
 
-enum { PH_INIT = 0, PH_MID = 1, PH_ACCEPT = 2, PH_DROW = 3, PH_PREP = 4 };
+enum { PH_INIT = 0, PH_MID = 1, PH_ACCEPT = 2, PH_DROW = 3, PH_PREP = 4, PH_OUT = 5 };
 
-/* Dense form: a lane whose step was accepted waits (PH_PREP, evaluating a
- * dummy point like an idle lane) until this many lanes of its wavefront
- * wait, or no other lane is busy, and then they form their interpolants
- * together.  prepare_dense is a long chain of per-lane scratch accesses; run
- * for one lane at a time it stalled the whole wavefront at almost every
- * iteration.  Each lane's arithmetic is unchanged (same results). */
-#ifndef BS_PREP_BATCH
-#define BS_PREP_BATCH 16
-#endif
+/* What a lane does at the end of an iteration.  The parts of a step that
+ * several phases lead to are run once there, for all lanes that came to them
+ * (bs_tail), instead of in a copy per phase: one copy of the code, lanes from
+ * different phases in it together, and half the registers. */
+enum { NX_NONE = 0, NX_ACCEPT = 1, NX_START = 2, NX_ATTEMPT = 3, NX_SEQ = 4, NX_FAIL = 5,
+       NX_DONE = 6 };
+
+/* Dense form: a lane whose step was accepted waits (PH_PREP, evaluating no
+ * point, like an idle lane) until a quarter of its wavefront's lanes wait, or
+ * no other lane is busy, and then they form their interpolants together.
+ * prepare_dense is a long chain of per-lane scratch accesses; run for one
+ * lane at a time it stalled the whole wavefront at almost every iteration.
+ * Each lane's arithmetic is unchanged (same results). */
 enum { Q_HEAD = 0, Q_ACC = 1, Q_REJ = 2, Q_RHS = 3, Q_FAIL = 4, Q_N = 8 };
 
 struct BsConsts {
@@ -60,31 +67,33 @@ struct BsConsts {
     int nseq[10], cost[10], ipoint[11];
     double coeff[10][10];
     double errfac[19];
+    double facmin[10];           /* STEPFAC3^(1 / (2k + 1)) */
 };
 
-/* dense output: per lane, in HBM, ysave (9 x 6), fsave (162 x 6: every
- * substep derivative of sequences 0..8, ipoint[9] = 162 rows) and the
- * interpolation coefficients (23 x 6); slot s of lane g at ds[s * nl + g] */
-#define DS_YSAVE 0
-#define DS_FSAVE (9 * BS_N)
-#define DS_DENS (DS_FSAVE + 162 * BS_N)
-#define DS_YV (DS_DENS + (2 * 9 + 5) * BS_N)
-/* largest kmax of the dense form; YV: the values each interpolation order
- * takes from each sequence, for one component at a time ([order][sequence]) */
+/* largest kmax */
 #define BS_KMAX 8
-#define DS_SLOTS (DS_YV + (2 * BS_KMAX - 1) * (BS_KMAX + 1))
+/* dense output: per lane, in HBM, rows of the six components: ysave (9
+ * rows), fsave (162: every substep derivative of sequences 0..8, ipoint[9]
+ * = 162) and the interpolation coefficients (23); row r of lane g at
+ * ds[(r * nl + g) * 6] */
+#define DS_YSAVE 0
+#define DS_FSAVE 9
+#define DS_DENS (DS_FSAVE + 162)
+#define DS_ROWS (DS_DENS + 2 * 9 + 5)
 
 struct BsArgs {
     FieldDev f;
     BsConsts c;
     int n, cap;
+    int lanes;                   /* lanes of a wavefront that take particles */
+    int lds_quads;               /* mode groups copied to LDS (0: none) */
     double qm, rtol, atol, t_end, t_end_gyro, b_ref, h0;
     double *x, *y, *z, *ux, *uy, *uz, *t;
     int *nsteps, *flag;
     unsigned long long *ctr;
     /* the dense form with the fixed-step loop's diagnostics */
-    double *ds;                  /* dense-output scratch, DS_SLOTS per lane */
-    long nl;                     /* lanes of the launch */
+    double *ds;                  /* dense-output scratch, DS_ROWS x 6 per lane */
+    long nl;                     /* lanes of the launch that take particles */
     double dt;                   /* output grid: times t0 + j dt */
     int estep, ei, di, nd, nframes, nbins, nt_out, bc, fix_stale;
     double lo[3], hi[3], logemin, logde;
@@ -132,6 +141,7 @@ static void bs_consts(int kmax, double rtol, int dense, BsConsts *c)
         double e = 0.5 * sqrt(((double)(i + 1)) / ip5);
         for (int j = 0; j <= i; j++) c->errfac[i] *= e / (j + 1);
     }
+    for (int k = 0; k <= kmax; k++) c->facmin[k] = tp_pow(BS_STEPFAC3, 1.0 / (2 * k + 1));
     c->ipoint[0] = 0;
     for (int i = 1; i <= kmax + 1; i++) {
         int njadd = 4 * i - 2;
@@ -172,7 +182,6 @@ struct BsLane {
     /* yv: the last accepted state, which is also the start of the step being
      * attempted (the reference's ysav) */
     double yv[BS_N], ycur[BS_N], dydx[BS_N], ym[BS_N], yn[BS_N];
-    double tab[8][BS_N], hopt[9], work[9];
     int rhs;
     /* dense form: next fsave row, the polynomial's step (start, size), the
      * step-size cap of the interpolation error, the output-time grid (t0,
@@ -183,8 +192,20 @@ struct BsLane {
     double xs[3];
 };
 
-/* slot s of this lane's dense-output scratch */
-#define DSV(a, s) ((a).ds[(size_t)(s) * (a).nl + gl])
+/* The extrapolation tableau of a lane, at constant indices only (bs_end_seq),
+ * and its rows' step sizes and costs, which are indexed by the lane's own row
+ * numbers.  Each is a variable of its own beside BsLane: the compiler keeps a
+ * variable with one such access in private memory as a whole. */
+struct BsTab {
+    double t[BS_KMAX][BS_N];
+};
+
+struct BsCost {
+    double hopt[BS_KMAX + 1], work[BS_KMAX + 1];
+};
+
+/* component i of row r of this lane's dense-output scratch */
+#define DSR(a, r, i) ((a).ds[((size_t)(r) * (a).nl + gl) * BS_N + (i)])
 
 __device__ __forceinline__ double bs_time(const BsArgs &a, const BsLane &L, long j)
 {
@@ -290,9 +311,17 @@ __device__ __forceinline__ void bs_finish(const BsArgs &a, BsLane &L, int failed
     L.pi = -1;
 }
 
-__device__ __forceinline__ void bs_begin_seq(const BsArgs &a, BsLane &L)
+/* step number of row k: bs_consts' nseq */
+template <bool DENSE>
+__device__ __forceinline__ int bs_nseq(int k)
 {
-    L.nstep = a.c.nseq[L.k];
+    return DENSE ? 4 * k + 2 : 2 * (k + 1);
+}
+
+template <bool DENSE>
+__device__ __forceinline__ void bs_begin_seq(BsLane &L)
+{
+    L.nstep = bs_nseq<DENSE>(L.k);
     L.hsub = L.h / L.nstep;
     for (int i = 0; i < BS_N; i++) {
         L.ym[i] = L.yv[i];
@@ -301,20 +330,6 @@ __device__ __forceinline__ void bs_begin_seq(const BsArgs &a, BsLane &L)
     L.xe = L.t + L.hsub;
     L.nn = 1;
     L.phase = PH_MID;
-}
-
-template <bool DENSE>
-__device__ __forceinline__ void bs_begin_attempt(const BsArgs &a, BsLane &L, long gl)
-{
-    L.h = L.hnew;
-    L.reject = 0;
-    if (++L.attempts > a.cap) {
-        bs_finish<DENSE>(a, L, 1, gl);
-        return;
-    }
-    L.k = 0;
-    L.ipt = 0;
-    bs_begin_seq(a, L);
 }
 
 /* one trajectory point of the lane's particle: state y at time t with the
@@ -348,7 +363,7 @@ __device__ __forceinline__ void bs_traj_record(const BsArgs &a, const BsLane &L,
 /* the output times at the end time: the remaining frames from the final
  * state; the remaining D rows each need the field there (PH_DROW) */
 template <bool DENSE>
-__device__ __forceinline__ void bs_begin_end_outputs(const BsArgs &a, BsLane &L, long gl)
+__device__ __forceinline__ int bs_begin_end_outputs(const BsArgs &a, BsLane &L, long gl)
 {
     for (; L.nf < a.nframes; L.nf++)
         atomicAdd(&a.espect[L.nf * a.nbins + bs_energy_bin(a, L.yv[3], L.yv[4], L.yv[5])], 1u);
@@ -359,23 +374,20 @@ __device__ __forceinline__ void bs_begin_end_outputs(const BsArgs &a, BsLane &L,
         for (int i = 0; i < BS_N; i++) L.yn[i] = L.yv[i];
         L.xe = bs_time(a, L, (long)L.nr * a.di);
         L.phase = PH_DROW;
-        return;
+        return NX_NONE;
     }
-    bs_finish<DENSE>(a, L, 0, gl);
+    return NX_DONE;
 }
 
 /* top of step(): src/unused/StepperBS.c:173-191 */
 template <bool DENSE>
-__device__ __forceinline__ void bs_start_step(const BsArgs &a, BsLane &L, long gl)
+__device__ __forceinline__ int bs_start_step(const BsArgs &a, BsLane &L, BsCost &W, long gl)
 {
-    if (!(L.t < L.tend - 1e-13 * fabs(L.tend))) {
-        if (DENSE) bs_begin_end_outputs<DENSE>(a, L, gl);
-        else bs_finish<DENSE>(a, L, 0, gl);
-        return;
-    }
+    if (!(L.t < L.tend - 1e-13 * fabs(L.tend)))
+        return DENSE ? bs_begin_end_outputs<DENSE>(a, L, gl) : NX_DONE;
     double h = L.hnext;
     if (L.t + h > L.tend) h = L.tend - L.t;
-    L.work[0] = 0.0;
+    W.work[0] = 0.0;
     if (h != L.hnext && !L.first) L.last = 1;
     if (L.reject) {
         L.prev_reject = 1;
@@ -383,38 +395,57 @@ __device__ __forceinline__ void bs_start_step(const BsArgs &a, BsLane &L, long g
     }
     L.reject = 0;
     L.hnew = fabs(h);
-    bs_begin_attempt<DENSE>(a, L, gl);
+    return NX_ATTEMPT;
 }
 
 /* after row k's midpoint sequence: extrapolation, error and the
- * convergence/rejection tests of src/unused/StepperBS.c:206-272 */
+ * convergence/rejection tests of src/unused/StepperBS.c:206-272.  The
+ * tableau is read at once, updated at constant indices (rows a lane does not
+ * have keep their values) and written back: one wait for private memory
+ * instead of one per element.  C: the constants in LDS, indexed by the
+ * lane's own k. */
 template <bool DENSE>
-__device__ __forceinline__ void bs_end_seq(const BsArgs &a, BsLane &L, const double *yseq,
-                                           long gl)
+__device__ __forceinline__ int bs_end_seq(const BsArgs &a, const BsConsts &C, BsLane &L,
+                                          BsTab &T, BsCost &W, const double *yseq)
 {
     const int k = L.k;
     if (k == 0) {
+#pragma unroll
         for (int i = 0; i < BS_N; i++) L.ycur[i] = yseq[i];
         L.k = 1;
-        bs_begin_seq(a, L);
-        return;
+        return NX_SEQ;
     }
-    for (int i = 0; i < BS_N; i++) L.tab[k - 1][i] = yseq[i];
-    for (int j = k - 1; j > 0; j--)
-        for (int i = 0; i < BS_N; i++)
-            L.tab[j - 1][i] = L.tab[j][i] + a.c.coeff[k][j] * (L.tab[j][i] - L.tab[j - 1][i]);
-    for (int i = 0; i < BS_N; i++)
-        L.ycur[i] = L.tab[0][i] + a.c.coeff[k][0] * (L.tab[0][i] - L.ycur[i]);
+    /* the lane's coefficients; rows from k - 1 on take no part */
+    double cf[BS_KMAX], d[BS_N];
+#pragma unroll
+    for (int j = 0; j < BS_KMAX; j++) cf[j] = C.coeff[k][j];
+#pragma unroll
+    for (int i = 0; i < BS_N; i++) {
+        double t[BS_KMAX];
+#pragma unroll
+        for (int r = 0; r < BS_KMAX; r++) t[r] = r == k - 1 ? yseq[i] : T.t[r][i];
+#pragma unroll
+        for (int j = BS_KMAX - 1; j > 0; j--) {
+            const double v = t[j] + cf[j] * (t[j] - t[j - 1]);
+            t[j - 1] = j <= k - 1 ? v : t[j - 1];
+        }
+#pragma unroll
+        for (int r = 0; r < BS_KMAX; r++) T.t[r][i] = t[r];
+        L.ycur[i] = t[0] + cf[0] * (t[0] - L.ycur[i]);
+        d[i] = L.ycur[i] - t[0];
+        if (i % 2) __builtin_amdgcn_sched_barrier(0);
+    }
     double err = 0.0;
+#pragma unroll
     for (int i = 0; i < BS_N; i++) {
         double p = fabs(L.yv[i]), q = fabs(L.ycur[i]);
         double scale = a.atol + a.rtol * (p > q ? p : q);
-        double r = (L.ycur[i] - L.tab[0][i]) / scale;
+        double r = d[i] / scale;
         err += r * r;
     }
     err = sqrt(err / BS_N);
     double expo = 1.0 / (2 * k + 1);
-    double facmin = tp_pow(BS_STEPFAC3, expo);
+    double facmin = C.facmin[k];
     double fac;
     if (err == 0.0) {
         fac = 1.0 / facmin;
@@ -424,21 +455,24 @@ __device__ __forceinline__ void bs_end_seq(const BsArgs &a, BsLane &L, const dou
         fac = fac < hi ? fac : hi;
         fac = lo > fac ? lo : fac;
     }
-    L.hopt[k] = fabs(L.h * fac);
-    L.work[k] = a.c.cost[k] / L.hopt[k];
+    const double hk = fabs(L.h * fac), wk = C.cost[k] / hk;
+    W.hopt[k] = hk;
+    W.work[k] = wk;
     bool brk = false;
+    /* every rejection below lowers ktarg (to k, or to itself) by one more
+     * when the row before cost less, and takes that row's step size */
+    bool rej = false;
+    int kt = L.ktarg;
     if ((L.first || L.last) && err <= 1.0) brk = true;
     if (!brk && k == L.ktarg - 1 && !L.prev_reject && !L.first && !L.last) {
         if (err <= 1.0) {
             brk = true;
         } else {
-            double r = (double)(a.c.nseq[L.ktarg] * a.c.nseq[L.ktarg + 1] /
-                                (a.c.nseq[0] * a.c.nseq[0]));
+            double r = (double)(bs_nseq<DENSE>(L.ktarg) * bs_nseq<DENSE>(L.ktarg + 1) /
+                                (bs_nseq<DENSE>(0) * bs_nseq<DENSE>(0)));
             if (err > r * r) {
-                L.reject = 1;
-                L.ktarg = k;
-                if (L.ktarg > 1 && L.work[k - 1] < BS_KFAC1 * L.work[k]) L.ktarg--;
-                L.hnew = L.hopt[L.ktarg];
+                rej = true;
+                kt = k;
                 brk = true;
             }
         }
@@ -447,268 +481,290 @@ __device__ __forceinline__ void bs_end_seq(const BsArgs &a, BsLane &L, const dou
         if (err <= 1.0) {
             brk = true;
         } else {
-            double r = (double)a.c.nseq[k + 1] / a.c.nseq[0];
+            double r = (double)bs_nseq<DENSE>(k + 1) / bs_nseq<DENSE>(0);
             if (err > r * r) {
-                L.reject = 1;
-                if (L.ktarg > 1 && L.work[k - 1] < BS_KFAC1 * L.work[k]) L.ktarg--;
-                L.hnew = L.hopt[L.ktarg];
+                rej = true;
                 brk = true;
             }
         }
     }
     if (!brk && k == L.ktarg + 1) {
-        if (err > 1.0) {
-            L.reject = 1;
-            if (L.ktarg > 1 && L.work[L.ktarg - 1] < BS_KFAC1 * L.work[L.ktarg]) L.ktarg--;
-            L.hnew = L.hopt[L.ktarg];
-        }
+        if (err > 1.0) rej = true;
         brk = true;
     }
     if (!brk) {
         L.k = k + 1;
-        bs_begin_seq(a, L);
-        return;
+        return NX_SEQ;
     }
-    if (L.reject) {
+    if (rej) {
+        /* kt is k or ktarg: at k = ktarg + 1 the rows compared are ktarg - 1
+         * and ktarg, otherwise k - 1 and k */
+        if (kt > 1 && W.work[kt - 1] < BS_KFAC1 * W.work[kt]) kt--;
+        L.ktarg = kt;
+        L.hnew = W.hopt[kt];
+        L.reject = 1;
         L.prev_reject = 1;
         L.rej++;
-        bs_begin_attempt<DENSE>(a, L, gl);
-        return;
+        return NX_ATTEMPT;
     }
     /* accepted: the derivative at the new point comes next */
     L.xe = L.t + L.h;
     L.phase = PH_ACCEPT;
+    return NX_NONE;
 }
 
-/* dense_interp, src/unused/StepperBS.c:478-524, on the lane's dens slots;
- * the coefficient array is indexed by compile-time orders (unrolled up to
- * 2 BS_KMAX - 1) so that it stays in registers */
-__device__ __forceinline__ void bs_dense_interp(const BsArgs &a, long gl, int imit)
+/* ------------------------------------------------------------------ */
+/* dense output: a lane per component                                   */
+/* ------------------------------------------------------------------ */
+/* prepare_dense (src/unused/StepperBS.c:526-615) treats the six components
+ * of a step separately, so a wavefront forms the interpolants of up to
+ * BS_PREP steps at once with lane 6 p + i on component i of the p-th.  The
+ * reference updates its ysave and fsave arrays in place, order by order; here
+ * a component goes through the same operations in registers, a sequence KK at
+ * a time: its rows are read together, their differences formed order by
+ * order, and each order's value (times (n_KK / 2)^(order - 1)) enters that
+ * order's extrapolation as soon as it is known:
+ *   y[l-1] = y[l] + (y[l] - y[l-1]) / ((n_KK / n_{l-1})^2 - 1), l = KK..KB+1,
+ * KB = (order - 1) / 2 (src/unused/StepperBS.c:545-553, 564-572).  Same
+ * operations on the same operands: the oracle's bits.
+ * Bound: k + 2 waits for the scratch rows (from HBM) and the chain of
+ * divisions.  A lane per step, with the values of an order passing through
+ * scratch, took 367,000 cycles for the 8 steps of a batch (30,000 particles,
+ * 200 modes, one wavefront per SIMD); a lane per component takes 48,000. */
+#define BS_PREP 10
+#define BS_PREP_IN (4 * BS_N + 1)    /* doubles a lane hands over: y, y', ends, h */
+
+/* n / d - n and d the sequences' step numbers, known at compile time */
+template <int J, int L1>
+struct BsFactor {
+    static __device__ __forceinline__ double get()
+    {
+        const double r = (double)(4 * J + 2) / (double)(4 * L1 + 2);
+        return r * r - 1.0;
+    }
+};
+
+/* y[KB .. J-1] extrapolated with sequence J's value v */
+template <int KB, int J, int LL>
+__device__ __forceinline__ void bs_extrap_step(double (&y)[BS_KMAX + 1])
 {
-    const int n = BS_N;
-    for (int i = 0; i < n; i++) {
-        double y0 = DSV(a, DS_DENS + i), y1 = DSV(a, DS_DENS + 2 * n + i);
-        double yp0 = DSV(a, DS_DENS + n + i), yp1 = DSV(a, DS_DENS + 3 * n + i);
-        double ydiff = y1 - y0;
-        double aspl = -yp1 + ydiff;
-        double bspl = yp0 - ydiff;
-        DSV(a, DS_DENS + n + i) = ydiff;
-        DSV(a, DS_DENS + 2 * n + i) = aspl;
-        DSV(a, DS_DENS + 3 * n + i) = bspl;
-        if (imit < 0) continue;
-        double ph0 = (y0 + y1) * 0.5 + 0.125 * (aspl + bspl);
-        double ph1 = ydiff + (aspl - bspl) * 0.25;
-        double ph2 = -(yp0 - yp1);
-        double ph3 = 6.0 * (bspl - aspl);
-        double av[2 * BS_KMAX];
-        if (imit >= 1) {
-            av[1] = 16.0 * (DSV(a, DS_DENS + 5 * n + i) - ph1);
-            if (imit >= 3) {
-                av[3] = 16.0 * (DSV(a, DS_DENS + 7 * n + i) - ph3 + 3 * av[1]);
-#pragma unroll
-                for (int im = 5; im <= 2 * BS_KMAX - 1; im += 2) {
-                    if (im > imit) break;
-                    double fac1 = im * (im - 1) / 2.0;
-                    double fac2 = fac1 * (im - 2) * (im - 3) * 2.0;
-                    av[im] = 16.0 * (DSV(a, DS_DENS + (im + 4) * n + i) + fac1 * av[im - 2] -
-                                     fac2 * av[im - 4]);
-                }
-            }
-        }
-        av[0] = (DSV(a, DS_DENS + 4 * n + i) - ph0) * 16.0;
-        if (imit >= 2) {
-            av[2] = (DSV(a, DS_DENS + 6 * n + i) - ph2 + av[0]) * 16.0;
-#pragma unroll
-            for (int im = 4; im <= 2 * BS_KMAX - 1; im += 2) {
-                if (im > imit) break;
-                double fac1 = im * (im - 1) / 2.0;
-                double fac2 = (double)(im * (im - 1) * (im - 2) * (im - 3));
-                av[im] = 16.0 * (DSV(a, DS_DENS + (im + 4) * n + i) + fac1 * av[im - 2] -
-                                 fac2 * av[im - 4]);
-            }
-        }
-#pragma unroll
-        for (int im = 0; im <= 2 * BS_KMAX - 1; im++) {
-            if (im > imit) break;
-            DSV(a, DS_DENS + n * (im + 4) + i) = av[im];
-        }
+    if constexpr (LL >= KB + 1) {
+        y[LL - 1] = y[LL] + (y[LL] - y[LL - 1]) / BsFactor<J, LL - 1>::get();
+        bs_extrap_step<KB, J, LL - 1>(y);
     }
 }
 
-/* prepare_dense's polynomial extrapolation over sequences KB..k of one
- * component held in y: y[l-1] = y[l] + (y[l] - y[l-1]) / (r^2 - 1), r =
- * n_j / n_{l-1}, for j = KB+1..k and l = j..KB+1 (src/unused/StepperBS.c:
- * 545-553 and 564-572); returns y[KB] */
-template <int KB>
-__device__ __forceinline__ double bs_dense_extrap(const BsArgs &a, double (&y)[BS_KMAX + 1],
-                                                  int k)
+template <int KB, int J>
+__device__ __forceinline__ void bs_extrap(double (&y)[BS_KMAX + 1], double v)
 {
-#pragma unroll
-    for (int j = KB + 1; j <= BS_KMAX; j++) {
-        if (j > k) break;
-        double dblenj = a.c.nseq[j];
-#pragma unroll
-        for (int l = j; l >= KB + 1; l--) {
-            double r = dblenj / a.c.nseq[l - 1];
-            double factor = r * r - 1.0;
-            y[l - 1] = y[l] + (y[l] - y[l - 1]) / factor;
-        }
-    }
-    return y[KB];
+    y[J] = v;
+    bs_extrap_step<KB, J, J>(y);
 }
 
-/* sequence KK's derivative rows of component i (rows 2 KK^2 .. 2 (KK+1)^2 - 1
- * of fsave: ipoint[kk] = 2 kk^2 for nseq = 4k + 2) in registers, order by
- * order: the value order KMI takes from them (times (n_KK/2)^(KMI-1)) goes to
- * YV, then the differences prepare_dense takes between orders
- * (src/unused/StepperBS.c:558-601), element by element in its order.  Each
- * difference pairs rows two apart, so the rows at odd and at even offsets
- * in the sequence evolve separately: P selects one half (offset o is held
- * in row[o / 2]), which halves the registers held. */
-template <int KK, int P, int KMI>
-__device__ __forceinline__ void bs_dense_orders(const BsArgs &a, long gl, int mu, double dydx_i,
-                                                double (&row)[2 * KK + 1])
+constexpr double bs_const_pow(double x, int e)
 {
-    if constexpr (KMI <= 2 * BS_KMAX - 1) {
-        constexpr int R = 4 * KK + 2;
+    double r = 1.0;
+    for (int i = 0; i < e; i++) r = r * x;
+    return r;
+}
+
+/* sequence KK's derivative rows (offsets o in the sequence; row 0 of the
+ * sequence is row 2 KK^2 of fsave, ipoint for nseq = 4k + 2), from order KMI
+ * on: the value order KMI takes, then the differences between orders
+ * (src/unused/StepperBS.c:558-601) */
+template <int KK, int KMI>
+__device__ __forceinline__ void bs_dense_orders(int mu, double dydx_i, double (&row)[4 * KK + 2],
+                                                double (&Y)[2 * BS_KMAX][BS_KMAX + 1])
+{
+    constexpr int R = 4 * KK + 2, KB = (KMI - 1) / 2;
+    if constexpr (KMI <= 2 * BS_KMAX - 1 && KK >= KB) {
         if (KMI > mu) return;
-        if constexpr (KK >= (KMI - 1) / 2 && (2 * KK + KMI - 1) % 2 == P)
-            DSV(a, DS_YV + (KMI - 1) * (BS_KMAX + 1) + KK) =
-                row[(2 * KK + KMI - 1) / 2] * tp_powi(a.c.nseq[KK] / 2.0, KMI - 1);
+        constexpr double scale = bs_const_pow((4 * KK + 2) / 2.0, KMI - 1);
+        bs_extrap<KB, KK>(Y[KMI], row[2 * KK + KMI - 1] * scale);
         if (KMI == mu) return;
         if constexpr (KK >= KMI / 2) {
-            if constexpr (P == 1) {
 #pragma unroll
-                for (int o = R - 1; o >= (KMI == 1 ? 3 : KMI); o -= 2)
-                    row[o / 2] = row[o / 2] - row[(o - 2) / 2];
-                if constexpr (KMI == 1) row[0] = row[0] - dydx_i;    /* offset 1 */
-            } else {
-#pragma unroll
-                for (int o = R - 2; o >= KMI + 1; o -= 2)
-                    row[o / 2] = row[o / 2] - row[(o - 2) / 2];
-            }
+            for (int o = R - 1; o >= (KMI == 1 ? 2 : KMI); o--) row[o] = row[o] - row[o - 2];
+            if constexpr (KMI == 1) row[1] = row[1] - dydx_i;
         }
-        bs_dense_orders<KK, P, KMI + 1>(a, gl, mu, dydx_i, row);
+        bs_dense_orders<KK, KMI + 1>(mu, dydx_i, row, Y);
     }
 }
 
 template <int KK>
-__device__ __forceinline__ void bs_dense_seq(const BsArgs &a, long gl, int i, int k, int mu,
-                                             double dydx_i)
+__device__ __forceinline__ void bs_dense_seqs(const BsArgs &a, long gl, int i, int k, int mu,
+                                              double dydx_i,
+                                              double (&Y)[2 * BS_KMAX][BS_KMAX + 1])
 {
     if constexpr (KK <= BS_KMAX) {
         if (KK <= k) {
-            constexpr int R0 = 2 * KK * KK;
+            double row[4 * KK + 2];
+            const double ys = DSR(a, DS_YSAVE + KK, i);
 #pragma unroll
-            for (int P = 0; P < 2; P++) {
-                double row[2 * KK + 1];
+            for (int o = 0; o < 4 * KK + 2; o++) row[o] = DSR(a, DS_FSAVE + 2 * KK * KK + o, i);
+            bs_extrap<0, KK>(Y[0], ys);
+            bs_dense_orders<KK, 1>(mu, dydx_i, row, Y);
+            bs_dense_seqs<KK + 1>(a, gl, i, k, mu, dydx_i, Y);
+        }
+    }
+}
+
+/* component i of a step of size h with ends y0, y1 and derivatives yp0, yp1
+ * there (times h): prepare_dense and dense_interp (src/unused/StepperBS.c:
+ * 478-524) into the lane's dens rows; returns the last coefficient, which
+ * estimates the interpolation error */
+__device__ __forceinline__ double bs_dense_component(const BsArgs &a, long gl, int i, int k,
+                                                     double h, double y0, double y1, double f0,
+                                                     double f1)
+{
+    const int mu = 2 * k - 1;
+    double Y[2 * BS_KMAX][BS_KMAX + 1];
+    bs_dense_seqs<0>(a, gl, i, k, mu, f0, Y);
+    const double yp0 = h * f0, yp1 = f1 * h;
+    const double ydiff = y1 - y0;
+    const double aspl = -yp1 + ydiff;
+    const double bspl = yp0 - ydiff;
+    DSR(a, DS_DENS + 0, i) = y0;
+    DSR(a, DS_DENS + 1, i) = ydiff;
+    DSR(a, DS_DENS + 2, i) = aspl;
+    DSR(a, DS_DENS + 3, i) = bspl;
+    const double ph0 = (y0 + y1) * 0.5 + 0.125 * (aspl + bspl);
+    const double ph1 = ydiff + (aspl - bspl) * 0.25;
+    const double ph2 = -(yp0 - yp1);
+    const double ph3 = 6.0 * (bspl - aspl);
+    /* order m's coefficient before dense_interp: Y[m][KB] h */
+    double av[2 * BS_KMAX];
+    av[0] = (Y[0][0] - ph0) * 16.0;
+    double last = av[0];
+    DSR(a, DS_DENS + 4, i) = av[0];
 #pragma unroll
-                for (int q = 0; q < 2 * KK + 1; q++)
-                    row[q] = DSV(a, DS_FSAVE + (R0 + 2 * q + P) * BS_N + i);
-                if (P == 0) bs_dense_orders<KK, 0, 1>(a, gl, mu, dydx_i, row);
-                else bs_dense_orders<KK, 1, 1>(a, gl, mu, dydx_i, row);
+    for (int im = 1; im <= 2 * BS_KMAX - 1; im++) {
+        if (im <= mu) {
+            const double d = Y[im][(im - 1) / 2] * h;
+            if (im == 1) {
+                av[1] = 16.0 * (d - ph1);
+            } else if (im == 2) {
+                av[2] = (d - ph2 + av[0]) * 16.0;
+            } else if (im == 3) {
+                av[3] = 16.0 * (d - ph3 + 3 * av[1]);
+            } else {
+                const double fac1 = im * (im - 1) / 2.0;
+                const double fac2 = im % 2 ? fac1 * (im - 2) * (im - 3) * 2.0
+                                           : (double)(im * (im - 1) * (im - 2) * (im - 3));
+                av[im] = 16.0 * (d + fac1 * av[im - 2] - fac2 * av[im - 4]);
+            }
+            DSR(a, DS_DENS + im + 4, i) = av[im];
+            last = av[im];
+        }
+    }
+    return last;
+}
+
+/* The interpolants of the lanes with `pend`, whose steps were accepted with
+ * the derivatives dydxnew in ym; every lane of the wavefront calls it.  Returns
+ * the interpolation error estimate of the lane's own step.  xp: the
+ * wavefront's MODES_WAVE_LDS doubles of LDS. */
+__device__ __forceinline__ double bs_prepare_dense(const BsArgs &a, const BsConsts &C,
+                                                   const BsLane &L, bool pend, long gl,
+                                                   double *xp)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned long long mask = __ballot(pend);
+    const int total = __popcll(mask);
+    const int rank = __popcll(mask & ((1ull << lane) - 1ull));
+    double error = 0.0;
+    for (int base = 0; base < total; base += BS_PREP) {
+        const int cnt = total - base < BS_PREP ? total - base : BS_PREP;
+        const bool mine = pend && rank >= base && rank < base + BS_PREP;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        if (mine) {
+            double *o = xp + BS_PREP_IN * (rank - base);
+#pragma unroll
+            for (int i = 0; i < BS_N; i++) {
+                o[i] = L.yv[i];
+                o[BS_N + i] = L.ycur[i];
+                o[2 * BS_N + i] = L.dydx[i];
+                o[3 * BS_N + i] = L.ym[i];
+            }
+            o[4 * BS_N] = L.h;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        /* the lane of the p-th step of this batch */
+        const int p = lane / BS_N, i = lane - BS_N * p;
+        int src = 0;
+        {
+            unsigned long long m = mask;
+            for (int q = 0; q < base; q++) m &= m - 1;
+            for (int q = 0; q < BS_PREP; q++) {
+                if (q == p) src = __ffsll((long long)m) - 1;
+                m &= m - 1;
             }
         }
-        bs_dense_seq<KK + 1>(a, gl, i, k, mu, dydx_i);
-    }
-}
-
-/* order KMI's dens coefficient of component i: the extrapolation of its
- * values over sequences (KMI-1)/2 .. k */
-template <int KMI>
-__device__ __forceinline__ void bs_dense_coeffs(const BsArgs &a, long gl, int i, int k, int mu,
-                                                double h)
-{
-    if constexpr (KMI <= 2 * BS_KMAX - 1) {
-        if (KMI > mu) return;
-        constexpr int KB = (KMI - 1) / 2;
-        double y[BS_KMAX + 1];
+        const bool work = p < cnt;
+        src = work ? src : 0;
+        const int k = __shfl(L.k, src, 64);
+        double v2 = 0.0;
+        if (work) {
+            const double *o = xp + BS_PREP_IN * p;
+            const double y0 = o[i], y1 = o[BS_N + i];
+            const double v = bs_dense_component(a, gl - lane + src, i, k, o[4 * BS_N], y0, y1,
+                                                o[2 * BS_N + i], o[3 * BS_N + i]);
+            const double q0 = fabs(y0), q1 = fabs(y1);
+            const double scale = a.atol + a.rtol * (q0 > q1 ? q0 : q1);
+            const double r = v / scale;
+            v2 = r * r;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        if (work) xp[lane] = v2;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        if (mine) {
+            double e = 0.0;
 #pragma unroll
-        for (int kk = KB; kk <= BS_KMAX; kk++) {
-            if (kk > k) break;
-            y[kk] = DSV(a, DS_YV + (KMI - 1) * (BS_KMAX + 1) + kk);
+            for (int q = 0; q < BS_N; q++) e += xp[BS_N * (rank - base) + q];
+            const int mu = 2 * L.k - 1;
+            error = mu >= 1 ? sqrt(e / BS_N) * C.errfac[mu - 1] : 0.0;
         }
-        DSV(a, DS_DENS + (KMI + 4) * BS_N + i) = bs_dense_extrap<KB>(a, y, k) * h;
-        bs_dense_coeffs<KMI + 1>(a, gl, i, k, mu, h);
-    }
-}
-
-/* prepare_dense, src/unused/StepperBS.c:526-615: the dense-output values of
- * the accepted step of size h (start yv, end ycur, derivatives dydx and
- * dydxnew), extrapolated from the midpoint values and derivative differences
- * of sequences 0..k; returns the interpolation error estimate.  The
- * reference updates its ysave and fsave arrays in place order by order;
- * here each component's values go through the same operations in
- * registers, a sequence at a time, and the values each order needs pass
- * through the YV slots: the same results with a few hundred scratch
- * accesses per step instead of thousands of dependent ones. */
-__device__ __forceinline__ double bs_prepare_dense(const BsArgs &a, const BsLane &L, long gl,
-                                                   const double *dydxnew)
-{
-    const int n = BS_N, k = L.k, mu = 2 * k - 1;
-    const double h = L.h;
-    for (int i = 0; i < n; i++) {
-        DSV(a, DS_DENS + i) = L.yv[i];
-        DSV(a, DS_DENS + n + i) = h * L.dydx[i];
-        DSV(a, DS_DENS + 2 * n + i) = L.ycur[i];
-        DSV(a, DS_DENS + 3 * n + i) = dydxnew[i] * h;
-    }
-    for (int i = 0; i < n; i++) {
-        /* the midpoint values, extrapolated */
-        double y[BS_KMAX + 1];
-#pragma unroll
-        for (int kk = 0; kk <= BS_KMAX; kk++) {
-            if (kk > k) break;
-            y[kk] = DSV(a, DS_YSAVE + kk * BS_N + i);
-        }
-        DSV(a, DS_DENS + 4 * n + i) = bs_dense_extrap<0>(a, y, k);
-        /* the derivative differences, order by order */
-        bs_dense_seq<0>(a, gl, i, k, mu, L.dydx[i]);
-        bs_dense_coeffs<1>(a, gl, i, k, mu, h);
-    }
-    bs_dense_interp(a, gl, mu);
-    double error = 0.0;
-    if (mu >= 1) {
-        for (int i = 0; i < n; i++) {
-            double p = fabs(L.yv[i]), q = fabs(L.ycur[i]);
-            double scale = a.atol + a.rtol * (p > q ? p : q);
-            double v = DSV(a, DS_DENS + (mu + 4) * n + i) / scale;
-            error += v * v;
-        }
-        error = sqrt(error / n) * a.c.errfac[mu - 1];
     }
     return error;
 }
 
 /* dense_out, src/unused/StepperBS.c:617-644: component i at time x of the
- * lane's last accepted step */
+ * lane's last accepted step (its rows read together) */
 __device__ __forceinline__ double bs_dense_out(const BsArgs &a, const BsLane &L, long gl, int i,
                                                double x)
 {
-    const int n = BS_N, mu = 2 * L.k - 1;
+    const int mu = 2 * L.k - 1;
+    double d[2 * BS_KMAX + 4];
+#pragma unroll
+    for (int r = 0; r < 2 * BS_KMAX + 4; r++) d[r] = DSR(a, DS_DENS + r, i);
     double theta = (x - L.told) / L.hd;
     double theta1 = 1.0 - theta;
-    double yinterp = DSV(a, DS_DENS + i) +
-                     theta * (DSV(a, DS_DENS + n + i) +
-                              theta1 * (DSV(a, DS_DENS + 2 * n + i) * theta +
-                                        DSV(a, DS_DENS + 3 * n + i) * theta1));
+    double yinterp = d[0] + theta * (d[1] + theta1 * (d[2] * theta + d[3] * theta1));
     if (mu < 0) return yinterp;
     double theta05 = theta - 0.5;
     double tt = theta * theta1;
     double t4 = tt * tt;
-    double cc = DSV(a, DS_DENS + n * (mu + 4) + i);
-    for (int j = mu; j > 0; j--) cc = DSV(a, DS_DENS + n * (j + 3) + i) + cc * theta05 / j;
+    double cc = 0.0;
+#pragma unroll
+    for (int j = 2 * BS_KMAX - 1; j >= 0; j--) {
+        if (j == mu) cc = d[j + 4];
+        if (j < mu) cc = d[j + 4] + cc * theta05 / (j + 1);
+    }
     return yinterp + t4 * cc;
 }
 
 /* the step's own output times (strictly before its end) next: a D row
  * needs the field at its point, evaluated in the next iteration */
-template <bool DENSE>
 __device__ __forceinline__ bool bs_next_drow(const BsArgs &a, BsLane &L, long gl)
 {
     if (L.nr >= a.nd) return false;
     const double tr = bs_time(a, L, (long)L.nr * a.di);
     if (!(tr < L.told + L.hd)) return false;
+#pragma unroll
     for (int i = 0; i < BS_N; i++) L.yn[i] = bs_dense_out(a, L, gl, i, tr);
     L.xe = tr;
     L.phase = PH_DROW;
@@ -719,151 +775,159 @@ __device__ __forceinline__ bool bs_next_drow(const BsArgs &a, BsLane &L, long gl
  * order and step-size choice of src/unused/StepperBS.c:296-347, then (dense
  * form) the boundary and the escape */
 template <bool DENSE>
-__device__ __forceinline__ void bs_accept_finish(const BsArgs &a, BsLane &L, const double *f,
-                                                 long gl)
+__device__ __forceinline__ int bs_accept_finish(const BsArgs &a, const BsConsts &C, BsLane &L,
+                                                const BsCost &W)
 {
+#pragma unroll
     for (int i = 0; i < BS_N; i++) {
-        L.dydx[i] = f[i];
+        L.dydx[i] = L.ym[i];
         L.yv[i] = L.ycur[i];
     }
     L.t += L.h;
     L.first = 0;
     L.acc++;
-    const int k = L.k, KM1 = a.c.kmax - 1;
+    const int k = L.k, KM1 = C.kmax - 1;
+    const double wk = W.work[k], wk1 = W.work[k - 1];
     int kopt;
     if (k == 1) {
         kopt = 2;
     } else if (k <= L.ktarg) {
         kopt = k;
-        if (L.work[k - 1] < BS_KFAC1 * L.work[k]) kopt = k - 1;
-        else if (L.work[k] < BS_KFAC2 * L.work[k - 1]) kopt = (k + 1 < KM1) ? k + 1 : KM1;
+        if (wk1 < BS_KFAC1 * wk) kopt = k - 1;
+        else if (wk < BS_KFAC2 * wk1) kopt = (k + 1 < KM1) ? k + 1 : KM1;
     } else {
         kopt = k - 1;
-        if (k > 2 && L.work[k - 2] < BS_KFAC1 * L.work[k - 1]) kopt = k - 2;
-        if (L.work[k] < BS_KFAC2 * L.work[kopt]) kopt = (k < KM1) ? k : KM1;
+        if (k > 2 && W.work[k - 2] < BS_KFAC1 * wk1) kopt = k - 2;
+        if (wk < BS_KFAC2 * W.work[kopt]) kopt = (k < KM1) ? k : KM1;
     }
     double hnew;
     if (L.prev_reject) {
         L.ktarg = kopt < k ? kopt : k;
-        double p = fabs(L.h), q = L.hopt[L.ktarg];
+        double p = fabs(L.h), q = W.hopt[L.ktarg];
         hnew = p < q ? p : q;
         L.prev_reject = 0;
     } else {
         if (kopt <= k) {
-            hnew = L.hopt[kopt];
+            hnew = W.hopt[kopt];
         } else {
-            if (k < L.ktarg && L.work[k] < BS_KFAC2 * L.work[k - 1])
-                hnew = L.hopt[k] * a.c.cost[kopt + 1] / a.c.cost[k];
-            else
-                hnew = L.hopt[k] * a.c.cost[kopt] / a.c.cost[k];
+            const int num = k < L.ktarg && wk < BS_KFAC2 * wk1 ? kopt + 1 : kopt;
+            hnew = W.hopt[k] * C.cost[num] / C.cost[k];
         }
         L.ktarg = kopt;
     }
+    L.hnext = hnew;
     if (DENSE) {
         double hi = fabs(L.hopt_int);
-        hnew = hnew < hi ? hnew : hi;
-        L.hnext = hnew;
+        L.hnext = hnew < hi ? hnew : hi;
         bs_particle_bc(a, L);
         if (L.esc) {
             /* escape spectrum at the frame of the next output time */
             if (L.nf < a.nt_out)
                 atomicAdd(&a.espect_esc[L.nf * a.nbins +
                                         bs_energy_bin(a, L.yv[3], L.yv[4], L.yv[5])], 1u);
-            bs_finish<DENSE>(a, L, 0, gl);
-            return;
+            return NX_DONE;
         }
-        bs_start_step<DENSE>(a, L, gl);
-        return;
     }
-    L.hnext = hnew;
-    bs_start_step<DENSE>(a, L, gl);
+    return NX_START;
 }
 
-/* after the derivative at the accepted point: the dense form first checks
- * the interpolation error (above 10 the step is redone with the step size
- * it suggests), bins the frames inside the step and queues its D rows */
-template <bool DENSE>
-__device__ __forceinline__ void bs_accept(const BsArgs &a, BsLane &L, const double *f, long gl)
+/* the dense form's part of an accepted step before its bookkeeping, with the
+ * interpolation error err: above 10 the step is redone with the step size it
+ * suggests; otherwise the frames and trajectory points inside the step are
+ * taken from its interpolant and its D rows queued */
+__device__ __forceinline__ int bs_prep(const BsArgs &a, BsLane &L, double err, long gl)
 {
-    if (DENSE) {
-        /* dydxnew waits in ym (free after the step) for the lane's turn */
-        for (int i = 0; i < BS_N; i++) L.ym[i] = f[i];
-        L.phase = PH_PREP;
-        return;
+    const double pe = tp_pow(err, 1.0 / (2 * L.k + 3));
+    L.hopt_int = L.h / (pe > 0.01 ? pe : 0.01);
+    if (err > 10.0) {
+        L.hnew = fabs(L.hopt_int);
+        L.reject = 1;
+        L.prev_reject = 1;
+        L.rej++;
+        return NX_ATTEMPT;
     }
-    bs_accept_finish<DENSE>(a, L, f, gl);
-}
-
-/* the dense form's rest of the accepted step, with dydxnew in ym */
-template <bool DENSE>
-__device__ __forceinline__ void bs_prep(const BsArgs &a, BsLane &L, long gl)
-{
-    const double *f = L.ym;
-    {
-        const double err = bs_prepare_dense(a, L, gl, f);
-        const double pe = tp_pow(err, 1.0 / (2 * L.k + 3));
-        L.hopt_int = L.h / (pe > 0.01 ? pe : 0.01);
-        if (err > 10.0) {
-            L.hnew = fabs(L.hopt_int);
-            L.reject = 1;
-            L.prev_reject = 1;
-            L.rej++;
-            bs_begin_attempt<DENSE>(a, L, gl);
-            return;
-        }
-        L.told = L.t;
-        L.hd = L.h;
-        const double tnew = L.t + L.h;
-        for (; L.nf < a.nframes; L.nf++) {
-            const double tf = bs_time(a, L, (long)(L.nf + 1) * a.ei);
-            if (!(tf < tnew)) break;
-            const double ux = bs_dense_out(a, L, gl, 3, tf);
-            const double uy = bs_dense_out(a, L, gl, 4, tf);
-            const double uz = bs_dense_out(a, L, gl, 5, tf);
-            atomicAdd(&a.espect[L.nf * a.nbins + bs_energy_bin(a, ux, uy, uz)], 1u);
-        }
-        /* trajectory points strictly inside the step, from the polynomial */
-        if (a.traj) {
-            for (; L.jt <= a.estep; L.jt += a.traj_nout) {
-                const double tj = bs_time(a, L, L.jt);
-                if (!(tj < tnew)) break;
-                double yj[BS_N];
-                for (int m = 0; m < BS_N; m++) yj[m] = bs_dense_out(a, L, gl, m, tj);
-                bs_traj_record(a, L, yj, tj);
-            }
-        }
-        /* ym keeps dydxnew while the D rows run */
-        if (bs_next_drow<DENSE>(a, L, gl)) return;
+    L.told = L.t;
+    L.hd = L.h;
+    const double tnew = L.t + L.h;
+    for (; L.nf < a.nframes; L.nf++) {
+        const double tf = bs_time(a, L, (long)(L.nf + 1) * a.ei);
+        if (!(tf < tnew)) break;
+        const double ux = bs_dense_out(a, L, gl, 3, tf);
+        const double uy = bs_dense_out(a, L, gl, 4, tf);
+        const double uz = bs_dense_out(a, L, gl, 5, tf);
+        atomicAdd(&a.espect[L.nf * a.nbins + bs_energy_bin(a, ux, uy, uz)], 1u);
     }
-    bs_accept_finish<DENSE>(a, L, f, gl);
+    /* trajectory points strictly inside the step, from the polynomial */
+    if (a.traj) {
+        for (; L.jt <= a.estep; L.jt += a.traj_nout) {
+            const double tj = bs_time(a, L, L.jt);
+            if (!(tj < tnew)) break;
+            double yj[BS_N];
+#pragma unroll
+            for (int m = 0; m < BS_N; m++) yj[m] = bs_dense_out(a, L, gl, m, tj);
+            bs_traj_record(a, L, yj, tj);
+        }
+    }
+    /* ym keeps dydxnew while the D rows run */
+    return bs_next_drow(a, L, gl) ? NX_NONE : NX_ACCEPT;
 }
 
 /* after the field e at a D row's point: its terms, then the next row or
  * the rest of the step (or, at the end time, of the particle) */
-template <bool DENSE>
-__device__ __forceinline__ void bs_drow(const BsArgs &a, BsLane &L, const Emf &e, long gl)
+__device__ __forceinline__ int bs_drow(const BsArgs &a, BsLane &L, const Emf &e, long gl)
 {
     bs_dterms(a, L.pi, L.nr, 0, L.yn, L.xe, L.xs, e);
     L.nr++;
     if (L.ending) {
         if (L.nr < a.nd) {
             L.xe = bs_time(a, L, (long)L.nr * a.di);
-            return;                                    /* same point, next row */
+            return NX_NONE;                            /* same point, next row */
         }
-        bs_finish<DENSE>(a, L, 0, gl);
-        return;
+        return NX_DONE;
     }
-    if (bs_next_drow<DENSE>(a, L, gl)) return;
-    bs_accept_finish<DENSE>(a, L, L.ym, gl);
+    return bs_next_drow(a, L, gl) ? NX_NONE : NX_ACCEPT;
+}
+
+/* the rest of a lane's iteration, from `next` on */
+template <bool DENSE>
+__device__ __forceinline__ void bs_tail(const BsArgs &a, const BsConsts &C, BsLane &L, BsCost &W,
+                                        int next, long gl)
+{
+    if (next == NX_ACCEPT) next = bs_accept_finish<DENSE>(a, C, L, W);
+    if (next == NX_START) next = bs_start_step<DENSE>(a, L, W, gl);
+    if (next == NX_ATTEMPT) {
+        L.h = L.hnew;
+        L.reject = 0;
+        L.k = 0;
+        L.ipt = 0;
+        next = ++L.attempts > a.cap ? NX_FAIL : NX_SEQ;
+    }
+    if (next == NX_SEQ) bs_begin_seq<DENSE>(L);
+    if (next >= NX_FAIL) bs_finish<DENSE>(a, L, next == NX_FAIL ? 1 : 0, gl);
 }
 
 template <int FK, bool DENSE>
-__global__ void __launch_bounds__(256) k_bs(BsArgs a)
+__device__ __forceinline__ void bs_body(const BsArgs &a)
 {
+    extern __shared__ double modes_lds[];
     const int lane = threadIdx.x & 63;
-    const long gl = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    /* scratch index of a lane that takes particles */
+    const long gl = ((long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * a.lanes + lane;
+    const int batch = a.lanes >> 2 < BS_PREP ? a.lanes >> 2 : BS_PREP;
+    __shared__ double points[FK == FK_MODES || DENSE ? 4 * MODES_WAVE_LDS : 1];
+    double *xp = points + (FK == FK_MODES || DENSE ? (threadIdx.x >> 6) * MODES_WAVE_LDS : 0);
+    __shared__ BsConsts C;
+    if (FK == FK_MODES && a.lds_quads) {
+        for (int q = threadIdx.x; q < 32 * a.lds_quads; q += blockDim.x)
+            modes_lds[q] = a.f.modesx[q];
+    }
+    for (unsigned q = threadIdx.x; q < sizeof(BsConsts) / 4; q += blockDim.x)
+        ((int *)&C)[q] = ((const int *)&a.c)[q];
+    __syncthreads();
     BsLane L;
-    L.pi = -1;
+    BsTab T;
+    BsCost W;
+    L.pi = lane < a.lanes ? -1 : -2;
     while (true) {
         /* refill idle lanes: one atomic per wavefront */
         unsigned long long need = __ballot(L.pi == -1);
@@ -889,7 +953,7 @@ __global__ void __launch_bounds__(256) k_bs(BsArgs a)
                     double T = 2.0 * TP_PI * g0 / (fabs(a.qm) * a.b_ref);
                     L.tend = a.t_end_gyro > 0.0 ? L.t + a.t_end_gyro * T : a.t_end;
                     L.hnext = a.h0 > 0.0 ? a.h0 : 0.01 * T;
-                    L.ktarg = a.c.ktarg0;
+                    L.ktarg = C.ktarg0;
                     L.first = 1;
                     L.last = L.reject = L.prev_reject = 0;
                     L.attempts = L.acc = L.rej = 0;
@@ -906,7 +970,7 @@ __global__ void __launch_bounds__(256) k_bs(BsArgs a)
                         bs_particle_bc(a, L);
                         if (L.esc) {
                             L.ending = -1;
-                            bs_finish<DENSE>(a, L, 0, gl);
+                            L.phase = PH_OUT;
                         }
                     }
                 } else {
@@ -916,39 +980,43 @@ __global__ void __launch_bounds__(256) k_bs(BsArgs a)
         }
         if (__ballot(L.pi >= 0) == 0ull) break;
         /* the one field evaluation of this iteration, executed by the whole
-         * wavefront (retired lanes evaluate a dummy point) so the field sum
-         * stays in uniform control flow and its uniform table reads become
-         * scalar loads */
-        const bool act = L.pi >= 0 && !(DENSE && L.phase == PH_PREP);
+         * wavefront: the mode sum packs the points of the lanes that need
+         * one; for the other fields the rest evaluate a dummy point */
+        const bool act = L.pi >= 0 && !(DENSE && L.phase >= PH_PREP);
         double ze[BS_N];
         for (int i = 0; i < BS_N; i++)
             ze[i] = !act ? 0.0
                          : (L.phase == PH_INIT ? L.yv[i]
                                                : (L.phase == PH_ACCEPT ? L.ycur[i] : L.yn[i]));
         Emf e;
-        get_emf64<FK>(a.f, ze[0], ze[1], ze[2], act ? L.xe : 0.0, e);
+        if constexpr (FK == FK_MODES) {
+            if (a.lds_quads)
+                modes_wave64(a.f, (lds_tab)modes_lds, act, ze[0], ze[1], ze[2], xp, e);
+            else
+                modes_wave64(a.f, a.f.modesx, act, ze[0], ze[1], ze[2], xp, e);
+        } else
+            get_emf64<FK>(a.f, ze[0], ze[1], ze[2], act ? L.xe : 0.0, e);
+        int next = DENSE && L.pi >= 0 && L.phase == PH_OUT ? NX_DONE : NX_NONE;
         if (act && DENSE && L.phase == PH_DROW) {
-            bs_drow<DENSE>(a, L, e, gl);
+            next = bs_drow(a, L, e, gl);
         } else if (act) {
             double f[BS_N];
             bs_deriv(e, a.qm, ze, f);
             L.rhs++;
-            if (L.phase == PH_INIT) {
-                for (int i = 0; i < BS_N; i++) L.dydx[i] = f[i];
-                bs_start_step<DENSE>(a, L, gl);
-            } else if (L.phase == PH_MID) {
-                if (L.nn < L.nstep) {
-                    if (DENSE) {
-                        if (L.nn == L.nstep / 2)
-                            for (int i = 0; i < BS_N; i++)
-                                DSV(a, DS_YSAVE + L.k * BS_N + i) = L.yn[i];
-                        if (abs(L.nn - L.nstep / 2) <= 2 * L.k + 1) {
-                            for (int i = 0; i < BS_N; i++)
-                                DSV(a, DS_FSAVE + L.ipt * BS_N + i) = f[i];
-                            L.ipt++;
-                        }
+            if (L.phase == PH_MID) {
+                if (DENSE) {
+                    if (L.nn == L.nstep / 2 && L.nn < L.nstep)
+#pragma unroll
+                        for (int i = 0; i < BS_N; i++) DSR(a, DS_YSAVE + L.k, i) = L.yn[i];
+                    if (abs(L.nn - L.nstep / 2) <= 2 * L.k + 1) {
+#pragma unroll
+                        for (int i = 0; i < BS_N; i++) DSR(a, DS_FSAVE + L.ipt, i) = f[i];
+                        L.ipt++;
                     }
+                }
+                if (L.nn < L.nstep) {
                     double h2 = 2.0 * L.hsub;
+#pragma unroll
                     for (int i = 0; i < BS_N; i++) {
                         double swap = L.ym[i] + h2 * f[i];
                         L.ym[i] = L.yn[i];
@@ -957,30 +1025,45 @@ __global__ void __launch_bounds__(256) k_bs(BsArgs a)
                     L.xe += L.hsub;
                     L.nn++;
                 } else {
-                    if (DENSE && L.nstep / 2 <= 2 * L.k + 1) {
-                        for (int i = 0; i < BS_N; i++)
-                            DSV(a, DS_FSAVE + L.ipt * BS_N + i) = f[i];
-                        L.ipt++;
-                    }
                     double yseq[BS_N];
+#pragma unroll
                     for (int i = 0; i < BS_N; i++)
                         yseq[i] = 0.5 * (L.ym[i] + L.yn[i] + L.hsub * f[i]);
-                    bs_end_seq<DENSE>(a, L, yseq, gl);
+                    next = bs_end_seq<DENSE>(a, C, L, T, W, yseq);
                 }
+            } else if (L.phase == PH_INIT) {
+#pragma unroll
+                for (int i = 0; i < BS_N; i++) L.dydx[i] = f[i];
+                next = NX_START;
             } else {
-                bs_accept<DENSE>(a, L, f, gl);
+                /* the derivative at the accepted point goes to ym (free after
+                 * the step), where the dense form's lanes keep it until their
+                 * interpolant is formed */
+#pragma unroll
+                for (int i = 0; i < BS_N; i++) L.ym[i] = f[i];
+                if (DENSE) L.phase = PH_PREP;
+                else next = NX_ACCEPT;
             }
         }
         if (DENSE) {
             const unsigned long long pend = __ballot(L.pi >= 0 && L.phase == PH_PREP);
             if (pend) {
-                const unsigned long long busy = __ballot(L.pi >= 0 && L.phase != PH_PREP);
-                if ((__popcll(pend) >= BS_PREP_BATCH || busy == 0ull) && L.pi >= 0 &&
-                    L.phase == PH_PREP)
-                    bs_prep<DENSE>(a, L, gl);
+                const unsigned long long busy = __ballot(L.pi >= 0 && L.phase < PH_PREP);
+                if (__popcll(pend) >= batch || busy == 0ull) {
+                    const bool mine = L.pi >= 0 && L.phase == PH_PREP;
+                    const double err = bs_prepare_dense(a, C, L, mine, gl, xp);
+                    if (mine) next = bs_prep(a, L, err, gl);
+                }
             }
         }
+        bs_tail<DENSE>(a, C, L, W, next, gl);
     }
+}
+
+template <int FK, bool DENSE>
+__global__ void __launch_bounds__(256) k_bs(BsArgs a)
+{
+    bs_body<FK, DENSE>(a);
 }
 
 /* counter reset as a kernel (graph-safe, no memset node) */
@@ -989,12 +1072,12 @@ __global__ void k_bs_reset(unsigned long long *ctr)
     if (threadIdx.x < Q_N) ctr[threadIdx.x] = 0ull;
 }
 
-typedef void (*bs_fn)(dim3, dim3, hipStream_t, const BsArgs &);
+typedef void (*bs_fn)(dim3, dim3, size_t, hipStream_t, const BsArgs &);
 
 template <int FK, bool DENSE>
-static void launch_bs(dim3 g, dim3 b, hipStream_t s, const BsArgs &a)
+static void launch_bs(dim3 g, dim3 b, size_t sh, hipStream_t s, const BsArgs &a)
 {
-    hipLaunchKernelGGL((k_bs<FK, DENSE>), g, b, 0, s, a);
+    hipLaunchKernelGGL((k_bs<FK, DENSE>), g, b, sh, s, a);
 }
 
 template <bool DENSE>
@@ -1103,6 +1186,7 @@ static void bs_fill_args(const tp_ctx *c, const tp_bs_params *p, BsArgs &a, int 
     bs_consts(p->kmax, p->rtol, dense, &a.c);
     a.n = n;
     a.cap = cap;
+    a.lanes = 64;
     a.qm = p->qm; a.rtol = p->rtol; a.atol = p->atol;
     a.t_end = p->t_end; a.t_end_gyro = p->t_end_gyro; a.b_ref = p->b_ref; a.h0 = p->h0;
     a.x = x; a.y = y; a.z = z; a.ux = ux; a.uy = uy; a.uz = uz; a.t = t;
@@ -1118,15 +1202,49 @@ static int bs_ensure_ctr(tp_ctx *c)
     return TP_OK;
 }
 
-static dim3 bs_grid(const tp_ctx *c, int block, int wpc, int n)
+/* Lanes of a wavefront that take particles.  The mode sum's cost follows a
+ * wavefront's particles in steps of 16 (modes_wave64), so wavefronts take 32
+ * or 16 as long as that still leaves at most one for each SIMD, which is what
+ * the kernels' registers allow to run at a time: 30,000 particles, 200 modes,
+ * dense form, 64 / 32 / 16 lanes: 32.0 / 23.1 / 28.8 ms (16 lanes take two
+ * rounds).  The other fields cost a wavefront the same however many of its
+ * lanes are in use. */
+static int bs_lanes(const tp_ctx *c, int wpc, int n)
+{
+    if (c->f.kind != FK_MODES) return 64;
+    const long waves = (long)(c->num_cu > 0 ? c->num_cu : 256) * (wpc < 4 ? wpc : 4);
+    int lanes = 64;
+    while (lanes > 16 && ((long)n + lanes / 2 - 1) / (lanes / 2) <= waves) lanes /= 2;
+    return lanes;
+}
+
+static dim3 bs_grid(const tp_ctx *c, int block, int wpc, int n, int lanes)
 {
     int cu = c->num_cu > 0 ? c->num_cu : 256;
-    long lanes = (long)cu * wpc * 64;
-    long need = ((long)n + 63) / 64 * 64;       /* no more lanes than particles */
-    if (lanes > need) lanes = need;
-    long blocks = (lanes + block - 1) / block;
+    long waves = (long)cu * wpc;
+    long need = ((long)n + lanes - 1) / lanes;  /* no more than the particles fill */
+    if (waves > need) waves = need;
+    long blocks = (waves * 64 + block - 1) / block;
     if (blocks < 1) blocks = 1;
     return dim3((unsigned)blocks);
+}
+
+/* The mode table goes to LDS when the copies of the blocks that share a
+ * compute unit fit beside their point buffers (up to 1008 modes): its reads
+ * then take some 100 cycles instead of those of an L2 hit, which a wavefront
+ * alone on its SIMD waits for (131,072 particles, 1000 modes, 0.3
+ * gyroperiods: 22.9 -> 20.5 ms).  Returns the launch's dynamic LDS. */
+static size_t bs_lds(const tp_ctx *c, int block, int wpc, BsArgs &a)
+{
+    a.lds_quads = 0;
+    if (c->f.kind != FK_MODES) return 0;
+    const int quads = c->f.nquads + MODES_PAD_QUADS;
+    const size_t bytes = (size_t)32 * sizeof(double) * quads;
+    const size_t per_cu = (size_t)(wpc * 64 + block - 1) / block;
+    const size_t fixed = 4 * MODES_WAVE_LDS * sizeof(double);
+    if (bytes > 64 * 1024 || (bytes + fixed) * per_cu > 160 * 1024) return 0;
+    a.lds_quads = quads;
+    return bytes;
 }
 
 /* grow a device buffer of a context to at least `need` elements */
@@ -1160,7 +1278,7 @@ int tp_gpu_run_adaptive(tp_ctx *c, const tp_bs_params *p, tp_bs_stats *stats)
     const int n = c->s.n;
     int block = p->block, wpc = p->waves_per_cu;
     if (block == 0 || wpc == 0) {
-        int tb = 64, tw = 8;
+        int tb = c->f.kind == FK_MODES ? 256 : 64, tw = 8;
         if (c->bs_tune_block) { tb = c->bs_tune_block[0]; tw = c->bs_tune_block[1]; }
         if (block == 0) block = tb;
         if (wpc == 0) wpc = tw;
@@ -1170,7 +1288,9 @@ int tp_gpu_run_adaptive(tp_ctx *c, const tp_bs_params *p, tp_bs_stats *stats)
     State &S = c->s;
     bs_fill_args(c, p, a, n, S.x, S.y, S.z, S.ux, S.uy, S.uz, S.t, S.nsteps, S.esc, c->bs_ctr,
                  cap);
-    dim3 grid = bs_grid(c, block, wpc, n);
+    a.lanes = bs_lanes(c, wpc, n);
+    dim3 grid = bs_grid(c, block, wpc, n, a.lanes);
+    const size_t lds = bs_lds(c, block, wpc, a);
     if (n > 0) {
         if (p->use_graph) {
             unsigned long long key = 1469598103934665603ull;
@@ -1185,7 +1305,7 @@ int tp_gpu_run_adaptive(tp_ctx *c, const tp_bs_params *p, tp_bs_stats *stats)
                 hipGraph_t g;
                 HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
                 hipLaunchKernelGGL(k_bs_reset, dim3(1), dim3(64), 0, c->stream, c->bs_ctr);
-                fn(grid, dim3(block), c->stream, a);
+                fn(grid, dim3(block), lds, c->stream, a);
                 HIPCHK(hipStreamEndCapture(c->stream, &g));
                 hipError_t e = hipGraphInstantiate(&c->bs_graph, g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
@@ -1202,7 +1322,7 @@ int tp_gpu_run_adaptive(tp_ctx *c, const tp_bs_params *p, tp_bs_stats *stats)
             hipLaunchKernelGGL(k_bs_reset, dim3(1), dim3(64), 0, c->stream, c->bs_ctr);
             HIPCHK(hipGetLastError());
             HIPCHK(hipEventRecord(c->ev0, c->stream));
-            fn(grid, dim3(block), c->stream, a);
+            fn(grid, dim3(block), lds, c->stream, a);
             HIPCHK(hipGetLastError());
             HIPCHK(hipEventRecord(c->ev1, c->stream));
         }
@@ -1248,13 +1368,14 @@ int tp_gpu_run_adaptive_diag(tp_ctx *c, const tp_bs_params *p, const tp_track_pa
     if (nframes > q->nt_out) nframes = q->nt_out;
     int block = p->block, wpc = p->waves_per_cu;
     if (block == 0 || wpc == 0) {
-        int tb = 64, tw = 8;
+        int tb = c->f.kind == FK_MODES ? 256 : 64, tw = 8;
         if (c->bs_tune_block) { tb = c->bs_tune_block[0]; tw = c->bs_tune_block[1]; }
         if (block == 0) block = tb;
         if (wpc == 0) wpc = tw;
     }
-    const dim3 grid = bs_grid(c, block, wpc, n);
-    const long nl = (long)grid.x * block;
+    const int lanes = bs_lanes(c, wpc, n);
+    const dim3 grid = bs_grid(c, block, wpc, n, lanes);
+    const long nl = (long)grid.x * (block / 64) * lanes;
     /* the run's outputs in the context's diagnostics buffers (read back by
      * tp_gpu_read_diagnostics), the scratch of the dense form */
     const size_t need = (size_t)q->nbins * q->nt_out;
@@ -1277,10 +1398,10 @@ int tp_gpu_run_adaptive_diag(tp_ctx *c, const tp_bs_params *p, const tp_track_pa
     const size_t dneed = (size_t)nd * 8 * (n > 0 ? n : 1);
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) == hipSuccess &&
-        (dneed + (size_t)nl * DS_SLOTS) * sizeof(double) > fr / 2 + c->bs_dbuf_cap * sizeof(double))
+        (dneed + (size_t)nl * DS_ROWS * BS_N) * sizeof(double) > fr / 2 + c->bs_dbuf_cap * sizeof(double))
         return TP_E_NOMEM;
     if ((rc = bs_grow(&c->bs_dbuf, &c->bs_dbuf_cap, dneed)) ||
-        (rc = bs_grow(&c->bs_ds, &c->bs_ds_cap, (size_t)nl * DS_SLOTS)) ||
+        (rc = bs_grow(&c->bs_ds, &c->bs_ds_cap, (size_t)nl * DS_ROWS * BS_N)) ||
         (rc = bs_grow(&c->bs_outhist, &c->bs_outhist_cap, (size_t)nd)))
         return rc;
     hipLaunchKernelGGL(k_bs_zero_u32, dim3(256), dim3(256), 0, c->stream, c->espect, need);
@@ -1294,6 +1415,8 @@ int tp_gpu_run_adaptive_diag(tp_ctx *c, const tp_bs_params *p, const tp_track_pa
     State &S = c->s;
     bs_fill_args(c, p, a, n, S.x, S.y, S.z, S.ux, S.uy, S.uz, S.t, S.nsteps, S.esc, c->bs_ctr,
                  cap, 1);
+    a.lanes = lanes;
+    const size_t lds = bs_lds(c, block, wpc, a);
     a.ds = c->bs_ds; a.nl = nl;
     a.dt = q->dt; a.estep = q->estep; a.ei = q->einterval_t; a.di = q->dcoeff_interval;
     a.nd = nd; a.nframes = nframes; a.nbins = q->nbins; a.nt_out = q->nt_out;
@@ -1314,7 +1437,7 @@ int tp_gpu_run_adaptive_diag(tp_ctx *c, const tp_bs_params *p, const tp_track_pa
     hipLaunchKernelGGL(k_bs_reset, dim3(1), dim3(64), 0, c->stream, c->bs_ctr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(c->ev0, c->stream));
-    if (n > 0) fn(grid, dim3(block), c->stream, a);
+    if (n > 0) fn(grid, dim3(block), lds, c->stream, a);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     hipLaunchKernelGGL(k_bs_dsum, dim3(8 * nd), dim3(256), 0, c->stream,
@@ -1410,9 +1533,12 @@ int tp_gpu_tune_adaptive(tp_ctx *c, const tp_bs_params *p, const char *cache_pat
                 bs_fill_args(c, p, a, nt, buf, buf + nt, buf + 2 * (size_t)nt,
                              buf + 3 * (size_t)nt, buf + 4 * (size_t)nt, buf + 5 * (size_t)nt,
                              buf + 6 * (size_t)nt, ib, ib + nt, c->bs_ctr, 24);
+                a.lanes = bs_lanes(c, wpcs[wi], c->s.n);
+                const size_t lds = bs_lds(c, blocks[bi], wpcs[wi], a);
                 hipLaunchKernelGGL(k_bs_reset, dim3(1), dim3(64), 0, c->stream, c->bs_ctr);
                 (void)hipEventRecord(c->ev0, c->stream);
-                fn(bs_grid(c, blocks[bi], wpcs[wi], nt), dim3(blocks[bi]), c->stream, a);
+                fn(bs_grid(c, blocks[bi], wpcs[wi], nt, a.lanes), dim3(blocks[bi]), lds,
+                   c->stream, a);
                 (void)hipEventRecord(c->ev1, c->stream);
                 if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
                     rc = TP_E_HIP;

@@ -39,6 +39,7 @@ struct tp_ctx {
     double *vgrid = nullptr, *modes = nullptr;
     double *gridd = nullptr;                       /* double PIC nodes */
     float *modes32 = nullptr;
+    double *modesx = nullptr;                      /* mode rows for the matrix cores */
     WlcsSys *wl = nullptr;
     State s;
     /* diagnostics of the last run */

@@ -95,6 +95,12 @@ struct FieldDev {
     /* modes: rows kx ky kz ax ay az phi */
     int nmodes;
     const double *modes;
+    /* the same rows for the matrix cores (modes_wave64): per four modes 16
+     * doubles (phi kx ky kz) and 16 (ax ay az 0), nquads such groups (a
+     * multiple of four, padded with zero rows; MODES_PAD_QUADS groups of
+     * zeros follow) */
+    const double *modesx;
+    int nquads;
     double b0z;
     /* the same table for FP32: (kx ky kz phi) / 2 pi, ax ay az 0 per mode */
     const float *modes32;
@@ -954,6 +960,124 @@ __device__ __forceinline__ void get_emf64(const FieldDev &f, double x, double y,
         }
         o.ex = ax; o.ey = ay; o.ez = az;
         o.bx = bx; o.by = by; o.bz = bz;
+    }
+}
+
+/* ------------------------------------------------------------------ */
+/* the multi-mode field of a wavefront's points on the matrix cores     */
+/* ------------------------------------------------------------------ */
+/* FP64 sum over the modes at up to 64 points of a wavefront, of which only
+ * some are wanted: the points are packed into groups of 16, and a group's
+ * sum goes four modes at a time over all 64 lanes (16 points x 4 modes), so
+ * its cost follows the number of wanted points and not the wavefront's size.
+ *
+ * v_mfma_f64_4x4x4_4b (four independent 4x4x4 products, blocks b) has, in
+ * lane l with i = l & 3, b = (l >> 2) & 3, k = l >> 4:
+ *   A[i][k],  B[k][i],  D[k][i]  of block b (A the same in every block here),
+ * and adds its four products to C one after another, each a fused
+ * multiply-add with one rounding (checked bit for bit on the device).  So
+ *   phase[mode][point] = (phi kx ky kz)[mode] . (1 x y z)[point]
+ * is fma(kz, z, fma(ky, y, fma(kx, x, phi))) and
+ *   sum[component][point] += a[component][mode] cos[mode][point]
+ * runs over the modes in order: the bits of get_emf64<FK_MODES>.  The phase
+ * product leaves mode k of point l & 15 in lane l, which is where the second
+ * product takes it from: no exchange of lanes between the two.
+ *
+ * Bound: FP64 issue, 17 operations of the cosine and two 16-cycle products
+ * per 4 modes x 16 points (FP64 products and vector FMAs share one unit).
+ * Measured in k_bs, where many lanes of a wavefront are idle at any time:
+ * 131,072 particles, 1000 modes, 0.3 gyroperiods 47.4 -> 22 ms together with
+ * the cheaper cosine; in a loop over full wavefronts, four per SIMD, the
+ * cosine alone gives 150 -> 119 cycles per 64 points and mode and the matrix
+ * cores 114. */
+#define MODES_WAVE_LDS (64 * 4)      /* doubles of LDS per wavefront */
+#define MODES_PAD_QUADS 4            /* zero groups read ahead past the last */
+
+/* TAB: the table through global memory (const double *) or a copy of it in
+ * LDS (lds_tab) */
+typedef const double __attribute__((address_space(3))) *lds_tab;
+
+template <int G, class TAB>
+__device__ __forceinline__ void modes_groups64(TAB tab, int nquads, double *xp)
+{
+    constexpr int U = G == 1 ? 4 : (G == 2 ? 2 : 1);    /* quads in flight */
+    const int lane = threadIdx.x & 63, k = lane >> 4, m = lane & 3;
+    double *slot = xp + (lane & 15) * 4 + k;
+    double b[G], acc[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        b[g] = slot[64 * g];
+        acc[g] = 0.0;
+    }
+    const tp_cos_pi_consts ck = tp_cos_pi_init();
+    TAB ph = tab + 4 * m + k, am = tab + 16 + 4 * k + m;
+    double pn[U], an[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        pn[u] = ph[32 * u];
+        an[u] = am[32 * u];
+    }
+#pragma unroll 1
+    for (int q = 0; q < nquads; q += U) {
+        double p[U], a[U];
+        ph += 32 * U;
+        am += 32 * U;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            p[u] = pn[u];
+            a[u] = an[u];
+            pn[u] = ph[32 * u];          /* past the end: the zero groups */
+            an[u] = am[32 * u];
+        }
+        double c[U][G];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                c[u][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(p[u], b[g], 0.0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int g = 0; g < G; g++) c[u][g] = tp_cos_pi_with(c[u][g], &ck);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                acc[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[u], c[u][g], acc[g], 0, 0, 0);
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) slot[64 * g] = acc[g];
+}
+
+/* get_emf64<FK_MODES> at the points of the lanes with `want`; every lane of
+ * the wavefront calls it (uniform control flow), xp is the wavefront's own
+ * MODES_WAVE_LDS doubles of LDS, tab the table or its copy. */
+template <class TAB>
+__device__ __forceinline__ void modes_wave64(const FieldDev &f, TAB tab, bool want, double x,
+                                             double y, double z, double *xp, Emf &o)
+{
+    o.bx = o.by = o.bz = o.ex = o.ey = o.ez = 0.0;
+    const unsigned long long mask = __ballot(want);
+    const int n = __popcll(mask);
+    if (n == 0) return;
+    const int lane = threadIdx.x & 63;
+    const int rank = __popcll(mask & ((1ull << lane) - 1ull));
+    double *mine = xp + 4 * rank;
+    /* unused points of the last group hold what an earlier call left there:
+     * every column of the products is independent of the others */
+    if (want) {
+        mine[0] = 1.0; mine[1] = x; mine[2] = y; mine[3] = z;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (n <= 16) modes_groups64<1>(tab, f.nquads, xp);
+    else if (n <= 32) modes_groups64<2>(tab, f.nquads, xp);
+    else if (n <= 48) modes_groups64<3>(tab, f.nquads, xp);
+    else modes_groups64<4>(tab, f.nquads, xp);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (want) {
+        o.bx = mine[0]; o.by = mine[1]; o.bz = f.b0z + mine[2];
     }
 }
 

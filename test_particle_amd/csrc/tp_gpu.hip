@@ -693,6 +693,7 @@ static void free_field(tp_ctx *c)
     (void)hipFree(c->vgrid); c->vgrid = nullptr;
     (void)hipFree(c->modes); c->modes = nullptr;
     (void)hipFree(c->modes32); c->modes32 = nullptr;
+    (void)hipFree(c->modesx); c->modesx = nullptr;
     (void)hipFree(c->wl); c->wl = nullptr;
     (void)hipFree(c->gridd); c->gridd = nullptr;
     c->have_field = false;
@@ -1418,9 +1419,30 @@ int tp_gpu_set_field_modes(tp_ctx *c, int nmodes, const double *rows, double b0z
                                  hipMemcpyHostToDevice);
         free(t32);
         HIPCHK(e);
+        /* rows for the matrix cores, 32 doubles per four modes */
+        const int nquads = (nmodes + 15) / 16 * 4;
+        const size_t nx = (size_t)32 * (nquads + MODES_PAD_QUADS);
+        double *tx = (double *)calloc(nx, sizeof(double));
+        if (!tx) return TP_E_NOMEM;
+        for (int m = 0; m < nmodes; m++) {
+            const double *r = rows + 7 * m;
+            double *o = tx + 32 * (size_t)(m / 4) + 4 * (m % 4);
+            o[0] = r[6]; o[1] = r[0]; o[2] = r[1]; o[3] = r[2];
+            o[16] = r[3]; o[17] = r[4]; o[18] = r[5];
+        }
+        if (hipMalloc(&c->modesx, nx * sizeof(double)) != hipSuccess) {
+            c->modesx = nullptr;
+            free(tx);
+            return TP_E_NOMEM;
+        }
+        e = hipMemcpy(c->modesx, tx, nx * sizeof(double), hipMemcpyHostToDevice);
+        free(tx);
+        HIPCHK(e);
+        c->f.nquads = nquads;
     }
     c->f.nmodes = nmodes;
     c->f.modes = c->modes;
+    c->f.modesx = c->modesx;
     c->f.modes32 = c->modes32;
     c->f.b0z = b0z;
     c->f.kind = FK_MODES;

@@ -25,10 +25,10 @@
  * the next layer's input.  The feature layer is done in two halves (sin,
  * then cos) so that a wave's tile is 64 x 128 (17 KB, 8 waves per CU).
  *
- * Backward: dZ_{l-1} = (dZ_l W_l^T) * gelu'(Z_{l-1}) with W_l fragments in
- * a second order (rows = layer input); weight gradients dW_l = X_{l-1}^T dZ_l
- * per chunk of 256 samples, with both operands transposed through LDS so the
- * reduction runs along the samples; chunk partials are summed in a fixed
+ * Training: one kernel takes 64 samples through the forward and the backward
+ * pass (dZ_{l-1} = (dZ_l W_l^T) * gelu'(Z_{l-1}), W_l fragments in a second
+ * order, rows = layer input), a second forms the weight gradients dW_l =
+ * X_{l-1}^T dZ_l per chunk of samples; their partial sums are added in a fixed
  * order by the optimiser kernel (deterministic).
  */
 #include <hip/hip_runtime.h>
@@ -86,12 +86,16 @@ __host__ __device__ inline int frag_bwd(int k, int n)
     return (((k >> 4) * 4 + (n >> 5)) * 64 + ((n >> 3) & 3) * 16 + (k & 15)) * 8 + (n & 7);
 }
 
+/* Batch buffers in tiles of 64 samples, feature-major within a tile: element
+ * (feature f, row 64 t + m) of a buffer with F features at (t F + f) 64 + m, so
+ * that 8 consecutive samples of a feature are 16 bytes, the operand of a
+ * product whose sum runs along the samples, and a block's part of a buffer is
+ * contiguous. */
 struct TrainBufs {
-    __bf16 *h0, *h1, *h2;        /* layer inputs, row-major [rows][256 | 128] */
-    float *g1, *g2, *g3, *h3;    /* gelu'(z1..z3) and h3, [rows][128] */
+    __bf16 *h0, *h1, *h2;        /* layer inputs, 256 | 128 features */
+    __bf16 *dz1, *dz2, *dz3;     /* 128 features */
+    long rows;
 };
-
-enum { MLP_EVAL = 0, MLP_TRAIN = 1 };
 
 #define GELU_C1 1.5957691216057308f   /* 2 sqrt(2/pi) */
 #define GELU_C2 0.044715f
@@ -168,12 +172,10 @@ __device__ __forceinline__ f32x4 mfma(const bf16x8 &a, const bf16x8 &b, const f3
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-/* hidden-layer epilogue: bias, gelu; layers 1-2 write the bf16 result into
- * the tile (and in training, h and gelu' to the batch buffers); layer 3
- * keeps FP32 h in acc for the output layer. */
-template <int MODE, int LAYER>
-__device__ __forceinline__ void hidden_epilogue(f32x4 (&acc)[8][4], __bf16 *tile,
-                                                const TrainBufs &tb, long row0)
+/* hidden-layer epilogue: gelu; layers 1-2 write the bf16 result into the
+ * tile; layer 3 keeps FP32 h in acc for the output layer. */
+template <int LAYER>
+__device__ __forceinline__ void hidden_epilogue(f32x4 (&acc)[8][4], __bf16 *tile)
 {
     const int lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
 #pragma unroll
@@ -182,32 +184,18 @@ __device__ __forceinline__ void hidden_epilogue(f32x4 (&acc)[8][4], __bf16 *tile
 #pragma unroll
         for (int mb = 0; mb < 4; mb++) {
             const int m = mb * 16 + i16;
-            f32x4 h, gd;
+            f32x4 h;
             float h0, h1, h2, h3;
             gelu_pk(acc[nb][mb][0], acc[nb][mb][1], h0, h1);
             gelu_pk(acc[nb][mb][2], acc[nb][mb][3], h2, h3);
             h[0] = h0; h[1] = h1; h[2] = h2; h[3] = h3;
-            if (MODE == MLP_TRAIN) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) gd[r] = gelu_deriv(acc[nb][mb][r]);
-            }
             if (LAYER < 3) {
                 bf16x4 hb;
                 hb[0] = (__bf16)h[0]; hb[1] = (__bf16)h[1];
                 hb[2] = (__bf16)h[2]; hb[3] = (__bf16)h[3];
                 *(bf16x4 *)(tile + m * TS + n0) = hb;
-                if (MODE == MLP_TRAIN) {
-                    __bf16 *ho = LAYER == 1 ? tb.h1 : tb.h2;
-                    float *go = LAYER == 1 ? tb.g1 : tb.g2;
-                    *(bf16x4 *)(ho + (row0 + m) * NH + n0) = hb;
-                    *(f32x4 *)(go + (row0 + m) * NH + n0) = gd;
-                }
             } else {
                 acc[nb][mb] = h;
-                if (MODE == MLP_TRAIN) {
-                    *(f32x4 *)(tb.h3 + (row0 + m) * NH + n0) = h;
-                    *(f32x4 *)(tb.g3 + (row0 + m) * NH + n0) = gd;
-                }
             }
         }
     }
@@ -271,12 +259,9 @@ __device__ __forceinline__ void layer128(f32x4 (&acc)[8][4], const bf16x8 *wf,
 
 /* The network at the wave's 64 points (x, y, z of this lane's sample);
  * every lane of the wave must call it.  out = h3 W4 + b4 of this lane's
- * sample.  In training, row0 is the batch row of lane 0 and the
- * activations are stored for the backward pass. */
-template <int MODE>
+ * sample. */
 __device__ __forceinline__ void mlp_wave(const MlpNet &net, float x, float y, float z,
-                                         __bf16 *tile, float out[3], const TrainBufs &tb,
-                                         long row0)
+                                         __bf16 *tile, float out[3])
 {
     const int lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
     typedef const float __attribute__((address_space(4))) *cf;
@@ -300,16 +285,14 @@ __device__ __forceinline__ void mlp_wave(const MlpNet &net, float x, float y, fl
                 v[t] = (__bf16)(h ? __builtin_amdgcn_cosf(r) : __builtin_amdgcn_sinf(r));
             }
             *(bf16x8 *)(tile + lane * TS + j8 * 8) = v;
-            if (MODE == MLP_TRAIN)
-                *(bf16x8 *)(tb.h0 + (row0 + lane) * NIN + h * NF + j8 * 8) = v;
         }
         mfma_kblocks(acc, net.w1f, 8, h * 4, 4, tile);
     }
-    hidden_epilogue<MODE, 1>(acc, tile, tb, row0);
+    hidden_epilogue<1>(acc, tile);
     layer128(acc, net.w2f, net.b2, tile);
-    hidden_epilogue<MODE, 2>(acc, tile, tb, row0);
+    hidden_epilogue<2>(acc, tile);
     layer128(acc, net.w3f, net.b3, tile);
-    hidden_epilogue<MODE, 3>(acc, tile, tb, row0);
+    hidden_epilogue<3>(acc, tile);
 
     /* output layer in FP32: partial sums over this lane's 32 hidden units
      * for its 4 samples, completed across the 4 lane groups */
@@ -359,265 +342,424 @@ __global__ void __launch_bounds__(256, 2) k_mlp_eval(MlpNet net, int n, const do
         px = (float)x[3 * i]; py = (float)x[3 * i + 1]; pz = (float)x[3 * i + 2];
     }
     float o[3];
-    TrainBufs tb = {};
-    mlp_wave<MLP_EVAL>(net, px, py, pz, tiles + (threadIdx.x >> 6) * TILE, o, tb, 0);
+    mlp_wave(net, px, py, pz, tiles + (threadIdx.x >> 6) * TILE, o);
     if (i < n) {
         out[3 * i] = o[0]; out[3 * i + 1] = o[1]; out[3 * i + 2] = o[2];
     }
 }
 
-/* training forward over batch rows [0, rows): sample s0 + row of the set
- * (x, targets y); rows >= nvalid are padding (zero gradient).  Writes the
- * activations, dL/dout and one loss partial (sum of squared errors) per
- * block. */
-__global__ void __launch_bounds__(256, 2) k_mlp_train_fwd(MlpNet net, const float *dsx,
-        const float *dsy, long s0, int nvalid, float inv3n, TrainBufs tb, float *dout,
-        double *lossp)
+/* ------------------------------------------------------------------ */
+/* training                                                            */
+/* ------------------------------------------------------------------ */
+/* partial sums of the small parameters, one row per block of 64 samples */
+#define S_B1 0
+#define S_B2 (S_B1 + NH)
+#define S_B3 (S_B2 + NH)
+#define S_W4 (S_B3 + NH)
+#define S_B4 (S_W4 + 3 * NH)
+#define S_TOTAL (S_B4 + 3)
+
+/* stride of the feature tile: 256 bf16 and 8 (528 bytes, the 16 rows of a
+ * fragment read on distinct 4-bank groups) */
+#define TF 264
+
+/* the weight fragments of this wave's 32 outputs of a layer with KB k-blocks
+ * of 32 inputs (loaded well ahead of their use: after each Adam step they come
+ * from beyond the L2) */
+template <int KB>
+struct WFrag {
+    bf16x8 a[2][KB];
+    __device__ __forceinline__ void load(const bf16x8 *wf)
+    {
+        const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) a[nb][kb] = wf[((2 * w + nb) * KB + kb) * 64 + lane];
+    }
+};
+
+/* this wave's 32 outputs (features 32 w ..) of a layer over the block's 64
+ * samples: acc += W^T X^T with the layer's input in tile */
+template <int KB, int STRIDE>
+__device__ __forceinline__ void train_layer(f32x4 (&acc)[2][4], const WFrag<KB> &f,
+                                            const __bf16 *tile)
 {
-    __shared__ __attribute__((aligned(16))) __bf16 tiles[4 * TILE];
-    __shared__ double wl[4];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long row0 = (long)blockIdx.x * 256 + w * 64;
-    const long row = row0 + lane;
+    const int lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+        bf16x8 b[4];
+#pragma unroll
+        for (int mb = 0; mb < 4; mb++)
+            b[mb] = *(const bf16x8 *)(tile + (mb * 16 + i16) * STRIDE + kb * 32 + 8 * g);
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+            for (int mb = 0; mb < 4; mb++) acc[nb][mb] = mfma(f.a[nb][kb], b[mb], acc[nb][mb]);
+    }
+}
+
+/* four values of consecutive features n0 .. n0 + 3 of block sample m: to the
+ * LDS tile (row-major) and the block's tile of a batch buffer */
+__device__ __forceinline__ bf16x4 train_store(const f32x4 &v, __bf16 *tile, __bf16 *buf, int m,
+                                              int n0)
+{
+    bf16x4 b;
+#pragma unroll
+    for (int r = 0; r < 4; r++) b[r] = (__bf16)v[r];
+    if (tile) *(bf16x4 *)(tile + m * TS + n0) = b;
+#pragma unroll
+    for (int r = 0; r < 4; r++) buf[(n0 + r) * 64 + m] = b[r];
+    return b;
+}
+
+/* sum over the 16 lanes of a row */
+__device__ __forceinline__ float row_sum(float v)
+{
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+/* Forward and backward pass of 64 samples in one block of four waves: batch
+ * rows 64 blockIdx.x .. of the set from sample s0 on (x, targets y); rows >=
+ * nvalid are padding (zero gradient).  Each wave takes 32 of every layer's 128
+ * outputs over all 64 samples; gelu' of its outputs stays in its registers
+ * from the forward to the backward pass, whose products leave the same
+ * elements in the same lanes, so nothing but the operands of the weight
+ * gradients goes to memory.  Writes those, the partial sums of the biases and
+ * the output layer (row of S_TOTAL in small) and the loss partial.
+ * Bound: the chain of layers on one wave per SIMD (the batch of 16,384 is 256
+ * blocks); a wave per 64 samples, which left three of four compute units
+ * idle, and two kernels with gelu' and h3 through memory took 47 + 33 us a
+ * batch, this 28. */
+__global__ void __launch_bounds__(256) k_mlp_train(MlpNet net, const float *dsx, const float *dsy,
+                                                   long s0, int nvalid, float inv3n, TrainBufs tb,
+                                                   float *small, double *lossp)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 feat[64 * TF];
+    __shared__ __attribute__((aligned(16))) __bf16 ta[TILE], tc[TILE];
+    __shared__ float red[4][64][3], dl[64][3];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
+    const long row = (long)blockIdx.x * 64 + lane;
     const bool valid = row < nvalid;
     float px = 0.f, py = 0.f, pz = 0.f;
     if (valid) {
-        const long s = s0 + row;
-        px = dsx[3 * s]; py = dsx[3 * s + 1]; pz = dsx[3 * s + 2];
+        const long sa = s0 + row;
+        px = dsx[3 * sa]; py = dsx[3 * sa + 1]; pz = dsx[3 * sa + 2];
     }
-    float o[3];
-    mlp_wave<MLP_TRAIN>(net, px, py, pz, tiles + w * TILE, o, tb, row0);
-    double e2 = 0.0;
+    WFrag<8> f1;
+    WFrag<4> f2, f3;
+    f1.load(net.w1f);
+    f2.load(net.w2f);
+    /* features of frequencies 32 w .. 32 w + 31 at the lane's sample */
+    {
+        typedef const float __attribute__((address_space(4))) *cf;
+        const cf q = (cf)net.q + 96 * __builtin_amdgcn_readfirstlane(w);
+        __bf16 *ho = tb.h0 + (size_t)blockIdx.x * (64 * NIN);
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-        float d = 0.f;
-        if (valid) {
-            float e = o[c] - dsy[3 * (s0 + row) + c];
-            e2 += (double)e * (double)e;
-            d = 2.0f * e * inv3n;
-        }
-        dout[3 * row + c] = d;
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) e2 += __shfl_xor(e2, off, 64);
-    if (lane == 0) wl[w] = e2;
-    __syncthreads();
-    if (threadIdx.x == 0) lossp[blockIdx.x] = ((wl[0] + wl[1]) + wl[2]) + wl[3];
-}
-
-/* backward through layers 3 and 2: dZ3 from dL/dout, W4 and gelu'(z3);
- * dZ2 = (dZ3 W3^T) gelu'(z2); dZ1 = (dZ2 W2^T) gelu'(z1).  All three are
- * stored row-major in bfloat16 for the weight gradients. */
-__global__ void __launch_bounds__(256, 2) k_mlp_train_bwd(MlpNet net, TrainBufs tb,
-        const float *dout, __bf16 *dz3, __bf16 *dz2, __bf16 *dz1)
-{
-    __shared__ __attribute__((aligned(16))) __bf16 tiles[4 * TILE];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
-    __bf16 *tile = tiles + w * TILE;
-    const long row0 = (long)blockIdx.x * 256 + w * 64;
-    f32x4 acc[8][4];
-#pragma unroll
-    for (int ib = 0; ib < 8; ib++)
-#pragma unroll
-        for (int mb = 0; mb < 4; mb++) acc[ib][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int kb = 0; kb < 4; kb++) {
-        bf16x8 bz[4];
-        const int n0 = kb * 32 + 8 * g;
-        const f32x4 *wp = (const f32x4 *)(net.w4 + 3 * n0);
-        f32x4 wv[6];
-#pragma unroll
-        for (int k = 0; k < 6; k++) wv[k] = wp[k];
-#pragma unroll
-        for (int mb = 0; mb < 4; mb++) {
-            const long r = row0 + mb * 16 + i16;
-            const float d0 = dout[3 * r], d1 = dout[3 * r + 1], d2 = dout[3 * r + 2];
-            const f32x4 ga = *(const f32x4 *)(tb.g3 + r * NH + n0);
-            const f32x4 gb = *(const f32x4 *)(tb.g3 + r * NH + n0 + 4);
+        for (int j8 = 0; j8 < 4; j8++) {
+            bf16x8 vs, vc;
 #pragma unroll
             for (int t = 0; t < 8; t++) {
-                const int e = 3 * t;
-                const float w0 = wv[e / 4][e % 4], w1 = wv[(e + 1) / 4][(e + 1) % 4],
-                            w2 = wv[(e + 2) / 4][(e + 2) % 4];
-                float dh = fmaf(d2, w2, fmaf(d1, w1, d0 * w0));
-                bz[mb][t] = (__bf16)(dh * (t < 4 ? ga[t] : gb[t - 4]));
+                const int j = j8 * 8 + t;
+                const float u = fmaf(q[3 * j + 2], pz, fmaf(q[3 * j + 1], py, q[3 * j] * px));
+                const float r = __builtin_amdgcn_fractf(u);
+                vs[t] = (__bf16)__builtin_amdgcn_sinf(r);
+                vc[t] = (__bf16)__builtin_amdgcn_cosf(r);
+                const int f = 32 * w + j;
+                ho[f * 64 + lane] = vs[t];
+                ho[(NF + f) * 64 + lane] = vc[t];
             }
-            *(bf16x8 *)(dz3 + r * NH + n0) = bz[mb];
-        }
-#pragma unroll
-        for (int ib = 0; ib < 8; ib++) {
-            const bf16x8 a = net.w3b[(ib * 4 + kb) * 64 + lane];
-#pragma unroll
-            for (int mb = 0; mb < 4; mb++) acc[ib][mb] = mfma(a, bz[mb], acc[ib][mb]);
+            *(bf16x8 *)(feat + lane * TF + 32 * w + j8 * 8) = vs;
+            *(bf16x8 *)(feat + lane * TF + NF + 32 * w + j8 * 8) = vc;
         }
     }
-    /* dZ2 */
+    f32x4 acc[2][4], g1[2][4], g2[2][4], g3[2][4];
+    const int nw = 32 * w + 4 * g;      /* the lane's outputs: nw + 16 nb + r */
+    const size_t at = (size_t)blockIdx.x * (64 * NH);   /* the block's tile */
+    auto bias = [&](const float *b) {
 #pragma unroll
-    for (int ib = 0; ib < 8; ib++)
+        for (int nb = 0; nb < 2; nb++) {
+            const f32x4 v = *(const f32x4 *)(b + nw + 16 * nb);
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++) {
-            const int m = mb * 16 + i16;
-            const int k0 = ib * 16 + 4 * g;
-            const f32x4 gg = *(const f32x4 *)(tb.g2 + (row0 + m) * NH + k0);
-            bf16x4 v;
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = (__bf16)(acc[ib][mb][r] * gg[r]);
-            *(bf16x4 *)(tile + m * TS + k0) = v;
-            *(bf16x4 *)(dz2 + (row0 + m) * NH + k0) = v;
+            for (int mb = 0; mb < 4; mb++) acc[nb][mb] = v;
         }
-    /* dZ1 */
+    };
+    /* gelu and its derivative; acc becomes h */
+    auto act = [&](f32x4 (&gd)[2][4]) {
 #pragma unroll
-    for (int ib = 0; ib < 8; ib++)
+        for (int nb = 0; nb < 2; nb++)
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++) acc[ib][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int kb = 0; kb < 4; kb++) {
-        bf16x8 bx[4];
+            for (int mb = 0; mb < 4; mb++) {
+                f32x4 z = acc[nb][mb];
+                float h0, h1, h2, h3;
+                gelu_pk(z[0], z[1], h0, h1);
+                gelu_pk(z[2], z[3], h2, h3);
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
-            bx[mb] = *(const bf16x8 *)(tile + (mb * 16 + i16) * TS + kb * 32 + 8 * g);
+                for (int r = 0; r < 4; r++) gd[nb][mb][r] = gelu_deriv(z[r]);
+                acc[nb][mb] = f32x4{h0, h1, h2, h3};
+            }
+    };
+    auto store = [&](__bf16 *tile, __bf16 *buf) {
 #pragma unroll
-        for (int ib = 0; ib < 8; ib++) {
-            const bf16x8 a = net.w2b[(ib * 4 + kb) * 64 + lane];
+        for (int nb = 0; nb < 2; nb++)
 #pragma unroll
-            for (int mb = 0; mb < 4; mb++) acc[ib][mb] = mfma(a, bx[mb], acc[ib][mb]);
-        }
-    }
-#pragma unroll
-    for (int ib = 0; ib < 8; ib++)
-#pragma unroll
-        for (int mb = 0; mb < 4; mb++) {
-            const int m = mb * 16 + i16;
-            const int k0 = ib * 16 + 4 * g;
-            const f32x4 gg = *(const f32x4 *)(tb.g1 + (row0 + m) * NH + k0);
-            bf16x4 v;
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = (__bf16)(acc[ib][mb][r] * gg[r]);
-            *(bf16x4 *)(dz1 + (row0 + m) * NH + k0) = v;
-        }
-}
+            for (int mb = 0; mb < 4; mb++)
+                train_store(acc[nb][mb], tile, buf + at, mb * 16 + i16, nw + 16 * nb);
+    };
+    bias(net.b1);
+    __syncthreads();
+    f3.load(net.w3f);
+    train_layer<8, TF>(acc, f1, feat);
+    act(g1);
+    store(ta, tb.h1);
+    bias(net.b2);
+    __syncthreads();
+    train_layer<4, TS>(acc, f2, ta);
+    f2.load(net.w3b);               /* the backward pass's fragments */
+    act(g2);
+    store(tc, tb.h2);
+    bias(net.b3);
+    __syncthreads();
+    train_layer<4, TS>(acc, f3, tc);
+    f3.load(net.w2b);
+    act(g3);
 
-/* LDS tiles of the weight-gradient kernel: 32 samples, transposed
- * (row = feature, 40 bf16 per row: 80 bytes, 16-byte aligned reads) */
-#define XS 40
-
-/* dW = X^T D over samples [row0, row0 + 256): X [rows][KIN], D [rows][128]
- * bf16; writes pw[k * 128 + n] and the bias gradient pb[n] = sum_s D[s][n] */
-template <int KIN>
-__device__ __forceinline__ void wgrad_layer(const __bf16 *X, const __bf16 *D, long row0,
-                                            float *pw, float *pb, __bf16 *xt, __bf16 *dt)
-{
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, i16 = lane & 15;
-    constexpr int IBW = KIN / 64;
-    constexpr int KC = KIN / 8;
-    f32x4 acc[IBW][8];
+    /* output layer in FP32: this wave's share of h3 W4, then the four waves' */
+    float wo[2][12];
 #pragma unroll
-    for (int ii = 0; ii < IBW; ii++)
+    for (int nb = 0; nb < 2; nb++) {
+        const f32x4 *wp = (const f32x4 *)(net.w4 + 3 * (nw + 16 * nb));
 #pragma unroll
-        for (int nb = 0; nb < 8; nb++) acc[ii][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.f;
-    for (int s0 = 0; s0 < 256; s0 += 32) {
-        for (int c = tid; c < 32 * KC; c += 256) {
-            const int s = c / KC, k8 = c % KC;
-            const bf16x8 v = *(const bf16x8 *)(X + (row0 + s0 + s) * KIN + k8 * 8);
-#pragma unroll
-            for (int t = 0; t < 8; t++) xt[(k8 * 8 + t) * XS + s] = v[t];
-        }
-        for (int c = tid; c < 32 * 16; c += 256) {
-            const int s = c / 16, n8 = c % 16;
-            const bf16x8 v = *(const bf16x8 *)(D + (row0 + s0 + s) * NH + n8 * 8);
-#pragma unroll
-            for (int t = 0; t < 8; t++) dt[(n8 * 8 + t) * XS + s] = v[t];
-        }
-        __syncthreads();
-        bf16x8 bfr[8];
-#pragma unroll
-        for (int nb = 0; nb < 8; nb++)
-            bfr[nb] = *(const bf16x8 *)(dt + (nb * 16 + i16) * XS + 8 * g);
-#pragma unroll
-        for (int ii = 0; ii < IBW; ii++) {
-            const int ib = w * IBW + ii;
-            const bf16x8 a = *(const bf16x8 *)(xt + (ib * 16 + i16) * XS + 8 * g);
-#pragma unroll
-            for (int nb = 0; nb < 8; nb++) acc[ii][nb] = mfma(a, bfr[nb], acc[ii][nb]);
-        }
-        if (tid < NH)
-            for (int s = 0; s < 32; s++) bsum += (float)dt[tid * XS + s];
-        __syncthreads();
+        for (int k = 0; k < 12; k++) wo[nb][k] = wp[k / 4][k % 4];
     }
 #pragma unroll
-    for (int ii = 0; ii < IBW; ii++)
+    for (int mb = 0; mb < 4; mb++)
 #pragma unroll
-        for (int nb = 0; nb < 8; nb++)
+        for (int c = 0; c < 3; c++) {
+            float o = 0.f;
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) o = fmaf(acc[nb][mb][r], wo[nb][3 * r + c], o);
+            o += __shfl_xor(o, 16, 64);
+            o += __shfl_xor(o, 32, 64);
+            if (g == 0) red[w][mb * 16 + i16][c] = o;
+        }
+    __syncthreads();
+    if (w == 0) {
+        double e2 = 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            float d = 0.f;
+            if (valid) {
+                const float o = ((red[0][lane][c] + red[1][lane][c]) +
+                                 (red[2][lane][c] + red[3][lane][c])) + net.b4[c];
+                const float e = o - dsy[3 * (s0 + row) + c];
+                e2 += (double)e * (double)e;
+                d = 2.0f * e * inv3n;
+            }
+            dl[lane][c] = d;
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) e2 += __shfl_xor(e2, off, 64);
+        if (lane == 0) lossp[blockIdx.x] = e2;
+    }
+    __syncthreads();
+    float *sp = small + (size_t)blockIdx.x * S_TOTAL;
+    if (threadIdx.x < 3) {
+        float b = 0.f;
+        for (int m = 0; m < 64; m++) b += dl[m][threadIdx.x];
+        sp[S_B4 + threadIdx.x] = b;
+    }
+
+    /* dZ3 = (dL/dout W4^T) gelu'(z3), and the output layer's gradient */
+    f32x4 bs[2];                        /* bias gradients of the lane's samples */
+    auto bias_out = [&](float *o) {
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int k = (w * IBW + ii) * 16 + 4 * g + r;
-                const int n = nb * 16 + i16;
-                pw[k * NH + n] = acc[ii][nb][r];
+                const float v = row_sum(bs[nb][r]);
+                if (i16 == 0) o[nw + 16 * nb + r] = v;
             }
-    if (tid < NH) pb[tid] = bsum;
+    };
+    {
+        float w4g[2][12];
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++) {
+            bs[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 12; k++) w4g[nb][k] = 0.f;
+        }
+#pragma unroll
+        for (int mb = 0; mb < 4; mb++) {
+            const int m = mb * 16 + i16;
+            const float d0 = dl[m][0], d1 = dl[m][1], d2 = dl[m][2];
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++) {
+                f32x4 dz;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float h = acc[nb][mb][r];
+                    w4g[nb][3 * r] = fmaf(h, d0, w4g[nb][3 * r]);
+                    w4g[nb][3 * r + 1] = fmaf(h, d1, w4g[nb][3 * r + 1]);
+                    w4g[nb][3 * r + 2] = fmaf(h, d2, w4g[nb][3 * r + 2]);
+                    const float dh = fmaf(d2, wo[nb][3 * r + 2],
+                                          fmaf(d1, wo[nb][3 * r + 1], d0 * wo[nb][3 * r]));
+                    dz[r] = dh * g3[nb][mb][r];
+                }
+                const bf16x4 b = train_store(dz, ta, tb.dz3 + at, m, nw + 16 * nb);
+#pragma unroll
+                for (int r = 0; r < 4; r++) bs[nb][r] += (float)b[r];
+            }
+        }
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+            for (int k = 0; k < 12; k++) {
+                const float v = row_sum(w4g[nb][k]);
+                if (i16 == 0) sp[S_W4 + 3 * (nw + 16 * nb) + k] = v;
+            }
+        bias_out(sp + S_B3);
+    }
+    /* dZ2 = (dZ3 W3^T) gelu'(z2), dZ1 = (dZ2 W2^T) gelu'(z1) */
+    auto back = [&](const WFrag<4> &wb, const __bf16 *from, const f32x4 (&gd)[2][4], __bf16 *tile,
+                    __bf16 *buf) {
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++) {
+            bs[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int mb = 0; mb < 4; mb++) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        __syncthreads();
+        train_layer<4, TS>(acc, wb, from);
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+            for (int mb = 0; mb < 4; mb++) {
+                f32x4 v;
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = acc[nb][mb][r] * gd[nb][mb][r];
+                const bf16x4 b = train_store(v, tile, buf + at, mb * 16 + i16, nw + 16 * nb);
+#pragma unroll
+                for (int r = 0; r < 4; r++) bs[nb][r] += (float)b[r];
+            }
+    };
+    back(f2, ta, g2, tc, tb.dz2);
+    bias_out(sp + S_B2);
+    back(f3, tc, g1, nullptr, tb.dz1);
+    bias_out(sp + S_B1);
 }
 
-/* per-chunk parameter gradients: blockIdx.x = chunk of 256 samples,
- * blockIdx.y = layer (0: W1 b1, 1: W2 b2, 2: W3 b3, 3: W4 b4).  part has
- * one row of P_TOTAL floats per chunk. */
-__global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, const __bf16 *dz1,
-        const __bf16 *dz2, const __bf16 *dz3, const float *dout, float *part)
+/* dW = X^T D of layers 1-3 over a chunk of samples (blockIdx.x; chunk rows,
+ * a multiple of 64): blockIdx.y = 64 inputs of a layer (0-3: layer 1, 4-5:
+ * layer 2, 6-7: layer 3) and all 128 outputs, a wave on 32 x 64 of them.  Both
+ * operands come straight from the batch buffers (16 bytes a lane, no
+ * LDS).  part has one row of P_TOTAL floats per chunk.
+ * Bound: latency of the operand reads (2048 MFMAs a chunk of 256, under a
+ * microsecond on the chip).  With the operands transposed through LDS in
+ * two-byte writes and a block per layer and 256 samples: 73 us a batch of
+ * 16,384; this 15, with half the partial sums (16 inputs x 128 outputs to a
+ * wave, which reads half as much again: 21). */
+__global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, int chunk, float *part)
 {
-    __shared__ __attribute__((aligned(16))) __bf16 xt[NIN * XS];
-    __shared__ __attribute__((aligned(16))) __bf16 dt[NH * XS];
-    const long row0 = (long)blockIdx.x * 256;
-    float *pr = part + (size_t)blockIdx.x * P_TOTAL;
-    const int layer = blockIdx.y;
-    if (layer == 0) {
-        wgrad_layer<NIN>(tb.h0, dz1, row0, pr + P_W1, pr + P_B1, xt, dt);
-    } else if (layer == 1) {
-        wgrad_layer<NH>(tb.h1, dz2, row0, pr + P_W2, pr + P_B2, xt, dt);
-    } else if (layer == 2) {
-        wgrad_layer<NH>(tb.h2, dz3, row0, pr + P_W3, pr + P_B3, xt, dt);
-    } else {
-        /* output layer, FP32: dW4[n][c] = sum_s h3[s][n] dout[s][c] */
-        const int tid = threadIdx.x, n = tid & 127, half = tid >> 7;
-        float a0 = 0.f, a1 = 0.f;
-        for (int s = 0; s < 256; s++) {
-            const long r = row0 + s;
-            const float h = tb.h3[r * NH + n];
-            if (half == 0) {
-                a0 = fmaf(h, dout[3 * r], a0);
-                a1 = fmaf(h, dout[3 * r + 1], a1);
-            } else {
-                a0 = fmaf(h, dout[3 * r + 2], a0);
-            }
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
+    const int y = blockIdx.y;
+    const __bf16 *X = y < 4 ? tb.h0 : (y < 6 ? tb.h1 : tb.h2);
+    const __bf16 *D = y < 4 ? tb.dz1 : (y < 6 ? tb.dz2 : tb.dz3);
+    const int k0 = 64 * (y < 4 ? y : (y < 6 ? y - 4 : y - 6)) + 32 * (w & 1);
+    const int n0 = 64 * (w >> 1);
+    const int nf = y < 4 ? NIN : NH;
+    const long t0 = (long)blockIdx.x * (chunk / 64), tn = tb.rows / 64;
+    const long t1 = t0 + chunk / 64 < tn ? t0 + chunk / 64 : tn;
+    const __bf16 *xp = X + (k0 + i16) * 64 + 8 * g, *dp = D + (n0 + i16) * 64 + 8 * g;
+    f32x4 acc[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++) acc[i][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (long t = t0; t < t1; t++) {
+        bf16x8 a[2][2], b[2][4];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                a[q][i] = *(const bf16x8 *)(xp + (t * nf + 16 * i) * 64 + 32 * q);
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++)
+                b[q][nb] = *(const bf16x8 *)(dp + (t * NH + 16 * nb) * 64 + 32 * q);
         }
-        if (half == 0) {
-            pr[P_W4 + 3 * n] = a0;
-            pr[P_W4 + 3 * n + 1] = a1;
-        } else {
-            pr[P_W4 + 3 * n + 2] = a0;
-        }
-        if (tid < 3) {
-            float b = 0.f;
-            for (int s = 0; s < 256; s++) b += dout[3 * (row0 + s) + tid];
-            pr[P_B4 + tid] = b;
-        }
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int nb = 0; nb < 4; nb++) acc[i][nb] = mfma(a[q][i], b[q][nb], acc[i][nb]);
     }
+    float *pw = part + (size_t)blockIdx.x * P_TOTAL + (y < 4 ? P_W1 : (y < 6 ? P_W2 : P_W3));
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                pw[(k0 + 16 * i + 4 * g + r) * NH + n0 + nb * 16 + i16] = acc[i][nb][r];
 }
 
 enum { ADAM_STEP = 0, ADAM_GRAD_ONLY = 1, ADAM_FRAG_ONLY = 2 };
 
-/* sum of the chunk partials in chunk order (deterministic), then the
- * mode's action: an Adam step (Kingma & Ba 2015, bias-corrected), the
- * gradient only, or nothing; finally the bf16 fragments of the weight. */
+/* parameters of layers 1-3's weights come first in the optimiser's blocks, a
+ * thread each; the small ones (biases and output layer) follow, a wave each */
+#define BIG_TOTAL (NIN * NH + 2 * NH * NH)
+#define BIG_BLOCKS (BIG_TOTAL / 256)
+static_assert(BIG_TOTAL % 256 == 0, "whole blocks of weights");
+
+/* The gradient of every parameter from its partial sums in a fixed order
+ * (deterministic): weights over the chunks in chunk order, small parameters
+ * over the blocks of 64 samples with lane-strided sums and a lane tree; then
+ * the mode's action: an Adam step (Kingma & Ba 2015, bias-corrected), the
+ * gradient only, or nothing; finally the bf16 fragments of the weight.  With
+ * lacc the last wave adds the loss partials to it (the same kind of sum). */
 __global__ void __launch_bounds__(256) k_mlp_adam(float *params, float *am, float *av,
-        const float *part, int nchunks, int mode, float lr, float b1, float b2, float eps,
-        float bc1, float bc2, float *gout, bf16x8 *frag)
+        const float *part, int nchunks, const float *small, int nsmall, const double *lossp,
+        double *lacc, int mode, float lr, float b1, float b2, float eps, float bc1, float bc2, float *gout, bf16x8 *frag)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= P_TOTAL) return;
+    int p;
+    float gs = 0.f;
+    if (blockIdx.x < BIG_BLOCKS) {
+        const int e = blockIdx.x * 256 + threadIdx.x;
+        p = e < NIN * NH ? P_W1 + e
+                         : (e < NIN * NH + NH * NH ? P_W2 + e - NIN * NH
+                                                   : P_W3 + e - NIN * NH - NH * NH);
+        if (mode != ADAM_FRAG_ONLY) {
+#pragma unroll 8
+            for (int c = 0; c < nchunks; c++) gs += part[(size_t)c * P_TOTAL + p];
+        }
+    } else {
+        const int q = (blockIdx.x - BIG_BLOCKS) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+        if (q == S_TOTAL && lacc) {
+            double s = 0.0;
+            for (int b = lane; b < nsmall; b += 64) s += lossp[b];
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+            if (lane == 0) *lacc += s;
+        }
+        if (q >= S_TOTAL) return;
+        p = q < S_B2 ? P_B1 + q
+                     : (q < S_B3 ? P_B2 + q - S_B2
+                                 : (q < S_W4 ? P_B3 + q - S_B3
+                                             : (q < S_B4 ? P_W4 + q - S_W4 : P_B4 + q - S_B4)));
+        if (mode != ADAM_FRAG_ONLY) {
+            for (int b = lane; b < nsmall; b += 64) gs += small[(size_t)b * S_TOTAL + q];
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) gs += __shfl_xor(gs, o, 64);
+        }
+        if (lane != 0) return;
+    }
     float w = params[p];
     if (mode != ADAM_FRAG_ONLY) {
-        float gs = 0.f;
-        for (int c = 0; c < nchunks; c++) gs += part[(size_t)c * P_TOTAL + p];
         if (mode == ADAM_GRAD_ONLY) {
             gout[p] = gs;
             return;
@@ -641,16 +783,6 @@ __global__ void __launch_bounds__(256) k_mlp_adam(float *params, float *am, floa
         const int e = p - P_W3;
         fr[FR_W3F * 8 + frag_fwd(e / NH, e % NH, NH / 32)] = wb;
         fr[FR_W3B * 8 + frag_bwd(e / NH, e % NH)] = wb;
-    }
-}
-
-/* sum of the loss partials in block order, added to *acc */
-__global__ void k_mlp_loss_acc(const double *lossp, int nblocks, double *acc)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int b = 0; b < nblocks; b++) s += lossp[b];
-        *acc += s;
     }
 }
 
@@ -710,9 +842,8 @@ __global__ void __launch_bounds__(256, 2) k_mlp_check(TrackArgs a, int first)
     }
     const bool chk = live && moving && fb == 0;
     float o[3] = {0.f, 0.f, 0.f};
-    TrainBufs tb = {};
     if (__any(chk))
-        mlp_wave<MLP_EVAL>(net, px, py, pz, tiles + (threadIdx.x >> 6) * TILE, o, tb, 0);
+        mlp_wave(net, px, py, pz, tiles + (threadIdx.x >> 6) * TILE, o);
     if (chk) {
         const float b0z = (float)a.f.b0z;
         float bx, by, bz;
@@ -803,7 +934,6 @@ __global__ void __launch_bounds__(256, 2) k_track_mlp(TrackArgs a)
     const float dtf = (float)a.dt;
     const float hf = (float)(a.qm * (0.5 * a.dt));
     const float b0z = (float)a.f.b0z;
-    TrainBufs tb = {};
     __syncthreads();
 
     int ntp = a.ntp0;
@@ -811,7 +941,7 @@ __global__ void __launch_bounds__(256, 2) k_track_mlp(TrackArgs a)
         const bool moving = live && (esc == 0 || a.bc == 0);
         float o[3] = {0.f, 0.f, 0.f};
         if (__any(moving))
-            mlp_wave<MLP_EVAL>(net, (float)p.x, (float)p.y, (float)p.z, tile, o, tb, 0);
+            mlp_wave(net, (float)p.x, (float)p.y, (float)p.z, tile, o);
         EmfF e;
         e.ex = 0.f; e.ey = 0.f; e.ez = 0.f;
         e.bx = net.scale * o[0];
@@ -874,9 +1004,8 @@ struct MlpState {
     long rows_cap = 0;
     __bf16 *h0 = nullptr, *h1 = nullptr, *h2 = nullptr;
     __bf16 *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
-    float *g1 = nullptr, *g2 = nullptr, *g3 = nullptr, *h3 = nullptr, *dout = nullptr;
     double *lossp = nullptr, *lacc = nullptr;
-    float *part = nullptr, *grad = nullptr;
+    float *part = nullptr, *small = nullptr, *grad = nullptr;
     /* training set (or the points of a gradient call) */
     long ds_cap = 0;
     float *dsx = nullptr, *dsy = nullptr;
@@ -888,8 +1017,8 @@ void tp_mlp_release(tp_ctx *c)
     if (!m) return;
     void *ptrs[] = {m->params, m->am, m->av, m->q, m->frag, m->fb, m->nfb, m->idx, m->cnt,
                     m->h0, m->h1,
-                    m->h2, m->dz1, m->dz2, m->dz3, m->g1, m->g2, m->g3, m->h3, m->dout,
-                    m->lossp, m->lacc, m->part, m->grad, m->dsx, m->dsy};
+                    m->h2, m->dz1, m->dz2, m->dz3, m->lossp, m->lacc, m->part, m->small,
+                    m->grad, m->dsx, m->dsy};
     for (void *p : ptrs) (void)hipFree(p);
     delete m;
     c->mlp = nullptr;
@@ -927,11 +1056,21 @@ static int dalloc(void **p, size_t bytes)
     return TP_OK;
 }
 
+/* Rows of a weight-gradient chunk: 256, doubled until there are at most 32
+ * chunks.  32 chunks are 256 blocks, one for each compute unit, and their
+ * partial sums 8.5 MB whatever the batch (64 of 256 rows for 16,384 samples
+ * were 17 MB to write and read again). */
+static int chunk_rows(long rows)
+{
+    long c = 256;
+    while ((rows + c - 1) / c > 32) c *= 2;
+    return (int)c;
+}
+
 static int ensure_rows(MlpState *m, long rows)
 {
     if (rows <= m->rows_cap) return TP_OK;
-    void *old[] = {m->h0, m->h1, m->h2, m->dz1, m->dz2, m->dz3, m->g1, m->g2, m->g3,
-                   m->h3, m->dout, m->lossp, m->part};
+    void *old[] = {m->h0, m->h1, m->h2, m->dz1, m->dz2, m->dz3, m->lossp, m->part, m->small};
     for (void *p : old) (void)hipFree(p);
     m->rows_cap = 0;
     const size_t r = (size_t)rows;
@@ -942,13 +1081,10 @@ static int ensure_rows(MlpState *m, long rows)
     rc |= dalloc((void **)&m->dz1, r * NH * 2);
     rc |= dalloc((void **)&m->dz2, r * NH * 2);
     rc |= dalloc((void **)&m->dz3, r * NH * 2);
-    rc |= dalloc((void **)&m->g1, r * NH * 4);
-    rc |= dalloc((void **)&m->g2, r * NH * 4);
-    rc |= dalloc((void **)&m->g3, r * NH * 4);
-    rc |= dalloc((void **)&m->h3, r * NH * 4);
-    rc |= dalloc((void **)&m->dout, r * 3 * 4);
-    rc |= dalloc((void **)&m->lossp, (r / 256) * sizeof(double));
-    rc |= dalloc((void **)&m->part, (r / 256) * (size_t)P_TOTAL * 4);
+    rc |= dalloc((void **)&m->lossp, (r / 64) * sizeof(double));
+    rc |= dalloc((void **)&m->small, (r / 64) * (size_t)S_TOTAL * 4);
+    const size_t chunks = r / 256 < 32 ? r / 256 : 32;
+    rc |= dalloc((void **)&m->part, chunks * (size_t)P_TOTAL * 4);
     if (rc) return TP_E_NOMEM;
     m->rows_cap = rows;
     return TP_OK;
@@ -965,37 +1101,35 @@ static int ensure_ds(MlpState *m, long n)
     return TP_OK;
 }
 
-static TrainBufs bufs_of(const MlpState *m)
+static TrainBufs bufs_of(const MlpState *m, long rows)
 {
     TrainBufs t;
     t.h0 = m->h0; t.h1 = m->h1; t.h2 = m->h2;
-    t.g1 = m->g1; t.g2 = m->g2; t.g3 = m->g3; t.h3 = m->h3;
+    t.dz1 = m->dz1; t.dz2 = m->dz2; t.dz3 = m->dz3;
+    t.rows = rows;
     return t;
 }
 
 /* forward + backward + chunk gradients over rows [0, rows) of batch
  * samples s0.. of the set; then the optimiser kernel in the given mode */
 static int train_pass(tp_ctx *c, long s0, int nvalid, long rows, int mode, float lr, float b1,
-                      float b2, float eps, float bc1, float bc2, float *gout)
+                      float b2, float eps, float bc1, float bc2, float *gout, double *lacc)
 {
     MlpState *m = c->mlp;
     const MlpNet net = net_of(m);
-    const TrainBufs tb = bufs_of(m);
-    const int nblk = (int)(rows / 256);
+    const TrainBufs tb = bufs_of(m, rows);
+    const int nblk = (int)(rows / 64), chunk = chunk_rows(rows);
+    const int nchunks = (int)((rows + chunk - 1) / chunk);
     const float inv3n = (float)(1.0 / (3.0 * (double)nvalid));
-    hipLaunchKernelGGL(k_mlp_train_fwd, dim3(nblk), dim3(256), 0, c->stream, net, m->dsx,
-                       m->dsy, s0, nvalid, inv3n, tb, m->dout, m->lossp);
+    hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(256), 0, c->stream, net, m->dsx, m->dsy, s0,
+                       nvalid, inv3n, tb, m->small, m->lossp);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_train_bwd, dim3(nblk), dim3(256), 0, c->stream, net, tb,
-                       (const float *)m->dout, m->dz3, m->dz2, m->dz1);
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(nchunks, 8), dim3(256), 0, c->stream, tb, chunk, m->part);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(nblk, 4), dim3(256), 0, c->stream, tb,
-                       (const __bf16 *)m->dz1, (const __bf16 *)m->dz2, (const __bf16 *)m->dz3,
-                       (const float *)m->dout, m->part);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_adam, dim3((P_TOTAL + 255) / 256), dim3(256), 0, c->stream,
-                       m->params, m->am, m->av, (const float *)m->part, nblk, mode, lr, b1, b2,
-                       eps, bc1, bc2, gout, m->frag);
+    hipLaunchKernelGGL(k_mlp_adam, dim3(BIG_BLOCKS + S_TOTAL / 4 + 1), dim3(256), 0, c->stream,
+                       m->params, m->am, m->av, (const float *)m->part, nchunks,
+                       (const float *)m->small, nblk, (const double *)m->lossp, lacc, mode, lr, b1,
+                       b2, eps, bc1, bc2, gout, m->frag);
     HIPCHK(hipGetLastError());
     return TP_OK;
 }
@@ -1035,9 +1169,11 @@ int tp_gpu_mlp_set(tp_ctx *c, const float *q, const float *params, double scale)
     HIPCHK(hipMemset(m->av, 0, P_TOTAL * 4));
     HIPCHK(hipMemset(m->frag, 0, FR_TOTAL * sizeof(bf16x8)));
     m->scale = (float)scale;
-    hipLaunchKernelGGL(k_mlp_adam, dim3((P_TOTAL + 255) / 256), dim3(256), 0, c->stream,
-                       m->params, m->am, m->av, (const float *)nullptr, 0, (int)ADAM_FRAG_ONLY,
-                       0.f, 0.f, 0.f, 0.f, 1.f, 1.f, (float *)nullptr, m->frag);
+    hipLaunchKernelGGL(k_mlp_adam, dim3(BIG_BLOCKS), dim3(256), 0, c->stream,
+                       m->params, m->am, m->av, (const float *)nullptr, 0,
+                       (const float *)nullptr, 0, (const double *)nullptr, (double *)nullptr,
+                       (int)ADAM_FRAG_ONLY, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f, (float *)nullptr,
+                       m->frag);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     m->set = true;
@@ -1096,12 +1232,9 @@ int tp_gpu_mlp_loss_grad(tp_ctx *c, int n, const float *x, const float *y, float
     if (rc) return rc;
     HIPCHK(hipMemcpyAsync(m->dsx, x, (size_t)n * 12, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(m->dsy, y, (size_t)n * 12, hipMemcpyHostToDevice, c->stream));
-    rc = train_pass(c, 0, n, rows, ADAM_GRAD_ONLY, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f, m->grad);
-    if (rc) return rc;
     HIPCHK(hipMemsetAsync(m->lacc, 0, sizeof(double), c->stream));
-    hipLaunchKernelGGL(k_mlp_loss_acc, dim3(1), dim3(64), 0, c->stream,
-                       (const double *)m->lossp, (int)(rows / 256), m->lacc);
-    HIPCHK(hipGetLastError());
+    rc = train_pass(c, 0, n, rows, ADAM_GRAD_ONLY, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f, m->grad, m->lacc);
+    if (rc) return rc;
     double l = 0.0;
     HIPCHK(hipMemcpyAsync(grad, m->grad, P_TOTAL * 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(&l, m->lacc, sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -1140,7 +1273,6 @@ int tp_gpu_train_surrogate(tp_ctx *c, const tp_mlp_train_params *p, tp_mlp_train
 
     const long spe = ns / p->batch;
     const long total = spe * p->epochs;
-    const int nblk = p->batch / 256;
     double first = 0.0;
     HIPCHK(hipEventRecord(e0, c->stream));
     double pb1 = 1.0, pb2 = 1.0;
@@ -1150,26 +1282,18 @@ int tp_gpu_train_surrogate(tp_ctx *c, const tp_mlp_train_params *p, tp_mlp_train
         pb1 *= p->beta1;
         pb2 *= p->beta2;
         const long s0 = (t % spe) * p->batch;
+        /* the first batch's loss, and the last epoch's mean */
+        if (t == 0 || t == total - spe)
+            HIPCHK(hipMemsetAsync(m->lacc, 0, sizeof(double), c->stream));
         rc = train_pass(c, s0, p->batch, p->batch, ADAM_STEP, (float)lr, (float)p->beta1,
                         (float)p->beta2, (float)p->eps, (float)(1.0 - pb1), (float)(1.0 - pb2),
-                        nullptr);
+                        nullptr, t == 0 || t >= total - spe ? m->lacc : nullptr);
         if (rc) return rc;
         if (t == 0) {
-            HIPCHK(hipMemsetAsync(m->lacc, 0, sizeof(double), c->stream));
-            hipLaunchKernelGGL(k_mlp_loss_acc, dim3(1), dim3(64), 0, c->stream,
-                               (const double *)m->lossp, nblk, m->lacc);
-            HIPCHK(hipGetLastError());
             HIPCHK(hipMemcpyAsync(&first, m->lacc, sizeof(double), hipMemcpyDeviceToHost,
                                   c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
             first /= 3.0 * (double)p->batch;
-        }
-        /* the last epoch's mean loss */
-        if (t == total - spe) HIPCHK(hipMemsetAsync(m->lacc, 0, sizeof(double), c->stream));
-        if (t >= total - spe) {
-            hipLaunchKernelGGL(k_mlp_loss_acc, dim3(1), dim3(64), 0, c->stream,
-                               (const double *)m->lossp, nblk, m->lacc);
-            HIPCHK(hipGetLastError());
         }
     }
     HIPCHK(hipEventRecord(e1, c->stream));

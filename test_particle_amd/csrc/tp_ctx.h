@@ -40,6 +40,8 @@ struct tp_ctx {
     double *gridd = nullptr;                       /* double PIC nodes */
     float *modes32 = nullptr;
     double *modesx = nullptr;                      /* mode rows for the matrix cores */
+    bf16x8 *modesb = nullptr;                      /* the FP32 forms' rows for them */
+    float4 *modesa = nullptr;
     WlcsSys *wl = nullptr;
     State s;
     /* diagnostics of the last run */

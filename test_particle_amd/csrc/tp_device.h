@@ -30,11 +30,13 @@ enum {
     FK_GRID2_TB = 9,  /* PIC grid, two time slices, textbook gather */
     FK_MHD_REF = 10,  /* MHD grids (system 3): float v and B, E = B x v */
     FK_GRIDD_REF = 11,/* PIC grid of double E and B, reference weights */
+    FK_MODES_WAVE = 12 /* FK_MODES in the FP32 step kernel with modes_wave32 */
 };
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 /* A surrogate network on the device (layout in tp_mlp.hip): bfloat16 weight
  * fragments of layers 1-3 in the order the matrix-core kernels read them,
@@ -104,6 +106,12 @@ struct FieldDev {
     double b0z;
     /* the same table for FP32: (kx ky kz phi) / 2 pi, ax ay az 0 per mode */
     const float *modes32;
+    /* and for the FP32 forms' matrix products (modes_wave32): n16 groups of 16
+     * modes, a zero group after them; the group's (k, phi) / 2 pi in three
+     * bfloat16 parts as a B operand, and its amplitudes */
+    const bf16x8 *modesb;
+    const float4 *modesa;
+    int n16;
     MlpNet mlp;
     /* WLCS */
     int nwlcs, ibessel, wlmode;
@@ -904,7 +912,7 @@ __device__ __forceinline__ void get_emf64(const FieldDev &f, double x, double y,
         }
         o.ex = v[0]; o.ey = v[1]; o.ez = v[2];
         o.bx = v[3]; o.by = v[4]; o.bz = v[5];
-    } else if (FK == FK_MODES || FK == FK_MLP) {
+    } else if (FK == FK_MODES || FK == FK_MLP || FK == FK_MODES_WAVE) {
         /* four independent cosines per iteration (instruction-level
          * parallelism for the FP64 FMA chains), summed in mode order */
         double bx = 0.0, by = 0.0, bz = 0.0;
@@ -1116,6 +1124,126 @@ __device__ __forceinline__ void modes_sum32(const float *tab32, int nmodes, floa
         bx = fmaf(m[4], c, bx); by = fmaf(m[5], c, by); bz = fmaf(m[6], c, bz);
     }
     bxo = bx; byo = by; bzo = bz;
+}
+
+/* ------------------------------------------------------------------ */
+/* the FP32 mode sum of a wavefront's points                            */
+/* ------------------------------------------------------------------ */
+/* FP32 sum over the modes at the 64 points of a wavefront, 16 points x 16
+ * modes at a time with v_mfma_f32_16x16x32_bf16 (lane l: j = l & 15, c =
+ * l >> 4): A[j][8c .. 8c+7] of point j, B[8c .. 8c+7][j] of mode j, D rows
+ * 4c .. 4c+3 (points) of column j (mode).  The phase in revolutions is the
+ * product of (x y z 1) and (kx ky kz phi) / 2 pi, one of them to each c, with
+ * every factor split into three bfloat16 parts h + m + l (24 bits and more:
+ * float x exactly, the table from double): the products h m', m h', m m', h l',
+ * l h', m l', l m' first, then h h' added to them, so that only the last sum
+ * rounds at the phase's own size (v_mfma_f32_16x16x16_bf16 with the first four
+ * of the table's eight).  Products are exact, sums FP32.  The lane
+ * then has the phases of one mode at 16 points and adds a_mode cos(phase) into
+ * sums of its own; the 16 lanes of a row are summed at the end.
+ *
+ * Against the sums in 64 bits (1000 modes, kmax 48): rms error of the largest
+ * k's phases 2.2e-5 revolutions at points up to 130, 1.3e-4 up to 1000, of the
+ * field 3.1e-7 and 1.5e-6; a lane per point with FP32 FMAs (modes_sum32) has
+ * 2.2e-5, 1.8e-4, 8.7e-7 and 2.0e-6.
+ * Bound: issue of the cosine (8 cycles), its fraction and three FMAs a mode;
+ * FMAs of vector registers only take 3 cycles, those of modes_sum32 with a
+ * scalar operand 4, and its scalar loads stall a wavefront.  Cycles per 64
+ * points and mode at one / two / four / eight waves a SIMD: 68 / 41 / 35 / 30,
+ * modes_sum32 128 / 64 / 52 / 41. */
+#define MODES_WAVE32_LDS (64 * 4)    /* floats of LDS per wavefront */
+/* modes from which it is used: the splits and the row sums cost as much as
+ * some 70 modes.  262,144 particles x 200 steps, per lane / per wavefront: 64
+ * modes 1.25 / 1.29 ms, 96 modes 1.80 / 1.64, 1000 modes 18.6 / 12.0; 5000
+ * particles: 64 modes 0.52 / 0.56, 1000 modes 9.2 / 4.6. */
+#define MODES_WAVE32_MIN 80
+
+__device__ __forceinline__ s16x4 first4(const bf16x8 &v)
+{
+    const bf16x4 f = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+    return __builtin_bit_cast(s16x4, f);
+}
+
+/* Every lane of the wavefront calls it (uniform control flow); xp is the
+ * wavefront's own MODES_WAVE32_LDS floats of LDS. */
+__device__ __forceinline__ void modes_wave32(const FieldDev &f, float x, float y, float z,
+                                             float *xp, float &bx, float &by, float &bz)
+{
+    const int lane = threadIdx.x & 63, c = lane >> 4, j = lane & 15;
+    *(f32x4 *)(xp + 4 * lane) = f32x4{x, y, z, 1.0f};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    s16x4 ph[4];
+    bf16x8 pl[4];
+    const __bf16 o = (__bf16)0.0f;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const float v = xp[4 * (16 * g + j) + c];
+        const __bf16 h = (__bf16)v;
+        const float r1 = v - (float)h;
+        const __bf16 m = (__bf16)r1;
+        const __bf16 l = (__bf16)(r1 - (float)m);
+        ph[g] = s16x4{__builtin_bit_cast(short, h), 0, 0, 0};
+        /* against the table's h h m m h l m l (phi: h m l) */
+        pl[g] = c == 3 ? bf16x8{o, h, h, o, o, o, o, o} : bf16x8{o, m, h, m, l, h, l, m};
+    }
+    float acc[4][4][3];
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[g][r][0] = acc[g][r][1] = acc[g][r][2] = 0.f;
+    const bf16x8 *mt = f.modesb + lane;
+    const float4 *at = f.modesa + j;
+    bf16x8 mn = *mt;
+    float4 an = *at;
+#pragma unroll 1
+    for (int q = 0; q < f.n16; q++) {
+        const bf16x8 mk = mn;
+        const s16x4 mh = first4(mk);
+        const float4 a = an;
+        mt += 64;
+        at += 16;
+        mn = *mt;                        /* past the end: the zero group */
+        an = *at;
+        f32x4 u[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            u[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[g], mk, f32x4{0.f, 0.f, 0.f, 0.f},
+                                                           0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            u[g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ph[g], mh, u[g], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float cs = __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(u[g][r]));
+                acc[g][r][0] = fmaf(a.x, cs, acc[g][r][0]);
+                acc[g][r][1] = fmaf(a.y, cs, acc[g][r][1]);
+                acc[g][r][2] = fmaf(a.z, cs, acc[g][r][2]);
+            }
+    }
+    /* the sums over the 16 lanes of a row, halving what each lane holds at
+     * every exchange: lane j is left with those of its row's j-th point */
+#pragma unroll
+    for (int h = 8; h >= 1; h /= 2)
+#pragma unroll
+        for (int q = 0; q < h; q++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                float &lo = acc[q >> 2][q & 3][k];
+                const float hi = acc[(q + h) >> 2][(q + h) & 3][k];
+                const bool up = (j & h) != 0;
+                const float keep = up ? hi : lo, send = up ? lo : hi;
+                lo = keep + __shfl_xor(send, h, 64);
+            }
+    *(f32x4 *)(xp + 4 * (16 * (j >> 2) + 4 * c + (j & 3))) =
+        f32x4{acc[0][0][0], acc[0][0][1], acc[0][0][2], 0.f};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    bx = xp[4 * lane]; by = xp[4 * lane + 1]; bz = xp[4 * lane + 2];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 /* ------------------------------------------------------------------ */

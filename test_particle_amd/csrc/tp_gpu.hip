@@ -211,13 +211,29 @@ __device__ __forceinline__ void track_body(const TrackArgs &a)
     int tpts = (TRAJ && live) ? a.traj_pts[i] : 0;
     typename CacheFor<FK>::type gc;
     gc_init(gc);
+    /* the FP32 mode sum is formed by the whole wavefront */
+    constexpr bool WAVE = FK == FK_MODES_WAVE;
+    static_assert(!WAVE || PREC == PREC32, "an FP32 form");
+    __shared__ __align__(16) float points[WAVE ? 4 * MODES_WAVE32_LDS : 4];
+    float *xp = points + (WAVE ? (tid >> 6) * MODES_WAVE32_LDS : 0);
     __syncthreads();
 
     int ntp = a.ntp0;
     for (int j = a.j0; j <= a.j1; j++) {
         int esc_after = esc;
-        if (live && (esc == 0 || a.bc == 0)) {
-            if (PREC == PREC64) {
+        const bool moving = live && (esc == 0 || a.bc == 0);
+        EmfF ew = {};
+        if constexpr (WAVE) {
+            if (__any(moving)) {
+                modes_wave32(a.f, (float)p.x, (float)p.y, (float)p.z, xp, ew.bx, ew.by, ew.bz);
+                ew.bz = (float)a.f.b0z + ew.bz;
+            }
+        }
+        if (moving) {
+            if constexpr (WAVE) {
+                boris_push32(ew, p, fux, fuy, fuz, a.dt, dtf, hf);
+                p.ux = fux; p.uy = fuy; p.uz = fuz;
+            } else if (PREC == PREC64) {
                 if (PUSH == TP_PUSH_WIRZ) wirz_step64<FK>(a.f, gc, p, a.dt, a.qm);
                 else boris_step64<FK>(a.f, gc, p, a.dt, a.qm);
             } else {
@@ -314,6 +330,14 @@ __global__ void __launch_bounds__(256) k_track(TrackArgs a)
 template <int PUSH, int FK, int PREC, bool TRAJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 k_track_w3(TrackArgs a)
+{
+    track_body<PUSH, FK, PREC, TRAJ>(a);
+}
+
+/* and for 4 (128 VGPRs) */
+template <int PUSH, int FK, int PREC, bool TRAJ>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_track_w4(TrackArgs a)
 {
     track_body<PUSH, FK, PREC, TRAJ>(a);
 }
@@ -516,6 +540,8 @@ static void launch_track(dim3 g, dim3 b, size_t sh, hipStream_t s, const TrackAr
     if constexpr ((PREC == PREC32 && (FK == FK_GRID2_REF || FK == FK_GRID2_TB)) ||
                   (PUSH == TP_PUSH_WIRZ && (FK == FK_GRID_REF || FK == FK_MHD_REF)))
         hipLaunchKernelGGL((k_track_w3<PUSH, FK, PREC, TRAJ>), g, b, sh, s, a);
+    else if constexpr (FK == FK_MODES_WAVE)
+        hipLaunchKernelGGL((k_track_w4<PUSH, FK, PREC, TRAJ>), g, b, sh, s, a);
     else
         hipLaunchKernelGGL((k_track<PUSH, FK, PREC, TRAJ>), g, b, sh, s, a);
 }
@@ -548,6 +574,8 @@ static track_fn pick_track(int fk, int push, int prec, bool traj)
     case FK_GRID_REF: return pick_track_fk<FK_GRID_REF>(push, prec, traj);
     case FK_GRID_TB: return pick_track_fk<FK_GRID_TB>(push, prec, traj);
     case FK_MODES: return pick_track_fk<FK_MODES>(push, prec, traj);
+    case FK_MODES_WAVE: return traj ? launch_track<TP_PUSH_BORIS, FK_MODES_WAVE, PREC32, true>
+                                    : launch_track<TP_PUSH_BORIS, FK_MODES_WAVE, PREC32, false>;
     case FK_WLCS: return pick_track_fk<FK_WLCS>(push, prec, traj);
     case FK_GRID2_REF: return pick_track_fk<FK_GRID2_REF>(push, prec, traj);
     case FK_GRID2_TB: return pick_track_fk<FK_GRID2_TB>(push, prec, traj);
@@ -694,6 +722,8 @@ static void free_field(tp_ctx *c)
     (void)hipFree(c->modes); c->modes = nullptr;
     (void)hipFree(c->modes32); c->modes32 = nullptr;
     (void)hipFree(c->modesx); c->modesx = nullptr;
+    (void)hipFree(c->modesb); c->modesb = nullptr;
+    (void)hipFree(c->modesa); c->modesa = nullptr;
     (void)hipFree(c->wl); c->wl = nullptr;
     (void)hipFree(c->gridd); c->gridd = nullptr;
     c->have_field = false;
@@ -1389,6 +1419,61 @@ int tp_gpu_set_field_wlcs_table(tp_ctx *c, int nwlcs, const double *tab, int ibe
     return TP_OK;
 }
 
+/* v's next bfloat16 part (to nearest, ties to even), taken off v */
+static unsigned short take_bf16(double &v)
+{
+    const float w = (float)v;
+    unsigned u;
+    memcpy(&u, &w, sizeof(u));
+    u = (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
+    float h;
+    memcpy(&h, &u, sizeof(h));
+    v -= (double)h;
+    return (unsigned short)(u >> 16);
+}
+
+/* the tables of modes_wave32 */
+static int modes_parts(tp_ctx *c, int nmodes, const double *rows)
+{
+    const int n16 = (nmodes + 15) / 16;
+    const size_t nb = (size_t)512 * (n16 + 1), na = (size_t)64 * (n16 + 1);
+    unsigned short *tb = (unsigned short *)calloc(nb, sizeof(unsigned short));
+    float *ta = (float *)calloc(na, sizeof(float));
+    if (!tb || !ta) { free(tb); free(ta); return TP_E_NOMEM; }
+    const double inv2pi = 1.0 / (2.0 * TP_PI);
+    for (int m = 0; m < nmodes; m++) {
+        const double *r = rows + 7 * m;
+        for (int q = 0; q < 4; q++) {
+            double v = r[q < 3 ? q : 6] * inv2pi;
+            const unsigned short h = take_bf16(v), md = take_bf16(v), l = take_bf16(v);
+            unsigned short *o = tb + 512 * (size_t)(m / 16) + 8 * (16 * q + m % 16);
+            if (q < 3) {
+                const unsigned short p[8] = {h, h, md, md, h, l, md, l};
+                memcpy(o, p, sizeof(p));
+            } else {
+                o[0] = h; o[1] = md; o[2] = l;
+            }
+        }
+        for (int q = 0; q < 3; q++) ta[64 * (size_t)(m / 16) + 4 * (m % 16) + q] = (float)r[3 + q];
+    }
+    int rc = TP_OK;
+    if (hipMalloc(&c->modesb, nb * sizeof(unsigned short)) != hipSuccess) {
+        c->modesb = nullptr;
+        rc = TP_E_NOMEM;
+    } else if (hipMalloc(&c->modesa, na * sizeof(float)) != hipSuccess) {
+        c->modesa = nullptr;
+        rc = TP_E_NOMEM;
+    } else if (hipMemcpy(c->modesb, tb, nb * sizeof(unsigned short), hipMemcpyHostToDevice) !=
+                   hipSuccess ||
+               hipMemcpy(c->modesa, ta, na * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
+        rc = TP_E_HIP;
+    }
+    free(tb);
+    free(ta);
+    c->f.n16 = n16;
+    return rc;
+}
+
 int tp_gpu_set_field_modes(tp_ctx *c, int nmodes, const double *rows, double b0z)
 {
     if (!c || nmodes < 0 || (nmodes > 0 && !rows)) return TP_E_ARG;
@@ -1439,10 +1524,14 @@ int tp_gpu_set_field_modes(tp_ctx *c, int nmodes, const double *rows, double b0z
         free(tx);
         HIPCHK(e);
         c->f.nquads = nquads;
+        int rc = modes_parts(c, nmodes, rows);
+        if (rc) return rc;
     }
     c->f.nmodes = nmodes;
     c->f.modes = c->modes;
     c->f.modesx = c->modesx;
+    c->f.modesb = c->modesb;
+    c->f.modesa = c->modesa;
     c->f.modes32 = c->modes32;
     c->f.b0z = b0z;
     c->f.kind = FK_MODES;
@@ -1627,8 +1716,11 @@ static int run_check(const tp_ctx *c, const tp_track_params *p, track_fn *fn, bo
     if (*mlp && (p->pusher != TP_PUSH_BORIS || p->precision != TP_FP32_MIXED)) return TP_E_ARG;
     if (*mlp && c->traj_nout > 0) return TP_E_ARG;
     /* surrogate field: the exact-field kernel runs the particles that fell back */
-    *fn = pick_track(*mlp ? FK_MODES : field_kind(c), p->pusher, p->precision,
-                     c->traj_nout > 0);
+    int fk = *mlp ? FK_MODES : field_kind(c);
+    if (fk == FK_MODES && p->precision == TP_FP32_MIXED && p->pusher == TP_PUSH_BORIS &&
+        c->f.nmodes >= MODES_WAVE32_MIN)
+        fk = FK_MODES_WAVE;
+    *fn = pick_track(fk, p->pusher, p->precision, c->traj_nout > 0);
     return *fn ? TP_OK : TP_E_ARG;
 }
 

@@ -842,12 +842,19 @@ __global__ void __launch_bounds__(256, 2) k_mlp_check(TrackArgs a, int first)
     }
     const bool chk = live && moving && fb == 0;
     float o[3] = {0.f, 0.f, 0.f};
-    if (__any(chk))
-        mlp_wave(net, px, py, pz, tiles + (threadIdx.x >> 6) * TILE, o);
+    float bx = 0.f, by = 0.f, bz = 0.f;
+    if (__any(chk)) {
+        __bf16 *tile = tiles + (threadIdx.x >> 6) * TILE;
+        mlp_wave(net, px, py, pz, tile, o);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (a.f.nmodes >= MODES_WAVE32_MIN)
+            modes_wave32(a.f, px, py, pz, (float *)tile, bx, by, bz);
+        else
+            modes_sum32(a.f.modes32, a.f.nmodes, px, py, pz, bx, by, bz);
+    }
     if (chk) {
         const float b0z = (float)a.f.b0z;
-        float bx, by, bz;
-        modes_sum32(a.f.modes32, a.f.nmodes, px, py, pz, bx, by, bz);
         bz += b0z;
         const float dx = net.scale * o[0] - bx, dy = net.scale * o[1] - by;
         const float dz = fmaf(net.scale, o[2], b0z) - bz;

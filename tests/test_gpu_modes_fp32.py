@@ -1,0 +1,66 @@
+"""The FP32 mode sum of a wavefront on the matrix cores against 64 bits: one
+Boris step in a field of B alone turns u by an angle of |B| h, so the momentum
+after a step gives the field the step used.  Table and wavefront edges, and
+both sides of the rule that chooses it (80 modes)."""
+import numpy as np
+import pytest
+
+from test_particle_amd import abi
+from test_particle_amd.fields import eval_modes_numpy, mode_table
+from test_particle_amd.particles import init_particles
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    from test_particle_amd.gpu import Tracker
+    t = Tracker(0)
+    yield t
+    t.close()
+
+
+@pytest.mark.parametrize("modes", [79, 80, 81, 96, 97, 1000])
+@pytest.mark.parametrize("n", [1, 63, 64, 257])
+def test_one_step(gpu, modes, n):
+    rows = mode_table(modes, kmin=0.05, kmax=50.0, rms=0.5, seed=71)
+    p = init_particles(n, (0, 0, 0), (100, 100, 100), 0.5, seed=72)
+    dt = 0.2
+    prm = abi.make_params(dt=dt, estep=1, lo=(0, 0, 0), hi=(100, 100, 100),
+                          pusher=abi.TP_PUSH_BORIS, precision=abi.TP_FP32_MIXED,
+                          bc_flag=abi.TP_BC_NONE)
+    gpu.set_field_modes(rows, 1.0)
+    r = gpu.track_fixed(prm, p)["ptl"]
+    b = eval_modes_numpy(rows, p[:, :3], 1.0)
+    u = p[:, 4:7]
+    g = np.sqrt(1 + (u * u).sum(1, keepdims=True))
+    t = 0.5 * dt / g * b
+    s = 2 * t / (1 + (t * t).sum(1, keepdims=True))
+    un = u + np.cross(u + np.cross(u, t), s)
+    # momentum rounding: 2^-24 in each of some 10 operations; field: float
+    # positions up to 100 (ulp 2^-17) shift the phases of kmax = 50 by up to
+    # 50 * 3 * 2^-18 = 6e-4, times the amplitude of those modes (k^-5/3: below
+    # 1e-3 of rms) -- 1e-6 of |B| in all, times |u| dt / g
+    assert np.abs(r[:, 4:7] - un).max() < 3e-6
+    x = p[:, :3] + un * dt / np.sqrt(1 + (un * un).sum(1, keepdims=True))
+    assert np.abs(r[:, :3] - x).max() < 3e-6
+
+
+def test_open_boundary_and_short_wavefronts(gpu):
+    """Particles that leave stop; those that stay do not depend on which others
+    share their wavefront."""
+    rows = mode_table(100, kmin=0.1, kmax=10.0, rms=0.5, seed=73)
+    lo, hi = (0, 0, 0), (4, 4, 4)
+    p = init_particles(300, lo, hi, 0.6, seed=74)
+    prm = abi.make_params(dt=0.1, estep=200, lo=lo, hi=hi, pusher=abi.TP_PUSH_BORIS,
+                          precision=abi.TP_FP32_MIXED, bc_flag=abi.TP_BC_OPEN, nt_out=2,
+                          emin=1e-4, emax=10.0)
+    gpu.set_field_modes(rows, 1.0)
+    r = gpu.track_fixed(prm, p)
+    out = r["nsteps"] < 201
+    # nsteps counts from 1: a particle that leaves at step j has j + 1
+    assert out.any() and r["remain"][-1] == 300 - (r["nsteps"] <= 101).sum()
+    perm = np.random.default_rng(75).permutation(300)[:77]
+    q = gpu.track_fixed(prm, p[perm])
+    assert np.array_equal(q["ptl"], r["ptl"][perm])
+    assert np.array_equal(q["nsteps"], r["nsteps"][perm])

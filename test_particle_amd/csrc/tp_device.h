@@ -1546,4 +1546,151 @@ __device__ __forceinline__ void boris_step32(const FieldDev &f, GC &gc, Ptl &p,
     boris_push32(e, p, ux, uy, uz, dt, dtf, hf);
 }
 
+/* ------------------------------------------------------------------ */
+/* quads of lanes                                                       */
+/* ------------------------------------------------------------------ */
+/* the value of lane A, B, C, D of the quad in its lanes 0, 1, 2, 3 (DPP
+ * quad_perm, no LDS) */
+template <int A, int B, int C, int D>
+__device__ __forceinline__ int quad_perm(int v)
+{
+    return __builtin_amdgcn_mov_dpp(v, A | (B << 2) | (C << 4) | (D << 6), 0xF, 0xF, false);
+}
+
+template <int A, int B, int C, int D>
+__device__ __forceinline__ float quad_perm(float v)
+{
+    return __int_as_float(quad_perm<A, B, C, D>(__float_as_int(v)));
+}
+
+template <int A, int B, int C, int D>
+__device__ __forceinline__ double quad_perm(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = quad_perm<A, B, C, D>((int)(unsigned)(b & 0xFFFFFFFFll));
+    const int hi = quad_perm<A, B, C, D>((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+/* value of lane K of the quad */
+template <int K, class T>
+__device__ __forceinline__ T quad_bcast(T v)
+{
+    return quad_perm<K, K, K, K>(v);
+}
+
+/* With component c of a vector in lane c (lane 3 repeats component 2): the
+ * next component (y z x) and the one before (z x y) */
+__device__ __forceinline__ double quad_next(double v) { return quad_perm<1, 2, 0, 0>(v); }
+__device__ __forceinline__ double quad_prev(double v) { return quad_perm<2, 0, 1, 1>(v); }
+
+/* ((start + x) + y) + z of the components */
+__device__ __forceinline__ double quad_sum(double start, double v)
+{
+    return ((start + quad_bcast<0>(v)) + quad_bcast<1>(v)) + quad_bcast<2>(v);
+}
+
+/* (x + y) + z */
+__device__ __forceinline__ double quad_sum(double v)
+{
+    return (quad_bcast<0>(v) + quad_bcast<1>(v)) + quad_bcast<2>(v);
+}
+
+/* component of a x b */
+__device__ __forceinline__ double quad_cross(double a, double b)
+{
+    return quad_next(a) * quad_prev(b) - quad_prev(a) * quad_next(b);
+}
+
+/* ABC field at a particle whose position's components lie in the quad's
+ * lanes: the sine and cosine of one coordinate to a lane (getb_ff as in
+ * get_emf64<FK_ABC>); k1, k2 the lane's coefficients (A B C) and (C A B) */
+__device__ __forceinline__ double quad_abc(const FieldDev &f, double k1, double k2, double x)
+{
+    double s, c;
+    tp_sincos(f.lam * x, &s, &c);
+    const double b = k1 * quad_prev(s) + k2 * quad_next(c);
+    return b * f.B0;
+}
+
+/* wirz_step64<FK_ABC> and boris_step64<FK_ABC> with component c of the
+ * position x and momentum u in lane c: the operations on vectors once to a
+ * lane instead of three times, those on scalars in every lane, each in the
+ * order of the one-lane step (same bits). */
+__device__ __forceinline__ void quad_wirz_abc(const FieldDev &f, double k1, double k2, double &x,
+                                              double &u, double &t, double dt, double qm)
+{
+    double b = quad_abc(f, k1, k2, x);
+    double Btot = sqrt(quad_sum(b * b));
+    double iB = 1.0 / Btot;
+    const double dth = dt * 0.5;
+    const double qd = qm * dth;
+    const double dm = u + qd * 0.0;
+    const double gama = sqrt(quad_sum(1.0, dm * dm));
+    const double ig = 1.0 / gama;
+    const double vm = dm * ig;
+    double h = b * iB;
+    double vd = quad_sum(0.0, vm * h);
+    double a = vm - vd * h;
+    double vp = sqrt(quad_sum(a * a));
+    double pe = (vm - vd * h) / vp;
+    double r = quad_cross(h, pe);
+    double gR = vp * gama * 1.0 * iB / qm;
+    double om = qm * Btot * ig;
+    double dthe = om * dt;
+    double sd, cd;
+    tp_sincos(dthe * 0.5, &sd, &cd);
+    double t1 = dth * vd * 1.0;
+    double t2 = gR * sd;
+    double t3 = -gR * (1.0 - cd);
+    const double xm = x + h * t1 + pe * t2 + r * t3;
+
+    b = quad_abc(f, k1, k2, xm);
+    Btot = sqrt(quad_sum(b * b));
+    iB = 1.0 / Btot;
+    h = b * iB;
+    vd = quad_sum(0.0, vm * h);
+    a = vm - vd * h;
+    vp = sqrt(quad_sum(a * a));
+    pe = (vm - vd * h) / vp;
+    r = quad_cross(h, pe);
+    om = qm * Btot * ig;
+    dthe = om * dt;
+    tp_sincos(dthe, &sd, &cd);
+    const double w = h * vd + vp * (cd * pe - sd * r);
+    const double bm = quad_sum(0.0, w * w);
+    const double g2 = 1.0 / sqrt(1.0 - bm);
+    u = g2 * w + qd * 0.0;
+    vd = quad_sum(0.0, w * h);
+    a = w - vd * h;
+    vp = sqrt(quad_sum(a * a));
+    gR = vp * gama * 1.0 * iB / qm;
+    t1 = dt * vd * 1.0;
+    t2 = gR * sd;
+    t3 = -gR * (1.0 - cd);
+    x += h * t1 + pe * t2 + r * t3;
+    t += dt;
+}
+
+__device__ __forceinline__ void quad_boris_abc(const FieldDev &f, double k1, double k2, double &x,
+                                               double &u, double &t, double dt, double qm)
+{
+    const double b = quad_abc(f, k1, k2, x);
+    const double h = qm * (0.5 * dt);
+    const double um = u + h * 0.0;
+    const double gm = sqrt(quad_sum(1.0, um * um));
+    const double fq = h / gm;
+    const double tv = fq * b;
+    const double t2 = quad_sum(tv * tv);
+    const double sf = 2.0 / (1.0 + t2);
+    const double sv = sf * tv;
+    const double up = um + quad_cross(um, tv);
+    const double uq = um + quad_cross(up, sv);
+    u = uq + h * 0.0;
+    const double g = sqrt(quad_sum(1.0, u * u));
+    const double ig = dt / g;
+    x += u * ig;
+    t += dt;
+}
+
 #endif /* TP_DEVICE_H */

@@ -492,28 +492,6 @@ __global__ void __launch_bounds__(256) k_pmap(PmapArgs a, int nact, const int *a
  * line's lanes take every branch together (their inputs are equal), so a
  * quad is always whole when it exchanges values. */
 
-/* value of lane K of the quad (quad_perm [K, K, K, K]) */
-template <int K>
-__device__ __forceinline__ int quad_bcast(int v)
-{
-    return __builtin_amdgcn_mov_dpp(v, K | (K << 2) | (K << 4) | (K << 6), 0xF, 0xF, false);
-}
-
-template <int K>
-__device__ __forceinline__ double quad_bcast(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = quad_bcast<K>((int)(unsigned)(b & 0xFFFFFFFFll));
-    const int hi = quad_bcast<K>((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-
-template <int K>
-__device__ __forceinline__ float quad_bcast(float v)
-{
-    return __int_as_float(quad_bcast<K>(__float_as_int(v)));
-}
-
 /* value of lane k (0..2, the same in every lane) of the quad */
 __device__ __forceinline__ double quad_pick(double v, int k)
 {

@@ -325,6 +325,122 @@ __global__ void __launch_bounds__(256) k_track(TrackArgs a)
     track_body<PUSH, FK, PREC, TRAJ>(a);
 }
 
+/* The step kernel with a quad of lanes to a particle (ABC field, FP64), for
+ * ensembles too small to fill the chip: component c of the position and
+ * momentum in lane c, so a wavefront carries 16 particles through about 0.45
+ * of the one-lane step's instructions and four times as many wavefronts run.
+ * The same bits as track_body; D partial sums over 16 particles a wavefront.
+ * Bound: the step's chain of FP64 operations on a wavefront alone on its SIMD
+ * (one instruction per 5 cycles).  us per 100 steps, one lane / a quad: Wirz
+ * 1000 particles 256 / 168, 16,384 particles 257 / 199; Boris 120 / 72 and
+ * 121 / 79. */
+template <int PUSH>
+__global__ void __launch_bounds__(256) k_track_quad(TrackArgs a)
+{
+    extern __shared__ unsigned hist[];
+    const int tid = threadIdx.x, sub = tid & 3, c = sub < 3 ? sub : 2;
+    const int gi = (int)(((unsigned)blockIdx.x * blockDim.x + tid) >> 2);
+    const bool live = gi < a.n;
+    const int i = live ? (a.idx ? a.idx[gi] : gi) : 0;
+    for (int b = tid; b < a.nbins; b += blockDim.x) hist[b] = 0u;
+
+    const double lo = c == 0 ? a.lo[0] : (c == 1 ? a.lo[1] : a.lo[2]);
+    const double hi = c == 0 ? a.hi[0] : (c == 1 ? a.hi[1] : a.hi[2]);
+    const double k1 = c == 0 ? a.f.A : (c == 1 ? a.f.B : a.f.C);
+    const double k2 = c == 0 ? a.f.C : (c == 1 ? a.f.A : a.f.B);
+    double *px = c == 0 ? a.x : (c == 1 ? a.y : a.z);
+    double *pu = c == 0 ? a.ux : (c == 1 ? a.uy : a.uz);
+    double *ps = c == 0 ? a.xs : (c == 1 ? a.ys : a.zs);
+    double x = 0.0, u = 0.0, t = 0.0, sh = 0.0;
+    int esc = 1, nst = 0;
+    /* particle_bc on the quad; whether the particle left an open box */
+    auto bc = [&](int e) {
+        if (a.bc == 0) {
+            const double d = hi - lo;
+            if (x > hi) { x -= d; sh += d; }
+            if (x < lo) { x += d; sh -= d; }
+        } else if (a.bc == 1) {
+            const int out = x > hi || x < lo ? 1 : 0;
+            if (quad_bcast<0>(out) | quad_bcast<1>(out) | quad_bcast<2>(out)) e = 1;
+        } else {
+            e = 0;
+        }
+        return e;
+    };
+    if (live) {
+        x = px[i]; u = pu[i]; sh = ps[i]; t = a.t[i];
+        esc = a.esc[i];
+        nst = a.nsteps[i];
+        if (a.first) {
+            /* initial wrap and escape check, src/tracking.c:314-332 */
+            nst = 1;
+            esc = bc(0);
+            if (esc && 1 < a.nd && sub == 0) atomicAdd(&a.rdec[1], 1);
+        }
+    }
+    __syncthreads();
+
+    int ntp = a.ntp0;
+    for (int j = a.j0; j <= a.j1; j++) {
+        int esc_after = esc;
+        if (live && (esc == 0 || a.bc == 0)) {
+            if (PUSH == TP_PUSH_WIRZ) quad_wirz_abc(a.f, k1, k2, x, u, t, a.dt, a.qm);
+            else quad_boris_abc(a.f, k1, k2, x, u, t, a.dt, a.qm);
+            esc_after = bc(esc_after);
+            nst++;
+        }
+        const bool left = live && esc == 0 && esc_after == 1 && a.bc == 1;
+        const bool frame = j % a.einterval == 0;
+        if (left || frame) {
+            const double ux = quad_bcast<0>(u), uy = quad_bcast<1>(u), uz = quad_bcast<2>(u);
+            if (ntp < a.nt_out && live && sub == 0) {
+                const int b = energy_bin(ux, uy, uz, a.nbins, a.logemin, a.logde);
+                if (left) atomicAdd(&a.espect_esc[ntp * a.nbins + b], 1u);
+                if (frame && esc_after == 0) atomicAdd(&hist[b], 1u);
+            }
+        }
+        if (frame) {
+            __syncthreads();
+            if (ntp < a.nt_out) {
+                for (int b = tid; b < a.nbins; b += blockDim.x) {
+                    const unsigned h = hist[b];
+                    if (h) {
+                        atomicAdd(&a.espect[ntp * a.nbins + b], h);
+                        hist[b] = 0u;
+                    }
+                }
+            }
+            __syncthreads();
+            ntp++;
+        }
+        esc = esc_after;
+    }
+    if (a.dstep >= 0) {
+        /* the D terms of the state after step j1, the particle's in lane 0 */
+        __shared__ double wsum[4][8];
+        KArgs *k = kargs_again();
+        double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (live) {
+            Emf e = {};
+            if (esc == 0) {
+                const double b = quad_abc(a.f, k1, k2, x);
+                e.bx = quad_bcast<0>(b); e.by = quad_bcast<1>(b); e.bz = quad_bcast<2>(b);
+            }
+            const double X[3] = {quad_bcast<0>(x), quad_bcast<1>(x), quad_bcast<2>(x)};
+            const double U[3] = {quad_bcast<0>(u), quad_bcast<1>(u), quad_bcast<2>(u)};
+            const double S[3] = {quad_bcast<0>(sh), quad_bcast<1>(sh), quad_bcast<2>(sh)};
+            if (sub == 0)
+                dterms_particle(k, i, esc, X[0], X[1], X[2], U[0], U[1], U[2], t, S[0], S[1], S[2],
+                                e, v);
+        }
+        dterms_reduce(k, v, live && sub == 0, live && sub == 0 ? esc : 0, tid, a.dstep, wsum);
+    }
+    if (live) {
+        if (sub < 3) { px[i] = x; pu[i] = u; ps[i] = sh; }
+        if (sub == 0) { a.t[i] = t; a.esc[i] = esc; a.nsteps[i] = nst; }
+    }
+}
+
 /* the same compiled for 3 waves per SIMD (168 VGPRs; the compiler's own
  * choice is 2 for the kernels launched this way) */
 template <int PUSH, int FK, int PREC, bool TRAJ>
@@ -530,6 +646,12 @@ __global__ void __launch_bounds__(256) k_eval(FieldDev f, int n, const double *p
 /* ------------------------------------------------------------------ */
 
 
+
+template <int PUSH>
+static void launch_track_quad(dim3 g, dim3 b, size_t sh, hipStream_t s, const TrackArgs &a)
+{
+    hipLaunchKernelGGL((k_track_quad<PUSH>), g, b, sh, s, a);
+}
 
 template <int PUSH, int FK, int PREC, bool TRAJ>
 static void launch_track(dim3 g, dim3 b, size_t sh, hipStream_t s, const TrackArgs &a)
@@ -1611,11 +1733,13 @@ int tp_gpu_load_particles(tp_ctx *c, int n, const tp_particle *ptl, const tp_par
 
 static int block_size_for(const tp_ctx *c, int n)
 {
-    /* 256 lanes per block unless that leaves compute units idle */
+    /* Blocks of four wavefronts, which go to the four SIMDs of a compute unit,
+     * unless that leaves compute units idle; then of one.  Blocks of two put
+     * both blocks of a compute unit on the same two SIMDs: 65,536 particles in
+     * the ABC field, one wavefront to a SIMD, 423 us per 100 Wirz steps in
+     * blocks of 128 lanes, 270 in blocks of 256. */
     int cu = c->num_cu > 0 ? c->num_cu : 256;
-    if ((n + 255) / 256 >= 2 * cu) return 256;
-    if ((n + 127) / 128 >= 2 * cu) return 128;
-    return 64;
+    return (n + 255) / 256 >= cu ? 256 : 64;
 }
 
 /* Buffers of one fixed-step run: the context's own (tp_gpu_run_fixed) or the
@@ -1701,6 +1825,18 @@ static int fill_f64(hipStream_t s, double *a, size_t n)
     return hipGetLastError() == hipSuccess ? TP_OK : TP_E_HIP;
 }
 
+/* Lanes to a particle: a quad in the ABC field in FP64 as long as that gives
+ * at most one wavefront to a SIMD (16,384 particles on 256 compute units);
+ * with two, the wavefronts of one lane each, which then fill half the SIMDs,
+ * are ahead (us per 100 Wirz steps: 16,384 particles 199 against 257, 24,000
+ * particles 293 against no more than the 256 of 32,769 particles). */
+static int run_lanes(const tp_ctx *c, const tp_track_params *p)
+{
+    const long cu = c->num_cu > 0 ? c->num_cu : 256;
+    return field_kind(c) == FK_ABC && p->precision == TP_FP64 && c->traj_nout == 0 &&
+           4l * c->s.n <= cu * 4 * 64 ? 4 : 1;
+}
+
 /* the checks of a run's parameters; the step kernel that runs it */
 static int run_check(const tp_ctx *c, const tp_track_params *p, track_fn *fn, bool *mlp)
 {
@@ -1721,12 +1857,16 @@ static int run_check(const tp_ctx *c, const tp_track_params *p, track_fn *fn, bo
         c->f.nmodes >= MODES_WAVE32_MIN)
         fk = FK_MODES_WAVE;
     *fn = pick_track(fk, p->pusher, p->precision, c->traj_nout > 0);
+    if (run_lanes(c, p) == 4)
+        *fn = p->pusher == TP_PUSH_WIRZ ? launch_track_quad<TP_PUSH_WIRZ>
+                                        : launch_track_quad<TP_PUSH_BORIS>;
     return *fn ? TP_OK : TP_E_ARG;
 }
 
 /* the sizes a run over n particles needs */
 struct RunSizes {
     int nd, bs, nblocks, nb256;
+    int lanes;              /* of the step kernel, to a particle */
     size_t prows, live_ints;
     long nlaunch;
 };
@@ -1736,8 +1876,9 @@ static RunSizes run_sizes(const tp_ctx *c, const tp_track_params *p, int n)
     RunSizes r;
     const int di = p->dcoeff_interval;
     r.nd = p->estep / di + 1;
-    r.bs = block_size_for(c, n);
-    r.nblocks = n > 0 ? (n + r.bs - 1) / r.bs : 0;
+    r.lanes = run_lanes(c, p);
+    r.bs = block_size_for(c, n * r.lanes);
+    r.nblocks = n > 0 ? (n * r.lanes + r.bs - 1) / r.bs : 0;
     r.nb256 = (n + 255) / 256;
     /* partial-sum rows: the step kernel's blocks, or with open boundaries a
      * launch over the particles inside plus k_dstale's blocks of 256 */
@@ -1835,7 +1976,7 @@ static int run_fixed_impl(tp_ctx *c, const tp_track_params *p, track_fn fn, bool
         row_blocks = nblocks;
         if (B.per_launch_events) HIPCHK(hipEventRecord(c->evs[2 * launches], c->stream));
         if (use_list) {
-            const int nbl = (nlive + bs - 1) / bs, nesc = n - nlive;
+            const int nbl = (nlive * R.lanes + bs - 1) / bs, nesc = n - nlive;
             if (nlive > 0) {
                 TrackArgs b = a;
                 b.idx = l_in;

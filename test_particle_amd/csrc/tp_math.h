@@ -67,6 +67,30 @@ TP_HD double tp_flip_by_low_bit(double v, double t)
 #endif
 }
 
+TP_HD uint32_t tp_low_word(double t)
+{
+    uint64_t b;
+    memcpy(&b, &t, sizeof(b));
+    return (uint32_t)b;
+}
+
+/* v with the bits of mask flipped in its high word */
+TP_HD double tp_flip_sign(double v, uint32_t mask)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 b = __builtin_bit_cast(u32x2, v);
+    b.y ^= mask;
+    return __builtin_bit_cast(double, b);
+#else
+    uint64_t b;
+    memcpy(&b, &v, sizeof(b));
+    b ^= (uint64_t)mask << 32;
+    memcpy(&v, &b, sizeof(v));
+    return v;
+#endif
+}
+
 #define TP_2_OVER_PI 0x1.45f306dc9c883p-1
 #define TP_PIO2_1    0x1.921fb54442d18p+0
 #define TP_PIO2_2    0x1.1a62633145c07p-54
@@ -75,7 +99,20 @@ TP_HD double tp_flip_by_low_bit(double v, double t)
 /* sin(x) and cos(x) together; NaN/Inf in give NaN out. */
 TP_HD void tp_sincos(double x, double *sp, double *cp)
 {
-    double k = rint(x * TP_2_OVER_PI);
+    /* k = rint(2x/pi); the quadrant k mod 4 is in the low bits of the sum that
+     * rounds it (adding 1.5 2^52), or, where that sum has no room for k, comes
+     * from k itself */
+    double k;
+    uint32_t q;
+    if (fabs(x) < 0x1p50) {
+        const double t = fma(x, TP_2_OVER_PI, 0x1.8p52);
+        k = t - 0x1.8p52;
+        q = tp_low_word(t);
+    } else {
+        k = rint(x * TP_2_OVER_PI);
+        const double m = k - 4.0 * floor(k * 0.25);
+        q = m == 1.0 ? 1u : (m == 2.0 ? 2u : (m == 3.0 ? 3u : 0u));
+    }
     double r1 = fma(-k, TP_PIO2_1, x);          /* exact */
     double w = k * TP_PIO2_2;
     double werr = fma(k, TP_PIO2_2, -w);        /* k*P2 = w + werr exactly */
@@ -111,19 +148,10 @@ TP_HD void tp_sincos(double x, double *sp, double *cp)
     double wc = 1.0 - hz;
     double c = wc + (((1.0 - wc) - hz) + fma(z * z, pc, -r * rlo));
 
-    /* quadrant q = k mod 4, kept in floating point (no int conversion of
-     * huge or non-finite k) */
-    double q = k - 4.0 * floor(k * 0.25);
-    double so, co;
-    if (q == 0.0) {
-        so = s; co = c;
-    } else if (q == 1.0) {
-        so = c; co = -s;
-    } else if (q == 2.0) {
-        so = -s; co = -c;
-    } else {
-        so = -c; co = s;
-    }
+    /* (s, c), (c, -s), (-s, -c), (-c, s) in quadrants 0 to 3: a swap and two
+     * sign bits */
+    const double so = tp_flip_sign(q & 1u ? c : s, (q & 2u) << 30);
+    const double co = tp_flip_sign(q & 1u ? s : c, ((q + 1u) & 2u) << 30);
     *sp = so;
     *cp = co;
 }

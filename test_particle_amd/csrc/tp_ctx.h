@@ -83,6 +83,10 @@ struct tp_ctx {
     float *stage_dev[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     size_t stage_floats = 0;
+    /* particles on their way to pageable host memory: pinned slots and an
+     * event for each (freed by tp_gpu_finalize) */
+    char *down_pin = nullptr;
+    hipEvent_t down_ev[8] = {};
     /* device address of the static scratch array on this context's GPU
      * (tp_gpu_run_fixed_noalloc); null if the lookup failed */
     double *scratch = nullptr;

@@ -313,19 +313,27 @@ class Tracker:
     def track_fixed(self, params, ptl, ptl_init=None):
         """The reference's fixed-step loop (src/tracking.c:90-190) on the
         GPU; returns the same raw arrays as the oracle."""
-        ptl = abi.as_particles(ptl).copy()
-        ptl_init = ptl.copy() if ptl_init is None else abi.as_particles(ptl_init)
-        n = ptl.shape[0]
+        start = abi.as_particles(ptl)
+        ptl_init = start if ptl_init is None else abi.as_particles(ptl_init)
+        n = start.shape[0]
         nd = abi.n_dcoeff_rows(params)
+        ptl = np.empty_like(start)
         nsteps = np.zeros(n, dtype=np.int32)
         esp = np.zeros((params.nt_out, params.nbins))
         ese = np.zeros((params.nt_out, params.nbins))
         dco = np.zeros((8, nd))
         rem = np.zeros(nd, dtype=np.int32)
-        _check(lib().tp_gpu_track_fixed(self._ctx, ctypes.byref(params), n, dptr(ptl),
-                                        dptr(ptl_init), iptr(nsteps), dptr(esp), dptr(ese),
-                                        dptr(dco), iptr(rem)), "track_fixed")
+        L = lib()
+        # tp_gpu_track_fixed in its four parts: the input needs no copy
+        rc = L.tp_gpu_load_particles(self._ctx, n, dptr(start), dptr(ptl_init))
+        _check(rc, "track_fixed")
         self._n = n
+        rc = L.tp_gpu_run_fixed(self._ctx, ctypes.byref(params))
+        _check(rc, "track_fixed")
+        rc = L.tp_gpu_store_particles(self._ctx, dptr(ptl), iptr(nsteps))
+        _check(rc, "track_fixed")
+        rc = L.tp_gpu_read_diagnostics(self._ctx, dptr(esp), dptr(ese), dptr(dco), iptr(rem))
+        _check(rc, "track_fixed")
         return dict(ptl=ptl, nsteps=nsteps, espect=esp, espect_escape=ese, dcoeff=dco,
                     remain=rem)
 

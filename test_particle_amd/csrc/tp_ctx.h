@@ -86,6 +86,7 @@ struct tp_ctx {
     /* particles on their way to pageable host memory: pinned slots and an
      * event for each (freed by tp_gpu_finalize) */
     char *down_pin = nullptr;
+    size_t down_slot = 0;
     hipEvent_t down_ev[8] = {};
     /* device address of the static scratch array on this context's GPU
      * (tp_gpu_run_fixed_noalloc); null if the lookup failed */

@@ -1845,6 +1845,11 @@ static int run_lanes(const tp_ctx *c, const tp_track_params *p)
            4l * c->s.n <= cu * 4 * 64 ? 4 : 1;
 }
 
+/* Spectrum bins (4 bytes of a block's LDS each) beside which the wavefront
+ * mode sum's 4 KiB have room in 64 KiB, with those of the D sums; larger
+ * histograms fit the one-lane sum's kernel only. */
+enum { WAVE_BINS_MAX = 14336 };
+
 /* the checks of a run's parameters; the step kernel that runs it */
 static int run_check(const tp_ctx *c, const tp_track_params *p, track_fn *fn, bool *mlp)
 {
@@ -1862,7 +1867,7 @@ static int run_check(const tp_ctx *c, const tp_track_params *p, track_fn *fn, bo
     /* surrogate field: the exact-field kernel runs the particles that fell back */
     int fk = *mlp ? FK_MODES : field_kind(c);
     if (fk == FK_MODES && p->precision == TP_FP32_MIXED && p->pusher == TP_PUSH_BORIS &&
-        c->f.nmodes >= MODES_WAVE32_MIN)
+        c->f.nmodes >= MODES_WAVE32_MIN && p->nbins <= WAVE_BINS_MAX)
         fk = FK_MODES_WAVE;
     *fn = pick_track(fk, p->pusher, p->precision, c->traj_nout > 0);
     if (run_lanes(c, p) == 4)
@@ -2244,32 +2249,40 @@ namespace {
  * by several threads).  hipMemcpyAsync into such memory pins it page by page
  * from one thread.  Ms into fresh pages, direct / this way: 262,141 particles
  * (23 MB) 2.6 / 1.3, 1,048,576 (92 MB) 9.4 / 3.7; 100,000 (8.8 MB) 1.2 / 0.6,
- * below which the threads have few chunks each.  The slots are the context's,
- * 8 MiB; memory that HIP knows (pinned, managed, of a device) goes the direct
- * way. */
+ * below which the threads have few chunks each.  Chunks of half a MiB take
+ * 4.9 ms for the 92 MB; small arrays have them for the first call's sake,
+ * which pins the slots (the context's, 4 or 8 MiB: about 0.1 ms a MiB).
+ * Memory that HIP knows (pinned, managed, of a device) goes the direct way. */
 enum { TP_DOWN_THREADS = 4 };
-const size_t DOWN_CHUNK = (size_t)1 << 20, DOWN_MIN = (size_t)8 << 20;
+const size_t DOWN_MIN = (size_t)8 << 20;
+
+size_t down_chunk(size_t bytes)
+{
+    return (size_t)1 << (bytes < 2 * DOWN_MIN ? 19 : 20);
+}
 
 void down_release(tp_ctx *c)
 {
     if (c->down_pin) (void)hipHostFree(c->down_pin);
     c->down_pin = nullptr;
+    c->down_slot = 0;
     for (hipEvent_t &e : c->down_ev) {
         if (e) (void)hipEventDestroy(e);
         e = nullptr;
     }
 }
 
-bool down_get(tp_ctx *c)
+bool down_get(tp_ctx *c, size_t chunk)
 {
-    if (c->down_pin) return true;
+    if (c->down_slot >= chunk) return true;
+    down_release(c);
     bool ok = true;
     for (hipEvent_t &e : c->down_ev)
         if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
             e = nullptr;
             ok = false;
         }
-    if (ok && hipHostMalloc((void **)&c->down_pin, DOWN_CHUNK * 2 * TP_DOWN_THREADS,
+    if (ok && hipHostMalloc((void **)&c->down_pin, chunk * 2 * TP_DOWN_THREADS,
                             hipHostMallocDefault) != hipSuccess) {
         c->down_pin = nullptr;
         ok = false;
@@ -2277,15 +2290,17 @@ bool down_get(tp_ctx *c)
     if (!ok) {
         down_release(c);
         (void)hipGetLastError();
+        return false;
     }
-    return ok;
+    c->down_slot = chunk;
+    return true;
 }
 
 struct Download {
     tp_ctx *c;
     char *dst;
     const char *src;
-    size_t bytes;
+    size_t bytes, chunk;
     std::atomic<size_t> next{0};
     std::atomic<int> err{0};
 
@@ -2298,13 +2313,13 @@ struct Download {
         }
         size_t off[2] = {0, 0}, len[2] = {0, 0};
         for (int b = 0;; b ^= 1) {
-            const size_t o = next.fetch_add(DOWN_CHUNK);
-            char *slot = c->down_pin + (size_t)(2 * t + b) * DOWN_CHUNK;
+            const size_t o = next.fetch_add(chunk);
+            char *slot = c->down_pin + (size_t)(2 * t + b) * chunk;
             hipEvent_t ev = c->down_ev[2 * t + b];
             off[b] = o;
             len[b] = 0;
             if (o < bytes && !err) {
-                const size_t l = bytes - o < DOWN_CHUNK ? bytes - o : DOWN_CHUNK;
+                const size_t l = bytes - o < chunk ? bytes - o : chunk;
                 if (hipMemcpyAsync(slot, src + o, l, hipMemcpyDeviceToHost, c->stream) !=
                         hipSuccess ||
                     hipEventRecord(ev, c->stream) != hipSuccess)
@@ -2315,7 +2330,7 @@ struct Download {
             const int q = b ^ 1;
             if (len[q]) {
                 if (hipEventSynchronize(c->down_ev[2 * t + q]) != hipSuccess) err = 1;
-                else memcpy(dst + off[q], c->down_pin + (size_t)(2 * t + q) * DOWN_CHUNK, len[q]);
+                else memcpy(dst + off[q], c->down_pin + (size_t)(2 * t + q) * chunk, len[q]);
                 len[q] = 0;
             }
             if (!len[b]) return;
@@ -2333,7 +2348,7 @@ int download(tp_ctx *c, void *dst, const void *src, size_t bytes)
         if (e != hipSuccess) (void)hipGetLastError();
         else if (at.type != hipMemoryTypeUnregistered) direct = true;
     }
-    if (direct || !down_get(c)) {
+    if (direct || !down_get(c, down_chunk(bytes))) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
         return TP_OK;
     }
@@ -2342,6 +2357,7 @@ int download(tp_ctx *c, void *dst, const void *src, size_t bytes)
     d.dst = (char *)dst;
     d.src = (const char *)src;
     d.bytes = bytes;
+    d.chunk = down_chunk(bytes);
     std::thread th[TP_DOWN_THREADS - 1];
     int started = 0;
     try {

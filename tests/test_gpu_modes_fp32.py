@@ -64,3 +64,20 @@ def test_open_boundary_and_short_wavefronts(gpu):
     q = gpu.track_fixed(prm, p[perm])
     assert np.array_equal(q["ptl"], r["ptl"][perm])
     assert np.array_equal(q["nsteps"], r["nsteps"][perm])
+
+
+@pytest.mark.parametrize("bins", [14336, 14337, 16000])
+def test_large_histograms(gpu, bins):
+    """Histograms that leave no LDS for the wavefront sum take the other kernel:
+    the same field to FP32 rounding, every particle counted."""
+    rows = mode_table(96, kmin=0.1, kmax=10.0, rms=0.5, seed=76)
+    p = init_particles(65, (0, 0, 0), (4, 4, 4), 0.6, seed=77)
+    kw = dict(dt=0.1, estep=10, lo=(0, 0, 0), hi=(4, 4, 4), pusher=abi.TP_PUSH_BORIS,
+              precision=abi.TP_FP32_MIXED, bc_flag=abi.TP_BC_NONE, nt_out=1, einterval_t=10,
+              emin=1e-4, emax=10.0)
+    gpu.set_field_modes(rows, 1.0)
+    a = gpu.track_fixed(abi.make_params(nbins=40, **kw), p)
+    b = gpu.track_fixed(abi.make_params(nbins=bins, **kw), p)
+    assert a["espect"].sum() == b["espect"].sum()
+    # ten steps of rounding in field and momentum (see above)
+    assert np.abs(a["ptl"] - b["ptl"]).max() < 3e-5

@@ -1,5 +1,6 @@
 """Particles to the GPU and back, whole bytes: around the size from which host
-threads copy them out in chunks of 1 MiB (8 MiB, 95,325.09 particles), with
+threads copy them out in chunks (8 MiB, 95,325.09 particles) and from which the
+chunks are larger (16 MiB, 190,650.2), with
 ragged last chunks, into pageable and pinned memory, and from several threads."""
 import ctypes
 import threading
@@ -25,7 +26,7 @@ def particles(n, seed):
     return np.random.default_rng(seed).standard_normal((n, 11))
 
 
-@pytest.mark.parametrize("n", [1, 95325, 95326, 107240, 200003, 700001])
+@pytest.mark.parametrize("n", [1, 95325, 95326, 107240, 190650, 190651, 700001])
 @pytest.mark.parametrize("pinned", [False, True])
 def test_round_trip(gpu, n, pinned):
     from hipmem import hip

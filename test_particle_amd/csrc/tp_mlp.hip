@@ -94,7 +94,7 @@ __host__ __device__ inline int frag_bwd(int k, int n)
 struct TrainBufs {
     __bf16 *h0, *h1, *h2;        /* layer inputs, 256 | 128 features */
     __bf16 *dz1, *dz2, *dz3;     /* 128 features */
-    long rows;
+    float *h3, *dout;            /* 128 features, sample-major; 3 */
 };
 
 #define GELU_C1 1.5957691216057308f   /* 2 sqrt(2/pi) */
@@ -351,17 +351,12 @@ __global__ void __launch_bounds__(256, 2) k_mlp_eval(MlpNet net, int n, const do
 /* ------------------------------------------------------------------ */
 /* training                                                            */
 /* ------------------------------------------------------------------ */
-/* partial sums of the small parameters, one row per block of 64 samples */
-#define S_B1 0
-#define S_B2 (S_B1 + NH)
-#define S_B3 (S_B2 + NH)
-#define S_W4 (S_B3 + NH)
-#define S_B4 (S_W4 + 3 * NH)
-#define S_TOTAL (S_B4 + 3)
-
 /* stride of the feature tile: 256 bf16 and 8 (528 bytes, the 16 rows of a
  * fragment read on distinct 4-bank groups) */
 #define TF 264
+/* and of h3 in its place: 128 floats and 4 */
+#define HF 132
+static_assert(sizeof(float) * HF <= sizeof(__bf16) * TF, "h3 fits the feature tile");
 
 /* the weight fragments of this wave's 32 outputs of a layer with KB k-blocks
  * of 32 inputs (loaded well ahead of their use: after each Adam step they come
@@ -401,8 +396,8 @@ __device__ __forceinline__ void train_layer(f32x4 (&acc)[2][4], const WFrag<KB> 
 
 /* four values of consecutive features n0 .. n0 + 3 of block sample m: to the
  * LDS tile (row-major) and the block's tile of a batch buffer */
-__device__ __forceinline__ bf16x4 train_store(const f32x4 &v, __bf16 *tile, __bf16 *buf, int m,
-                                              int n0)
+__device__ __forceinline__ void train_store(const f32x4 &v, __bf16 *tile, __bf16 *buf, int m,
+                                            int n0)
 {
     bf16x4 b;
 #pragma unroll
@@ -410,15 +405,6 @@ __device__ __forceinline__ bf16x4 train_store(const f32x4 &v, __bf16 *tile, __bf
     if (tile) *(bf16x4 *)(tile + m * TS + n0) = b;
 #pragma unroll
     for (int r = 0; r < 4; r++) buf[(n0 + r) * 64 + m] = b[r];
-    return b;
-}
-
-/* sum over the 16 lanes of a row */
-__device__ __forceinline__ float row_sum(float v)
-{
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
 }
 
 /* Forward and backward pass of 64 samples in one block of four waves: batch
@@ -427,27 +413,33 @@ __device__ __forceinline__ float row_sum(float v)
  * outputs over all 64 samples; gelu' of its outputs stays in its registers
  * from the forward to the backward pass, whose products leave the same
  * elements in the same lanes, so nothing but the operands of the weight
- * gradients goes to memory.  Writes those, the partial sums of the biases and
- * the output layer (row of S_TOTAL in small) and the loss partial.
+ * gradients goes to memory.  Writes those and the loss partial.  The sums of
+ * the network's outputs are mlp_wave's, in its order (same bits): each wave
+ * takes the output layer of 16 samples from the waves' h3 in LDS.
  * Bound: the chain of layers on one wave per SIMD (the batch of 16,384 is 256
  * blocks); a wave per 64 samples, which left three of four compute units
  * idle, and two kernels with gelu' and h3 through memory took 47 + 33 us a
- * batch, this 28. */
+ * batch, this 20. */
 __global__ void __launch_bounds__(256) k_mlp_train(MlpNet net, const float *dsx, const float *dsy,
                                                    long s0, int nvalid, float inv3n, TrainBufs tb,
-                                                   float *small, double *lossp)
+                                                   double *lossp)
 {
     __shared__ __attribute__((aligned(16))) __bf16 feat[64 * TF];
     __shared__ __attribute__((aligned(16))) __bf16 ta[TILE], tc[TILE];
-    __shared__ float red[4][64][3], dl[64][3];
+    __shared__ __attribute__((aligned(16))) float w4[3 * NH];
+    __shared__ float er[64][3], dl[64][3];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
     const long row = (long)blockIdx.x * 64 + lane;
-    const bool valid = row < nvalid;
     float px = 0.f, py = 0.f, pz = 0.f;
-    if (valid) {
+    if (row < nvalid) {
         const long sa = s0 + row;
         px = dsx[3 * sa]; py = dsx[3 * sa + 1]; pz = dsx[3 * sa + 2];
     }
+    /* output layer: component g of sample 16 w + i16 in this lane (g < 3) */
+    const int om = 16 * w + i16, oc = g < 3 ? g : 2;
+    const long orow = (long)blockIdx.x * 64 + om;
+    const float yo = orow < nvalid ? dsy[3 * (s0 + orow) + oc] : 0.f, b4 = net.b4[oc];
+    for (int k = threadIdx.x; k < 3 * NH; k += 256) w4[k] = net.w4[k];
     WFrag<8> f1;
     WFrag<4> f2, f3;
     f1.load(net.w1f);
@@ -526,113 +518,85 @@ __global__ void __launch_bounds__(256) k_mlp_train(MlpNet net, const float *dsx,
     f3.load(net.w2b);
     act(g3);
 
-    /* output layer in FP32: this wave's share of h3 W4, then the four waves' */
-    float wo[2][12];
+    /* h3 to the other waves (in the feature tile's place) and to memory */
+    float *hl = (float *)feat;
 #pragma unroll
-    for (int nb = 0; nb < 2; nb++) {
-        const f32x4 *wp = (const f32x4 *)(net.w4 + 3 * (nw + 16 * nb));
+    for (int nb = 0; nb < 2; nb++)
 #pragma unroll
-        for (int k = 0; k < 12; k++) wo[nb][k] = wp[k / 4][k % 4];
-    }
+        for (int mb = 0; mb < 4; mb++) {
+            const int m = mb * 16 + i16, n0 = nw + 16 * nb;
+            *(f32x4 *)(hl + m * HF + n0) = acc[nb][mb];
+            *(f32x4 *)(tb.h3 + at + m * NH + n0) = acc[nb][mb];
+        }
+    __syncthreads();
+
+    /* output layer in FP32, this wave's 16 samples: partial sums over the
+     * lane's 32 hidden units, completed across the 4 lane groups */
+    {
+        float o[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-    for (int mb = 0; mb < 4; mb++)
+        for (int nb = 0; nb < 8; nb++) {
+            const f32x4 h = *(const f32x4 *)(hl + om * HF + nb * 16 + 4 * g);
+            const f32x4 *wp = (const f32x4 *)(w4 + 3 * (nb * 16 + 4 * g));
+            const f32x4 wv[3] = {wp[0], wp[1], wp[2]};
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int c = 0; c < 3; c++)
+                    o[c] = fmaf(h[r], wv[(3 * r + c) / 4][(3 * r + c) % 4], o[c]);
+        }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            float o = 0.f;
-#pragma unroll
-            for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) o = fmaf(acc[nb][mb][r], wo[nb][3 * r + c], o);
-            o += __shfl_xor(o, 16, 64);
-            o += __shfl_xor(o, 32, 64);
-            if (g == 0) red[w][mb * 16 + i16][c] = o;
+            o[c] += __shfl_xor(o[c], 16, 64);
+            o[c] += __shfl_xor(o[c], 32, 64);
         }
+        if (g < 3) {
+            const float v = (g == 0 ? o[0] : g == 1 ? o[1] : o[2]) + b4;
+            const float e = orow < nvalid ? v - yo : 0.f;
+            const float d = 2.0f * e * inv3n;
+            er[om][g] = e;
+            dl[om][g] = d;
+            tb.dout[((size_t)blockIdx.x * 3 + g) * 64 + om] = d;
+        }
+    }
     __syncthreads();
     if (w == 0) {
         double e2 = 0.0;
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            float d = 0.f;
-            if (valid) {
-                const float o = ((red[0][lane][c] + red[1][lane][c]) +
-                                 (red[2][lane][c] + red[3][lane][c])) + net.b4[c];
-                const float e = o - dsy[3 * (s0 + row) + c];
-                e2 += (double)e * (double)e;
-                d = 2.0f * e * inv3n;
-            }
-            dl[lane][c] = d;
-        }
+        for (int c = 0; c < 3; c++) e2 += (double)er[lane][c] * (double)er[lane][c];
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) e2 += __shfl_xor(e2, off, 64);
         if (lane == 0) lossp[blockIdx.x] = e2;
     }
-    __syncthreads();
-    float *sp = small + (size_t)blockIdx.x * S_TOTAL;
-    if (threadIdx.x < 3) {
-        float b = 0.f;
-        for (int m = 0; m < 64; m++) b += dl[m][threadIdx.x];
-        sp[S_B4 + threadIdx.x] = b;
-    }
 
-    /* dZ3 = (dL/dout W4^T) gelu'(z3), and the output layer's gradient */
-    f32x4 bs[2];                        /* bias gradients of the lane's samples */
-    auto bias_out = [&](float *o) {
+    /* dZ3 = (dL/dout W4^T) gelu'(z3) */
 #pragma unroll
-        for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float v = row_sum(bs[nb][r]);
-                if (i16 == 0) o[nw + 16 * nb + r] = v;
-            }
-    };
-    {
-        float w4g[2][12];
-#pragma unroll
-        for (int nb = 0; nb < 2; nb++) {
-            bs[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < 12; k++) w4g[nb][k] = 0.f;
-        }
+    for (int nb = 0; nb < 2; nb++) {
+        const f32x4 *wp = (const f32x4 *)(w4 + 3 * (nw + 16 * nb));
+        const f32x4 wv[3] = {wp[0], wp[1], wp[2]};
 #pragma unroll
         for (int mb = 0; mb < 4; mb++) {
             const int m = mb * 16 + i16;
             const float d0 = dl[m][0], d1 = dl[m][1], d2 = dl[m][2];
+            f32x4 dz;
 #pragma unroll
-            for (int nb = 0; nb < 2; nb++) {
-                f32x4 dz;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float h = acc[nb][mb][r];
-                    w4g[nb][3 * r] = fmaf(h, d0, w4g[nb][3 * r]);
-                    w4g[nb][3 * r + 1] = fmaf(h, d1, w4g[nb][3 * r + 1]);
-                    w4g[nb][3 * r + 2] = fmaf(h, d2, w4g[nb][3 * r + 2]);
-                    const float dh = fmaf(d2, wo[nb][3 * r + 2],
-                                          fmaf(d1, wo[nb][3 * r + 1], d0 * wo[nb][3 * r]));
-                    dz[r] = dh * g3[nb][mb][r];
-                }
-                const bf16x4 b = train_store(dz, ta, tb.dz3 + at, m, nw + 16 * nb);
-#pragma unroll
-                for (int r = 0; r < 4; r++) bs[nb][r] += (float)b[r];
+            for (int r = 0; r < 4; r++) {
+                const int k = 3 * r;
+                const float dh = fmaf(d2, wv[(k + 2) / 4][(k + 2) % 4],
+                                      fmaf(d1, wv[(k + 1) / 4][(k + 1) % 4],
+                                           d0 * wv[k / 4][k % 4]));
+                dz[r] = dh * g3[nb][mb][r];
             }
+            train_store(dz, ta, tb.dz3 + at, m, nw + 16 * nb);
         }
-#pragma unroll
-        for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int k = 0; k < 12; k++) {
-                const float v = row_sum(w4g[nb][k]);
-                if (i16 == 0) sp[S_W4 + 3 * (nw + 16 * nb) + k] = v;
-            }
-        bias_out(sp + S_B3);
     }
     /* dZ2 = (dZ3 W3^T) gelu'(z2), dZ1 = (dZ2 W2^T) gelu'(z1) */
     auto back = [&](const WFrag<4> &wb, const __bf16 *from, const f32x4 (&gd)[2][4], __bf16 *tile,
                     __bf16 *buf) {
 #pragma unroll
-        for (int nb = 0; nb < 2; nb++) {
-            bs[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int nb = 0; nb < 2; nb++)
 #pragma unroll
             for (int mb = 0; mb < 4; mb++) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
         __syncthreads();
         train_layer<4, TS>(acc, wb, from);
 #pragma unroll
@@ -642,45 +606,130 @@ __global__ void __launch_bounds__(256) k_mlp_train(MlpNet net, const float *dsx,
                 f32x4 v;
 #pragma unroll
                 for (int r = 0; r < 4; r++) v[r] = acc[nb][mb][r] * gd[nb][mb][r];
-                const bf16x4 b = train_store(v, tile, buf + at, mb * 16 + i16, nw + 16 * nb);
-#pragma unroll
-                for (int r = 0; r < 4; r++) bs[nb][r] += (float)b[r];
+                train_store(v, tile, buf + at, mb * 16 + i16, nw + 16 * nb);
             }
     };
     back(f2, ta, g2, tc, tb.dz2);
-    bias_out(sp + S_B2);
     back(f3, tc, g1, nullptr, tb.dz1);
-    bias_out(sp + S_B1);
 }
 
-/* dW = X^T D of layers 1-3 over a chunk of samples (blockIdx.x; chunk rows,
- * a multiple of 64): blockIdx.y = 64 inputs of a layer (0-3: layer 1, 4-5:
- * layer 2, 6-7: layer 3) and all 128 outputs, a wave on 32 x 64 of them.  Both
- * operands come straight from the batch buffers (16 bytes a lane, no
- * LDS).  part has one row of P_TOTAL floats per chunk.
- * Bound: latency of the operand reads (2048 MFMAs a chunk of 256, under a
- * microsecond on the chip).  With the operands transposed through LDS in
- * two-byte writes and a block per layer and 256 samples: 73 us a batch of
- * 16,384; this 15, with half the partial sums (16 inputs x 128 outputs to a
- * wave, which reads half as much again: 21). */
-__global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, int chunk, float *part)
+/* the unit of the sums over samples */
+#define CHUNK 256
+
+/* Gradients of the biases and of the output layer over a chunk, whose first
+ * tile is t0: every sum runs over the samples one after another.  y 0: W4;
+ * 1-3: b1, b2, b3 (and b4).  lt: NH x LT of LDS, for a tile of dZ that is read
+ * coalesced and summed along its rows. */
+#define LT 72
+__device__ __forceinline__ void wgrad_small(const TrainBufs &tb, int y, long t0, float *pr,
+                                            __bf16 *lt)
 {
+    const int tid = threadIdx.x, n = tid & (NH - 1), half = tid >> 7;
+    if (y == 0) {
+        /* dW4[n][c] = sum_s h3[s][n] dout[s][c] in FP32: c = 0 and 1 in one
+         * half of the block, 2 in the other */
+        float a0 = 0.f, a1 = 0.f, h[16];
+        const float *hp = tb.h3 + t0 * (64 * NH) + n;
+#pragma unroll
+        for (int m = 0; m < 16; m++) h[m] = hp[m * NH];
+#pragma unroll 1
+        for (int s = 0; s < CHUNK; s += 16) {
+            const f32x4 *dp = (const f32x4 *)(tb.dout + (t0 + s / 64) * 192 + 128 * half + s % 64);
+            const int next = s + 16 < CHUNK ? s + 16 : s;
+            float hn[16];
+#pragma unroll
+            for (int m = 0; m < 16; m++) hn[m] = hp[(next + m) * NH];
+#pragma unroll
+            for (int m = 0; m < 16; m += 4) {
+                const f32x4 u = dp[m / 4], v = dp[(half ? 0 : 16) + m / 4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    a0 = fmaf(h[m + r], u[r], a0);
+                    a1 = fmaf(h[m + r], v[r], a1);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 16; m++) h[m] = hn[m];
+        }
+        pr[P_W4 + 3 * n + 2 * half] = a0;
+        if (half == 0) pr[P_W4 + 3 * n + 1] = a1;
+        return;
+    }
+    const __bf16 *dz = y == 1 ? tb.dz1 : (y == 2 ? tb.dz2 : tb.dz3);
+    const bf16x8 *dp = (const bf16x8 *)(dz + t0 * (64 * NH)) + tid;
+    bf16x8 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = dp[256 * k];
+    float s = 0.f;
+#pragma unroll 1
+    for (int t = 0; t < CHUNK / 64; t++) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            *(bf16x8 *)(lt + ((tid >> 3) + 32 * k) * LT + (tid & 7) * 8) = v[k];
+        __syncthreads();
+        if (t + 1 < CHUNK / 64) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = dp[(t + 1) * (8 * NH) + 256 * k];
+        }
+        if (half == 0) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const bf16x8 d = *(const bf16x8 *)(lt + n * LT + 8 * q);
+#pragma unroll
+                for (int r = 0; r < 8; r++) s += (float)d[r];
+            }
+        } else if (y == 3 && n < 3) {
+            const f32x4 *op = (const f32x4 *)(tb.dout + ((t0 + t) * 3 + n) * 64);
+#pragma unroll 4
+            for (int q = 0; q < 16; q++) {
+                const f32x4 d = op[q];
+#pragma unroll
+                for (int r = 0; r < 4; r++) s += d[r];
+            }
+        }
+    }
+    if (half == 0) pr[(y == 1 ? P_B1 : (y == 2 ? P_B2 : P_B3)) + n] = s;
+    else if (y == 3 && n < 3) pr[P_B4 + n] = s;
+}
+
+/* Parameter gradients of a chunk of 256 samples (blockIdx.x; part has one row
+ * of P_TOTAL floats per chunk).  The last eight blockIdx.y: dW = X^T D of
+ * layers 1-3, 64 inputs of a layer (0-3: layer 1, 4-5: layer 2, 6-7: layer 3)
+ * and all 128 outputs, a wave on 32 x 64 of them, both operands straight from
+ * the batch buffers (16 bytes a lane, no LDS); before them, so that these
+ * chains run beside the products, wgrad_small.
+ * The chunk is 256 samples whatever the batch: it is the unit of the sums'
+ * order, which decides the gradient's last bits and, through the bfloat16
+ * weights, more of the trained network than those.
+ * Bound: latency of the operand reads (2048 MFMAs a chunk, under a microsecond
+ * on the chip) and the partial sums' 17 MB a batch of 16,384.  With the
+ * operands transposed through LDS in two-byte writes and a block per layer and
+ * 256 samples: 73 us a batch; this 21. */
+#define WGRAD_SMALL 4
+__global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, float *part)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 lt[NH * LT];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, i16 = lane & 15;
-    const int y = blockIdx.y;
+    const long t0 = (long)blockIdx.x * (CHUNK / 64);
+    float *pr = part + (size_t)blockIdx.x * P_TOTAL;
+    if (blockIdx.y < WGRAD_SMALL) {
+        wgrad_small(tb, blockIdx.y, t0, pr, lt);
+        return;
+    }
+    const int y = blockIdx.y - WGRAD_SMALL;
     const __bf16 *X = y < 4 ? tb.h0 : (y < 6 ? tb.h1 : tb.h2);
     const __bf16 *D = y < 4 ? tb.dz1 : (y < 6 ? tb.dz2 : tb.dz3);
     const int k0 = 64 * (y < 4 ? y : (y < 6 ? y - 4 : y - 6)) + 32 * (w & 1);
     const int n0 = 64 * (w >> 1);
     const int nf = y < 4 ? NIN : NH;
-    const long t0 = (long)blockIdx.x * (chunk / 64), tn = tb.rows / 64;
-    const long t1 = t0 + chunk / 64 < tn ? t0 + chunk / 64 : tn;
     const __bf16 *xp = X + (k0 + i16) * 64 + 8 * g, *dp = D + (n0 + i16) * 64 + 8 * g;
     f32x4 acc[2][4];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int nb = 0; nb < 4; nb++) acc[i][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long t = t0; t < t1; t++) {
+    for (long t = t0; t < t0 + CHUNK / 64; t++) {
         bf16x8 a[2][2], b[2][4];
 #pragma unroll
         for (int q = 0; q < 2; q++) {
@@ -698,7 +747,7 @@ __global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, int chunk, floa
 #pragma unroll
                 for (int nb = 0; nb < 4; nb++) acc[i][nb] = mfma(a[q][i], b[q][nb], acc[i][nb]);
     }
-    float *pw = part + (size_t)blockIdx.x * P_TOTAL + (y < 4 ? P_W1 : (y < 6 ? P_W2 : P_W3));
+    float *pw = pr + (y < 4 ? P_W1 : (y < 6 ? P_W2 : P_W3));
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -710,53 +759,36 @@ __global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, int chunk, floa
 
 enum { ADAM_STEP = 0, ADAM_GRAD_ONLY = 1, ADAM_FRAG_ONLY = 2 };
 
-/* parameters of layers 1-3's weights come first in the optimiser's blocks, a
- * thread each; the small ones (biases and output layer) follow, a wave each */
-#define BIG_TOTAL (NIN * NH + 2 * NH * NH)
-#define BIG_BLOCKS (BIG_TOTAL / 256)
-static_assert(BIG_TOTAL % 256 == 0, "whole blocks of weights");
+#define ADAM_BLOCKS ((P_TOTAL + 255) / 256)
 
-/* The gradient of every parameter from its partial sums in a fixed order
- * (deterministic): weights over the chunks in chunk order, small parameters
- * over the blocks of 64 samples with lane-strided sums and a lane tree; then
- * the mode's action: an Adam step (Kingma & Ba 2015, bias-corrected), the
+/* The sum of the chunk partials in chunk order (deterministic), then the
+ * mode's action: an Adam step (Kingma & Ba 2015, bias-corrected), the
  * gradient only, or nothing; finally the bf16 fragments of the weight.  With
- * lacc the last wave adds the loss partials to it (the same kind of sum). */
+ * lacc a block after the parameters' adds the loss to it: the partials of a
+ * chunk's four tiles, then the chunks, each in order. */
 __global__ void __launch_bounds__(256) k_mlp_adam(float *params, float *am, float *av,
-        const float *part, int nchunks, const float *small, int nsmall, const double *lossp,
-        double *lacc, int mode, float lr, float b1, float b2, float eps, float bc1, float bc2, float *gout, bf16x8 *frag)
+        const float *part, int nchunks, const double *lossp, double *lacc, int mode, float lr,
+        float b1, float b2, float eps, float bc1, float bc2, float *gout, bf16x8 *frag)
 {
-    int p;
+    if (blockIdx.x == ADAM_BLOCKS) {
+        if (threadIdx.x >= 64) return;
+        double s = 0.0;
+        for (int c0 = 0; c0 < nchunks; c0 += 64) {
+            const int c = c0 + threadIdx.x, cnt = nchunks - c0 < 64 ? nchunks - c0 : 64;
+            double q = 0.0;
+            if (c < nchunks)
+                q = ((lossp[4 * c] + lossp[4 * c + 1]) + lossp[4 * c + 2]) + lossp[4 * c + 3];
+            for (int k = 0; k < cnt; k++) s += __shfl(q, k, 64);
+        }
+        if (threadIdx.x == 0) *lacc += s;
+        return;
+    }
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= P_TOTAL) return;
     float gs = 0.f;
-    if (blockIdx.x < BIG_BLOCKS) {
-        const int e = blockIdx.x * 256 + threadIdx.x;
-        p = e < NIN * NH ? P_W1 + e
-                         : (e < NIN * NH + NH * NH ? P_W2 + e - NIN * NH
-                                                   : P_W3 + e - NIN * NH - NH * NH);
-        if (mode != ADAM_FRAG_ONLY) {
-#pragma unroll 8
-            for (int c = 0; c < nchunks; c++) gs += part[(size_t)c * P_TOTAL + p];
-        }
-    } else {
-        const int q = (blockIdx.x - BIG_BLOCKS) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-        if (q == S_TOTAL && lacc) {
-            double s = 0.0;
-            for (int b = lane; b < nsmall; b += 64) s += lossp[b];
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-            if (lane == 0) *lacc += s;
-        }
-        if (q >= S_TOTAL) return;
-        p = q < S_B2 ? P_B1 + q
-                     : (q < S_B3 ? P_B2 + q - S_B2
-                                 : (q < S_W4 ? P_B3 + q - S_B3
-                                             : (q < S_B4 ? P_W4 + q - S_W4 : P_B4 + q - S_B4)));
-        if (mode != ADAM_FRAG_ONLY) {
-            for (int b = lane; b < nsmall; b += 64) gs += small[(size_t)b * S_TOTAL + q];
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) gs += __shfl_xor(gs, o, 64);
-        }
-        if (lane != 0) return;
+    if (mode != ADAM_FRAG_ONLY) {
+#pragma unroll 16
+        for (int c = 0; c < nchunks; c++) gs += part[(size_t)c * P_TOTAL + p];
     }
     float w = params[p];
     if (mode != ADAM_FRAG_ONLY) {
@@ -1012,7 +1044,7 @@ struct MlpState {
     __bf16 *h0 = nullptr, *h1 = nullptr, *h2 = nullptr;
     __bf16 *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
     double *lossp = nullptr, *lacc = nullptr;
-    float *part = nullptr, *small = nullptr, *grad = nullptr;
+    float *h3 = nullptr, *dout = nullptr, *part = nullptr, *grad = nullptr;
     /* training set (or the points of a gradient call) */
     long ds_cap = 0;
     float *dsx = nullptr, *dsy = nullptr;
@@ -1024,8 +1056,8 @@ void tp_mlp_release(tp_ctx *c)
     if (!m) return;
     void *ptrs[] = {m->params, m->am, m->av, m->q, m->frag, m->fb, m->nfb, m->idx, m->cnt,
                     m->h0, m->h1,
-                    m->h2, m->dz1, m->dz2, m->dz3, m->lossp, m->lacc, m->part, m->small,
-                    m->grad, m->dsx, m->dsy};
+                    m->h2, m->dz1, m->dz2, m->dz3, m->h3, m->dout, m->lossp, m->lacc,
+                    m->part, m->grad, m->dsx, m->dsy};
     for (void *p : ptrs) (void)hipFree(p);
     delete m;
     c->mlp = nullptr;
@@ -1063,21 +1095,11 @@ static int dalloc(void **p, size_t bytes)
     return TP_OK;
 }
 
-/* Rows of a weight-gradient chunk: 256, doubled until there are at most 32
- * chunks.  32 chunks are 256 blocks, one for each compute unit, and their
- * partial sums 8.5 MB whatever the batch (64 of 256 rows for 16,384 samples
- * were 17 MB to write and read again). */
-static int chunk_rows(long rows)
-{
-    long c = 256;
-    while ((rows + c - 1) / c > 32) c *= 2;
-    return (int)c;
-}
-
 static int ensure_rows(MlpState *m, long rows)
 {
     if (rows <= m->rows_cap) return TP_OK;
-    void *old[] = {m->h0, m->h1, m->h2, m->dz1, m->dz2, m->dz3, m->lossp, m->part, m->small};
+    void *old[] = {m->h0, m->h1, m->h2, m->dz1, m->dz2, m->dz3, m->h3, m->dout, m->lossp,
+                   m->part};
     for (void *p : old) (void)hipFree(p);
     m->rows_cap = 0;
     const size_t r = (size_t)rows;
@@ -1088,10 +1110,10 @@ static int ensure_rows(MlpState *m, long rows)
     rc |= dalloc((void **)&m->dz1, r * NH * 2);
     rc |= dalloc((void **)&m->dz2, r * NH * 2);
     rc |= dalloc((void **)&m->dz3, r * NH * 2);
+    rc |= dalloc((void **)&m->h3, r * NH * 4);
+    rc |= dalloc((void **)&m->dout, r * 3 * 4);
     rc |= dalloc((void **)&m->lossp, (r / 64) * sizeof(double));
-    rc |= dalloc((void **)&m->small, (r / 64) * (size_t)S_TOTAL * 4);
-    const size_t chunks = r / 256 < 32 ? r / 256 : 32;
-    rc |= dalloc((void **)&m->part, chunks * (size_t)P_TOTAL * 4);
+    rc |= dalloc((void **)&m->part, (r / CHUNK) * (size_t)P_TOTAL * 4);
     if (rc) return TP_E_NOMEM;
     m->rows_cap = rows;
     return TP_OK;
@@ -1108,12 +1130,12 @@ static int ensure_ds(MlpState *m, long n)
     return TP_OK;
 }
 
-static TrainBufs bufs_of(const MlpState *m, long rows)
+static TrainBufs bufs_of(const MlpState *m)
 {
     TrainBufs t;
     t.h0 = m->h0; t.h1 = m->h1; t.h2 = m->h2;
     t.dz1 = m->dz1; t.dz2 = m->dz2; t.dz3 = m->dz3;
-    t.rows = rows;
+    t.h3 = m->h3; t.dout = m->dout;
     return t;
 }
 
@@ -1124,19 +1146,18 @@ static int train_pass(tp_ctx *c, long s0, int nvalid, long rows, int mode, float
 {
     MlpState *m = c->mlp;
     const MlpNet net = net_of(m);
-    const TrainBufs tb = bufs_of(m, rows);
-    const int nblk = (int)(rows / 64), chunk = chunk_rows(rows);
-    const int nchunks = (int)((rows + chunk - 1) / chunk);
+    const TrainBufs tb = bufs_of(m);
+    const int nchunks = (int)(rows / CHUNK);
     const float inv3n = (float)(1.0 / (3.0 * (double)nvalid));
-    hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(256), 0, c->stream, net, m->dsx, m->dsy, s0,
-                       nvalid, inv3n, tb, m->small, m->lossp);
+    hipLaunchKernelGGL(k_mlp_train, dim3((unsigned)(rows / 64)), dim3(256), 0, c->stream, net,
+                       m->dsx, m->dsy, s0, nvalid, inv3n, tb, m->lossp);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(nchunks, 8), dim3(256), 0, c->stream, tb, chunk, m->part);
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(nchunks, WGRAD_SMALL + 8), dim3(256), 0, c->stream, tb, m->part);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_adam, dim3(BIG_BLOCKS + S_TOTAL / 4 + 1), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_BLOCKS + (lacc ? 1 : 0)), dim3(256), 0, c->stream,
                        m->params, m->am, m->av, (const float *)m->part, nchunks,
-                       (const float *)m->small, nblk, (const double *)m->lossp, lacc, mode, lr, b1,
-                       b2, eps, bc1, bc2, gout, m->frag);
+                       (const double *)m->lossp, lacc, mode, lr, b1, b2, eps, bc1, bc2, gout,
+                       m->frag);
     HIPCHK(hipGetLastError());
     return TP_OK;
 }
@@ -1176,9 +1197,9 @@ int tp_gpu_mlp_set(tp_ctx *c, const float *q, const float *params, double scale)
     HIPCHK(hipMemset(m->av, 0, P_TOTAL * 4));
     HIPCHK(hipMemset(m->frag, 0, FR_TOTAL * sizeof(bf16x8)));
     m->scale = (float)scale;
-    hipLaunchKernelGGL(k_mlp_adam, dim3(BIG_BLOCKS), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_BLOCKS), dim3(256), 0, c->stream,
                        m->params, m->am, m->av, (const float *)nullptr, 0,
-                       (const float *)nullptr, 0, (const double *)nullptr, (double *)nullptr,
+                       (const double *)nullptr, (double *)nullptr,
                        (int)ADAM_FRAG_ONLY, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f, (float *)nullptr,
                        m->frag);
     HIPCHK(hipGetLastError());

@@ -1,6 +1,6 @@
 """Loss and gradient of the surrogate at the edges of the training kernels'
-tiles (64 samples), rows (256) and weight-gradient chunks (256 rows up to
-8,192, then 512 and more), against the oracle with the GPU's rounding points;
+tiles (64 samples) and of rows and gradient chunks (256), against the oracle
+with the GPU's rounding points;
 the sum over samples must not depend on how they are cut."""
 import numpy as np
 import pytest

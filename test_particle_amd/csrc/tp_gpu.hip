@@ -1600,6 +1600,33 @@ static int modes_parts(tp_ctx *c, int nmodes, const double *rows)
     return rc;
 }
 
+/* The table of modes_wave64, 32 doubles per four modes.  An empty mode table
+ * (a uniform guide field) has its zero groups all the same: the kernels copy
+ * and read ahead of them before they look at the number of groups. */
+static int modes_quads(tp_ctx *c, int nmodes, const double *rows)
+{
+    const int nquads = (nmodes + 15) / 16 * 4;
+    const size_t nx = (size_t)32 * (nquads + MODES_PAD_QUADS);
+    double *tx = (double *)calloc(nx, sizeof(double));
+    if (!tx) return TP_E_NOMEM;
+    for (int m = 0; m < nmodes; m++) {
+        const double *r = rows + 7 * m;
+        double *o = tx + 32 * (size_t)(m / 4) + 4 * (m % 4);
+        o[0] = r[6]; o[1] = r[0]; o[2] = r[1]; o[3] = r[2];
+        o[16] = r[3]; o[17] = r[4]; o[18] = r[5];
+    }
+    if (hipMalloc(&c->modesx, nx * sizeof(double)) != hipSuccess) {
+        c->modesx = nullptr;
+        free(tx);
+        return TP_E_NOMEM;
+    }
+    const hipError_t e = hipMemcpy(c->modesx, tx, nx * sizeof(double), hipMemcpyHostToDevice);
+    free(tx);
+    HIPCHK(e);
+    c->f.nquads = nquads;
+    return TP_OK;
+}
+
 int tp_gpu_set_field_modes(tp_ctx *c, int nmodes, const double *rows, double b0z)
 {
     if (!c || nmodes < 0 || (nmodes > 0 && !rows)) return TP_E_ARG;
@@ -1630,29 +1657,11 @@ int tp_gpu_set_field_modes(tp_ctx *c, int nmodes, const double *rows, double b0z
                                  hipMemcpyHostToDevice);
         free(t32);
         HIPCHK(e);
-        /* rows for the matrix cores, 32 doubles per four modes */
-        const int nquads = (nmodes + 15) / 16 * 4;
-        const size_t nx = (size_t)32 * (nquads + MODES_PAD_QUADS);
-        double *tx = (double *)calloc(nx, sizeof(double));
-        if (!tx) return TP_E_NOMEM;
-        for (int m = 0; m < nmodes; m++) {
-            const double *r = rows + 7 * m;
-            double *o = tx + 32 * (size_t)(m / 4) + 4 * (m % 4);
-            o[0] = r[6]; o[1] = r[0]; o[2] = r[1]; o[3] = r[2];
-            o[16] = r[3]; o[17] = r[4]; o[18] = r[5];
-        }
-        if (hipMalloc(&c->modesx, nx * sizeof(double)) != hipSuccess) {
-            c->modesx = nullptr;
-            free(tx);
-            return TP_E_NOMEM;
-        }
-        e = hipMemcpy(c->modesx, tx, nx * sizeof(double), hipMemcpyHostToDevice);
-        free(tx);
-        HIPCHK(e);
-        c->f.nquads = nquads;
         int rc = modes_parts(c, nmodes, rows);
         if (rc) return rc;
     }
+    int rc = modes_quads(c, nmodes, rows);
+    if (rc) return rc;
     c->f.nmodes = nmodes;
     c->f.modes = c->modes;
     c->f.modesx = c->modesx;

@@ -72,3 +72,28 @@ def test_lanes_per_wavefront(gpu, oracle_tp, n, dense):
         ref = oracle_tp.bs_track(f, bs, p[pick])
     assert np.array_equal(r["ptl"][pick], ref["ptl"])
     assert np.array_equal(r["nsteps"][pick], ref["nsteps"])
+
+
+def test_empty_table(oracle_tp):
+    """No modes at all: the uniform guide field, through both forms and the
+    launch-shape trials."""
+    from test_particle_amd.gpu import Tracker
+    rows = np.zeros((0, 7))
+    f = oracle_tp.Field.modes(rows, 0.8)
+    p = _ptl(70)
+    with Tracker(0) as t:
+        t.set_field_modes(rows, 0.8)
+        bs = abi.make_bs_params(rtol=1e-8, atol=1e-10, t_end_gyro=0.5, b_ref=0.8)
+        r = t.track_adaptive(bs, p)
+        ref = oracle_tp.bs_track(f, bs, p)
+        assert np.array_equal(r["ptl"], ref["ptl"]) and np.array_equal(r["nsteps"], ref["nsteps"])
+        t.tune_adaptive(bs)
+        r = t.track_adaptive(bs, p)
+        assert np.array_equal(r["ptl"], ref["ptl"]) and np.array_equal(r["nsteps"], ref["nsteps"])
+        bs = abi.make_bs_params(rtol=1e-8, atol=1e-10)
+        prm = abi.make_params(dt=0.05, estep=20, lo=(0, 0, 0), hi=(10, 10, 10), nbins=52,
+                              nt_out=2, einterval_t=10, dcoeff_interval=10, emin=1e-4, emax=10.0)
+        r = t.track_adaptive_diag(bs, prm, p)
+        ref = oracle_tp.bs_track_diag(f, bs, prm, p)
+        for k in ("ptl", "nsteps", "espect"):
+            assert np.array_equal(r[k], ref[k]), k

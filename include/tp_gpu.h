@@ -401,7 +401,10 @@ int tp_gpu_tune_adaptive(tp_ctx *ctx, const tp_bs_params *p, const char *cache_p
 
 /* --- field probe -------------------------------------------------------- */
 /* get_emf (src/emfields.c:32-60) at n points pts[4*i] = (x, y, z, t);
- * out[6*i] = (Bx, By, Bz, Ex, Ey, Ez).  precision as in tp_track_params. */
+ * out[6*i] = (Bx, By, Bz, Ex, Ey, Ez).  precision as in tp_track_params: the
+ * field that a run of that precision uses in its steps (multi-mode field in
+ * FP32: with a histogram of up to 14,336 bins; beyond, the modes are summed in
+ * another order). */
 int tp_gpu_eval_field(tp_ctx *ctx, int n, const double *pts, double *out,
                       int precision);
 

@@ -629,6 +629,21 @@ __global__ void __launch_bounds__(256) k_eval(FieldDev f, int n, const double *p
                                               double *out)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if constexpr (FK == FK_MODES_WAVE) {
+        /* the FP32 mode sum of the step kernels, by the whole wavefront */
+        __shared__ __align__(16) float points[4 * MODES_WAVE32_LDS];
+        float x = 0.f, y = 0.f, z = 0.f, bx, by, bz;
+        if (i < n) {
+            x = (float)pts[4 * i]; y = (float)pts[4 * i + 1]; z = (float)pts[4 * i + 2];
+        }
+        modes_wave32(f, x, y, z, points + (threadIdx.x >> 6) * MODES_WAVE32_LDS, bx, by, bz);
+        if (i < n) {
+            double *o = out + 6 * i;
+            o[0] = bx; o[1] = by; o[2] = (float)f.b0z + bz;
+            o[3] = o[4] = o[5] = 0.0;
+        }
+        return;
+    }
     if (i >= n) return;
     double x = pts[4 * i], y = pts[4 * i + 1], z = pts[4 * i + 2], t = pts[4 * i + 3];
     double *o = out + 6 * i;
@@ -646,8 +661,6 @@ __global__ void __launch_bounds__(256) k_eval(FieldDev f, int n, const double *p
 /* ------------------------------------------------------------------ */
 /* dispatch                                                            */
 /* ------------------------------------------------------------------ */
-
-
 
 template <int PUSH>
 static void launch_track_quad(dim3 g, dim3 b, size_t sh, hipStream_t s, const TrackArgs &a)
@@ -774,6 +787,11 @@ static void launch_eval(dim3 g, dim3 b, hipStream_t s, const FieldDev &f, int n,
 static void dispatch_eval(int fk, dim3 g, dim3 b, hipStream_t s, const FieldDev &f,
                           int n, const double *pts, double *out, int prec)
 {
+    if (prec != TP_FP64 && (fk == FK_MODES || fk == FK_MLP) && f.nmodes >= MODES_WAVE32_MIN) {
+        /* the sum of the step kernels (run_check) */
+        hipLaunchKernelGGL((k_eval<FK_MODES_WAVE, PREC32>), g, b, 0, s, f, n, pts, out);
+        return;
+    }
     switch (fk) {
     case FK_TEST: launch_eval<FK_TEST>(g, b, s, f, n, pts, out, prec); break;
     case FK_ABC: launch_eval<FK_ABC>(g, b, s, f, n, pts, out, prec); break;

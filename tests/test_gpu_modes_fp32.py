@@ -81,3 +81,31 @@ def test_large_histograms(gpu, bins):
     assert a["espect"].sum() == b["espect"].sum()
     # ten steps of rounding in field and momentum (see above)
     assert np.abs(a["ptl"] - b["ptl"]).max() < 3e-5
+
+
+@pytest.mark.parametrize("modes", [1, 79, 80, 1000])
+def test_probe_is_the_steps_field(gpu, modes):
+    """eval_field in FP32 returns the step's field, bit for bit.  With |u| =
+    2^-13 (gamma rounds to 1) along one axis and qm dt / 2 = 2^-30, a step
+    turns the momentum by 2 t x u with t = 2^-30 B, all exact scalings by
+    powers of two: the terms left out are 2^-30 |B|^2 / B_c of what is kept,
+    below half a unit in the last place for |B_c| > |B|^2 / 32."""
+    rows = mode_table(modes, kmin=0.05, kmax=50.0, rms=0.5, seed=78)
+    n, w, hf = 333, 2.0 ** -13, 2.0 ** -30
+    p = init_particles(n, (0, 0, 0), (1000, 1000, 1000), 0.5, seed=79)
+    gpu.set_field_modes(rows, 1.0)
+    b = gpu.eval_field(np.c_[p[:, :3], np.zeros(n)], abi.TP_FP32_MIXED)[:, :3]
+    prm = abi.make_params(dt=2 * hf, estep=1, lo=(0, 0, 0), hi=(1000, 1000, 1000), qm=1.0,
+                          pusher=abi.TP_PUSH_BORIS, precision=abi.TP_FP32_MIXED,
+                          bc_flag=abi.TP_BC_NONE)
+    size = np.sqrt((b * b).sum(1))
+    for c in range(3):
+        a = (c + 1) % 3                      # u along a: component d gets 2 w hf B_c, up to sign
+        d = 3 - a - c
+        p[:, 4:7] = 0.0
+        p[:, 4 + a] = w
+        u = gpu.track_fixed(prm, p)["ptl"][:, 4:7]
+        ok = np.abs(b[:, c]) > size ** 2 / 32
+        assert ok.sum() > n // 2
+        sign = 1.0 if (a, c, d) in ((0, 1, 2), (1, 2, 0), (2, 0, 1)) else -1.0
+        assert np.array_equal(u[ok, d], sign * 2 * w * hf * b[ok, c]), c

@@ -1138,20 +1138,35 @@ __device__ __forceinline__ void modes_sum32(const float *tab32, int nmodes, floa
  * float x exactly, the table from double): the products h m', m h', m m', h l',
  * l h', m l', l m' first, then h h' added to them, so that only the last sum
  * rounds at the phase's own size (v_mfma_f32_16x16x16_bf16 with the first four
- * of the table's eight).  Products are exact, sums FP32.  The lane
+ * of the table's eight).  Products are exact.  The sums inside an instruction
+ * are the nearest float to the exact one in 0.997 of random cases with four
+ * terms; a small addend beside large products is cut off downwards, by 0.16
+ * units in the last place of the largest product on average.  The lane
  * then has the phases of one mode at 16 points and adds a_mode cos(phase) into
- * sums of its own; the 16 lanes of a row are summed at the end.
+ * sums of its own; the 16 lanes of a row are summed at the end.  The table's
+ * amplitudes make up for the hardware cosine, which is 3.2e-8 too small on
+ * average (COS_GAIN).
  *
- * Against the sums in 64 bits (1000 modes, kmax 48): rms error of the largest
- * k's phases 2.2e-5 revolutions at points up to 130, 1.3e-4 up to 1000, of the
- * field 3.1e-7 and 1.5e-6; a lane per point with FP32 FMAs (modes_sum32) has
- * 2.2e-5, 1.8e-4, 8.7e-7 and 2.0e-6.
+ * Against the sums in 64 bits at float points, 1000 modes, kmax 48: rms error
+ * of the field 3.0e-7 of its rms at points up to 130, 1.5e-6 up to 1000; a lane
+ * per point with FP32 FMAs (modes_sum32) has 8.3e-7 and 2.0e-6.  Over ten
+ * ensembles of 262,144 particles and 200 steps, this / modes_sum32 in the same
+ * step: positions 1.1e-8 / 1.6e-8, momenta 8.8e-7 / 1.0e-6, D sums 6.1e-9 (at
+ * most 9.7e-9) / 1.6e-8 (3.2e-8).  Taking the fraction of the h h' sum before
+ * the small products are added halves the field's error at 1000 and changes
+ * neither of the others' (1.3e-8, D 1.3e-8), for 1.9 of 11.0 ms.
  * Bound: issue of the cosine (8 cycles), its fraction and three FMAs a mode;
  * FMAs of vector registers only take 3 cycles, those of modes_sum32 with a
  * scalar operand 4, and its scalar loads stall a wavefront.  Cycles per 64
  * points and mode at one / two / four / eight waves a SIMD: 68 / 41 / 35 / 30,
  * modes_sum32 128 / 64 / 52 / 41. */
 #define MODES_WAVE32_LDS (64 * 4)    /* floats of LDS per wavefront */
+/* v_cos_f32 falls short of the cosine's magnitude by this share: projection of
+ * its values on the cosine over 2^22 arguments in [0, 1), -3.2e-8 (2.9e-8 to
+ * 3.5e-8 in each quadrant).  As an error of the whole field it adds up over the
+ * steps: without it in the amplitudes, the D sums are off by 4e-8 to 1e-7 with
+ * the same sign in every ensemble. */
+#define COS_GAIN 3.23e-8
 /* modes from which it is used: the splits and the row sums cost as much as
  * some 70 modes.  262,144 particles x 200 steps, per lane / per wavefront: 64
  * modes 1.25 / 1.29 ms, 96 modes 1.80 / 1.64, 1000 modes 18.6 / 12.0; 5000

@@ -1598,7 +1598,8 @@ static int modes_parts(tp_ctx *c, int nmodes, const double *rows)
                 o[0] = h; o[1] = md; o[2] = l;
             }
         }
-        for (int q = 0; q < 3; q++) ta[64 * (size_t)(m / 16) + 4 * (m % 16) + q] = (float)r[3 + q];
+        for (int q = 0; q < 3; q++)
+            ta[64 * (size_t)(m / 16) + 4 * (m % 16) + q] = (float)(r[3 + q] * (1.0 + COS_GAIN));
     }
     int rc = TP_OK;
     if (hipMalloc(&c->modesb, nb * sizeof(unsigned short)) != hipSuccess) {

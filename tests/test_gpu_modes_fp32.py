@@ -109,3 +109,32 @@ def test_probe_is_the_steps_field(gpu, modes):
         assert ok.sum() > n // 2
         sign = 1.0 if (a, c, d) in ((0, 1, 2), (1, 2, 0), (2, 0, 1)) else -1.0
         assert np.array_equal(u[ok, d], sign * 2 * w * hf * b[ok, c]), c
+
+
+@pytest.mark.parametrize("modes,box,rms", [(100, 130, 3.9e-7), (300, 130, 3.9e-7),
+                                           (1000, 130, 3.9e-7), (1000, 1000, 1.9e-6)])
+def test_field_error(gpu, modes, box, rms):
+    """The step's field (the probe returns its bits) against 64 bits at points
+    that are floats, where nothing but the sum errs.
+
+    rms: phases of up to kmax box / 2 pi = 1000 revolutions (8000) rounded at
+    2^-14 (2^-11), 1.9e-4 rad (1.5e-3) for the largest k, which hold 1e-3 of the
+    field's square; amplitude, cosine and sum, 2^-24 each and growing with the
+    partial sums.  Measured 2.3e-7 to 3.0e-7 (1.5e-6); FP32 FMAs a point to a
+    lane 4.0e-7 to 8.4e-7 (2.1e-6), twice the error.
+
+    Along the field: errors of either sign average out, but for the rounding of
+    the few largest amplitudes, up to 1.5e-8 a table and 5e-9 over eight of them;
+    the hardware cosine's own gain error of 3.2e-8 would show."""
+    gain = []
+    for seed in range(81, 89):
+        rows = mode_table(modes, kmin=0.05, kmax=48.0, rms=0.5, seed=seed)
+        x = np.random.default_rng(seed).uniform(0, box, (20000, 3))
+        pts = np.c_[x.astype(np.float32).astype(np.float64), np.zeros(len(x))]
+        gpu.set_field_modes(rows, 0.0)
+        b = gpu.eval_field(pts, abi.TP_FP32_MIXED)[:, :3]
+        e = gpu.eval_field(pts, abi.TP_FP64)[:, :3]      # the oracle's to 1e-14
+        n2 = (e * e).sum(1).mean()
+        assert np.sqrt(((b - e) ** 2).sum(1).mean() / n2) < rms
+        gain.append(((b - e) * e).sum(1).mean() / n2)
+    assert abs(np.mean(gain)) < 1.5e-8

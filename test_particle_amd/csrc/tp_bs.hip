@@ -994,6 +994,10 @@ __device__ __forceinline__ void bs_body(const BsArgs &a)
                 modes_wave64(a.f, (lds_tab)modes_lds, act, ze[0], ze[1], ze[2], xp, e);
             else
                 modes_wave64(a.f, a.f.modesx, act, ze[0], ze[1], ze[2], xp, e);
+            /* here, out of the sum's way: inside it, the same test made the
+             * adaptive form 4 % slower by moving the loops' code */
+            if (__builtin_expect(modes_far(a.f, ze[0], ze[1], ze[2]), 0))
+                modes_sum_far(a.f, ze[0], ze[1], ze[2], e);
         } else
             get_emf64<FK>(a.f, ze[0], ze[1], ze[2], act ? L.xe : 0.0, e);
         int next = DENSE && L.pi >= 0 && L.phase == PH_OUT ? NX_DONE : NX_NONE;

@@ -104,6 +104,7 @@ struct FieldDev {
     const double *modesx;
     int nquads;
     double b0z;
+    double modes_reach;          /* coordinates up to which no phase is far (modes_far) */
     /* the same table for FP32: (kx ky kz phi) / 2 pi, ax ay az 0 per mode */
     const float *modes32;
     /* and for the FP32 forms' matrix products (modes_wave32): n16 groups of 16
@@ -801,6 +802,32 @@ __device__ __forceinline__ void mhd_e32(EmfF &o)
     o.ez = o.bx * vy - o.by * vx;
 }
 
+/* whether a phase of the mode table can be beyond tp_cos_pi_with's range (or
+ * no number) at the point of any lane here */
+__device__ __forceinline__ bool modes_far(const FieldDev &f, double x, double y, double z)
+{
+    return __any(!(fmax(fmax(fabs(x), fabs(y)), fabs(z)) < f.modes_reach));
+}
+
+/* the mode sum there, mode by mode */
+__device__ __forceinline__ void modes_sum_far(const FieldDev &f, double x, double y, double z,
+                                              Emf &o)
+{
+    typedef const double __attribute__((address_space(4))) *ctab;
+    const ctab tab = (ctab)f.modes;
+    double bx = 0.0, by = 0.0, bz = 0.0;
+#pragma unroll 1
+    for (int n = 0; n < f.nmodes; n++) {
+        const ctab m = tab + 7 * n;
+        const double cs = tp_cos_pi(fma(m[2], z, fma(m[1], y, fma(m[0], x, m[6]))));
+        bx = fma(m[3], cs, bx);
+        by = fma(m[4], cs, by);
+        bz = fma(m[5], cs, bz);
+    }
+    o.bx = bx; o.by = by; o.bz = f.b0z + bz;
+    o.ex = 0.0; o.ey = 0.0; o.ez = 0.0;
+}
+
 /* ------------------------------------------------------------------ */
 /* get_emf, FP64 (src/emfields.c:32-60)                                */
 /* ------------------------------------------------------------------ */
@@ -916,6 +943,10 @@ __device__ __forceinline__ void get_emf64(const FieldDev &f, double x, double y,
         /* four independent cosines per iteration (instruction-level
          * parallelism for the FP64 FMA chains), summed in mode order */
         double bx = 0.0, by = 0.0, bz = 0.0;
+        if (__builtin_expect(modes_far(f, x, y, z), 0)) {
+            modes_sum_far(f, x, y, z, o);
+            return;
+        }
         const int n4 = f.nmodes & ~3;
         const tp_cos_pi_consts ck = tp_cos_pi_init();
         /* the table is read-only for the whole kernel: read it through the
@@ -1057,9 +1088,10 @@ __device__ __forceinline__ void modes_groups64(TAB tab, int nquads, double *xp)
     for (int g = 0; g < G; g++) slot[64 * g] = acc[g];
 }
 
-/* get_emf64<FK_MODES> at the points of the lanes with `want`; every lane of
- * the wavefront calls it (uniform control flow), xp is the wavefront's own
- * MODES_WAVE_LDS doubles of LDS, tab the table or its copy. */
+/* get_emf64<FK_MODES> at the points of the lanes with `want`, for phases within
+ * tp_cos_pi_with's range (modes_far); every lane of the wavefront calls it
+ * (uniform control flow), xp is the wavefront's own MODES_WAVE_LDS doubles of
+ * LDS, tab the table or its copy. */
 template <class TAB>
 __device__ __forceinline__ void modes_wave64(const FieldDev &f, TAB tab, bool want, double x,
                                              double y, double z, double *xp, Emf &o)

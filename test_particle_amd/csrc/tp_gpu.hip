@@ -1681,6 +1681,17 @@ int tp_gpu_set_field_modes(tp_ctx *c, int nmodes, const double *rows, double b0z
     }
     int rc = modes_quads(c, nmodes, rows);
     if (rc) return rc;
+    /* |kx x| + |ky y| + |kz z| + |phi| < TP_COS_PI_MAX for coordinates below
+     * modes_reach; a table that is not finite has no reach */
+    double k = 0.0, phi = 0.0;
+    bool finite = true;
+    for (int m = 0; m < nmodes; m++) {
+        const double *r = rows + 7 * m, s = fabs(r[0]) + fabs(r[1]) + fabs(r[2]);
+        if (!isfinite(s) || !isfinite(r[6])) finite = false;
+        k = fmax(k, s);
+        phi = fmax(phi, fabs(r[6]));
+    }
+    c->f.modes_reach = finite && phi < TP_COS_PI_MAX ? (TP_COS_PI_MAX - phi) / k : 0.0;
     c->f.nmodes = nmodes;
     c->f.modes = c->modes;
     c->f.modesx = c->modesx;

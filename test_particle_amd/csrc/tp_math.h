@@ -48,6 +48,15 @@ TP_HD double tp_const(double c)
     return c;
 }
 
+/* the same, not formed ahead of its use (of a loop around it) */
+TP_HD double tp_const_here(double c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(c));
+#endif
+    return c;
+}
+
 /* v with its sign flipped if the lowest bit of t is set */
 TP_HD double tp_flip_by_low_bit(double v, double t)
 {
@@ -180,8 +189,12 @@ TP_HD double tp_cos(double x)
  * first product exact by the same fma argument as above (|x| < 2^52); a
  * third part would move r by less than 2^-57 even there.  17 operations; the
  * comparison and the third part make it 22 and give the same bits (3e7
- * arguments in each of |x| < 1.5, 30, 1e3, 1e5, 1e9).
+ * arguments in each of |x| < 1.5, 30, 1e3, 1e5, 1e9).  From 2^51 pi on the sum
+ * has no room for k's lowest bit: a sum over modes whose phases can reach
+ * TP_COS_PI_MAX takes tp_cos_pi.
  */
+#define TP_COS_PI_MAX 7e15
+
 typedef struct tp_cos_pi_consts {
     double inv_pi, round, pi_hi, pi_lo, c[10];
 } tp_cos_pi_consts;
@@ -227,10 +240,33 @@ TP_HD double tp_cos_pi_with(double x, const tp_cos_pi_consts *q)
     return tp_flip_by_low_bit(fma(-z, p, 1.0), t);  /* 1 - z/2 + z^2/24 - ... */
 }
 
+/* the same for an argument of any size (NaN for NaN and infinities): from
+ * TP_COS_PI_MAX on k is rounded by itself, pi has a third part and the parity
+ * comes from k.  The constants are formed where they are used: beside a loop
+ * that holds tp_cos_pi_with's there is no room for them. */
 TP_HD double tp_cos_pi(double x)
 {
-    const tp_cos_pi_consts q = tp_cos_pi_init();
-    return tp_cos_pi_with(x, &q);
+    const int near = fabs(x) < TP_COS_PI_MAX;
+    const double inv_pi = tp_const_here(0x1.45f306dc9c883p-2);
+    const double t = fma(x, inv_pi, 0x1.8p52);
+    const double k = near ? t - 0x1.8p52 : rint(x * inv_pi);
+    double r = fma(-k, tp_const_here(0x1.921fb54442d18p+1), x);
+    r = fma(-k, tp_const_here(0x1.1a62633145c07p-53), r);
+    if (!near) r = fma(-k, tp_const_here(-0x1.f1976b7ed8fbcp-109), r);
+    const double z = r * r;
+    double p = tp_const_here(0x1.0ce396db7f853p-70);
+    p = fma(p, z, tp_const_here(-0x1.e542ba4020225p-62));
+    p = fma(p, z, tp_const_here(0x1.6827863b97d97p-53));
+    p = fma(p, z, tp_const_here(-0x1.ae7f3e733b81fp-45));
+    p = fma(p, z, tp_const_here(0x1.93974a8c07c9dp-37));
+    p = fma(p, z, tp_const_here(-0x1.1eed8eff8d898p-29));
+    p = fma(p, z, tp_const_here(0x1.27e4fb7789f5cp-22));
+    p = fma(p, z, tp_const_here(-0x1.a01a01a01a01ap-16));
+    p = fma(p, z, tp_const_here(0x1.6c16c16c16c17p-10));
+    p = fma(p, z, tp_const_here(-0x1.5555555555555p-5));
+    p = fma(p, z, 0.5);
+    const double c = fma(-z, p, 1.0), half = k * 0.5;
+    return near ? tp_flip_by_low_bit(c, t) : (half == floor(half) ? c : -c);
 }
 
 /*

@@ -74,6 +74,40 @@ def test_lanes_per_wavefront(gpu, oracle_tp, n, dense):
     assert np.array_equal(r["nsteps"][pick], ref["nsteps"])
 
 
+def test_far_phases(gpu, oracle_tp):
+    """Phases beyond the range in which the sum that rounds them keeps their
+    parity (7e15): the probe, and both adaptive forms' sum with near and far
+    points in one wavefront, bit for bit the oracle's."""
+    rows = mode_table(40, kmin=0.3, kmax=30.0, rms=0.5, seed=66)
+    f = oracle_tp.Field.modes(rows, 1.0)
+    gpu.set_field_modes(rows, 1.0)
+    rng = np.random.default_rng(67)
+    pts = np.exp(rng.uniform(np.log(1e12), np.log(1e16), (500, 4))) * rng.choice([-1, 1], (500, 4))
+    pts[7] = [np.nan, 0, 0, 0]
+    pts[8] = [0, np.inf, 0, 0]
+    b = gpu.eval_field(pts)
+    assert np.array_equal(b, oracle_tp.eval_field(f, pts), equal_nan=True)
+    assert np.isnan(b[7:9, :3]).all() and np.isfinite(b[9:]).all()
+    p = _ptl(100)
+    p[::3, 0] = 2.0 ** 49 + 1000.0 * np.arange(34)      # phases of up to 1.4e16
+    p[1::3, 1] = -2.0 ** 49
+    bs = abi.make_bs_params(rtol=1e-8, atol=1e-10, t_end_gyro=0.2, b_ref=1.0)
+    r = gpu.track_adaptive(bs, p)
+    ref = oracle_tp.bs_track(f, bs, p)
+    assert np.array_equal(r["ptl"], ref["ptl"]) and np.array_equal(r["nsteps"], ref["nsteps"])
+    rows[5, 6] = 1e16                                    # a phase that is far by itself
+    f = oracle_tp.Field.modes(rows, 1.0)
+    gpu.set_field_modes(rows, 1.0)
+    p = _ptl(100)
+    bs = abi.make_bs_params(rtol=1e-8, atol=1e-10)
+    prm = abi.make_params(dt=0.05, estep=20, lo=(0, 0, 0), hi=(10, 10, 10), nbins=52, nt_out=2,
+                          einterval_t=10, dcoeff_interval=10, emin=1e-4, emax=10.0)
+    r = gpu.track_adaptive_diag(bs, prm, p)
+    ref = oracle_tp.bs_track_diag(f, bs, prm, p)
+    for k in ("ptl", "nsteps", "espect"):
+        assert np.array_equal(r[k], ref[k]), k
+
+
 def test_empty_table(oracle_tp):
     """No modes at all: the uniform guide field, through both forms and the
     launch-shape trials."""

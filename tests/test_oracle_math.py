@@ -34,6 +34,20 @@ def test_tp_sincos_special_values(oracle_tp):
     assert np.isnan(s[4]) and np.isnan(c[5])
 
 
+@pytest.mark.parametrize("lo,hi,tol", [(1.0, 1e9, 5e-16), (1e9, 7e15, 5e-16),
+                                       (7e15, 2.0 ** 53, 1e-12), (2.0 ** 53, 2.0 ** 54, 1e-11)])
+def test_mode_cosine_of_large_phases(oracle_tp, lo, hi, tol):
+    """cos of a mode's phase up to 2^54.  Below 2^51 pi (7.07e15) within an ulp
+    or two; beyond, k = rint(x/pi) has lost its last bits, so |r| grows past pi/2 and
+    the polynomial's truncation with it: r = pi/2 + 1, 2 gives r^24 / 24! of
+    4e-14, 6e-12 -- but the sign is right."""
+    f = oracle_tp.Field.modes(np.array([[1.0, 0, 0, 1.0, 0, 0, 0], [0, 0, 0, 0, 1.0, 0, 0]]), 0.0)
+    x = np.exp(np.random.default_rng(8).uniform(np.log(lo), np.log(hi), 20000))
+    b = oracle_tp.eval_field(f, np.c_[np.minimum(x, hi), np.zeros((len(x), 3))])
+    assert np.abs(b[:, 0] - np.cos(np.minimum(x, hi))).max() < tol
+    assert (b[:, 1] == 1.0).all()
+
+
 def test_ellint_against_scipy(oracle_libm):
     from scipy.special import ellipe, ellipk
     for k in np.linspace(0, 0.999999, 200):

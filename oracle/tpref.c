@@ -54,6 +54,7 @@ void tpref_set_math(int use_libm) { g_use_libm = use_libm; }
 void tpref_set_carry_stale(int on) { g_carry_stale = on; }
 
 void tpref_sincos(double x, double *s, double *c) { tp_sincos(x, s, c); }
+void tpref_sincos_angle(double x, double *s, double *c) { tp_sincos_angle(x, s, c); }
 
 static void ellint_ref(double k, double *elle, double *ellk);
 void tpref_ellint_ref(double k, double *elle, double *ellk) { ellint_ref(k, elle, ellk); }

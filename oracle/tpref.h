@@ -104,6 +104,7 @@ int  tpref_poincare_map(const tpref_field *f, const tp_pmap_params *prm, int n,
                         int *ncrossed, long long *nsteps, int nthreads, double *seconds);
 /* exported for the tests of the shared routines */
 void tpref_sincos(double x, double *s, double *c);
+void tpref_sincos_angle(double x, double *s, double *c);
 void tpref_ellint(double k, double *elle, double *ellk);
 void tpref_ellint_ref(double k, double *elle, double *ellk);
 

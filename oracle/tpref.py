@@ -86,6 +86,7 @@ def lib():
                                          P(d), P(d), P(i), P(ctypes.c_longlong), i, P(d)]
         L.tpref_poincare_map.restype = i
         L.tpref_sincos.argtypes = [d, P(d), P(d)]
+        L.tpref_sincos_angle.argtypes = [d, P(d), P(d)]
         L.tpref_ellint.argtypes = [d, P(d), P(d)]
         L.tpref_ellint_ref.argtypes = [d, P(d), P(d)]
         L.tpref_set_trajectory.argtypes = [i, P(i), P(d), P(i)]
@@ -382,14 +383,15 @@ def bs_track(field, params, ptl, nthreads=1):
                 failed=tot[3], seconds=secs.value)
 
 
-def sincos(x):
+def sincos(x, angle=False):
     L = lib()
+    fn = L.tpref_sincos_angle if angle else L.tpref_sincos
     x = np.asarray(x, dtype=np.float64).ravel()
     s = np.empty_like(x)
     c = np.empty_like(x)
     a, b = ctypes.c_double(), ctypes.c_double()
     for i, v in enumerate(x):
-        L.tpref_sincos(float(v), ctypes.byref(a), ctypes.byref(b))
+        fn(float(v), ctypes.byref(a), ctypes.byref(b))
         s[i], c[i] = a.value, b.value
     return s, c
 

@@ -1472,7 +1472,7 @@ __device__ __forceinline__ void wirz_step64(const FieldDev &f, GC &gc, Ptl &p,
     double om = qm * Btot * ig;
     double dthe = om * dt;
     double sd, cd;
-    tp_sincos(dthe * 0.5, &sd, &cd);
+    tp_sincos_angle(dthe * 0.5, &sd, &cd);
     double t1 = dth * vd * 1.0;
     double t2 = gR * sd;
     double t3 = -gR * (1.0 - cd);
@@ -1492,7 +1492,7 @@ __device__ __forceinline__ void wirz_step64(const FieldDev &f, GC &gc, Ptl &p,
     rx = hy * pz - hz * py; ry = hz * px - hx * pz; rz = hx * py - hy * px;
     om = qm * Btot * ig;
     dthe = om * dt;
-    tp_sincos(dthe, &sd, &cd);
+    tp_sincos_angle(dthe, &sd, &cd);
     double wx = hx * vd + vp * (cd * px - sd * rx);
     double wy = hy * vd + vp * (cd * py - sd * ry);
     double wz = hz * vd + vp * (cd * pz - sd * rz);

@@ -105,6 +105,35 @@ TP_HD double tp_flip_sign(double v, uint32_t mask)
 #define TP_PIO2_2    0x1.1a62633145c07p-54
 #define TP_PIO2_3   -0x1.f1976b7ed8fbcp-110
 
+/* sin and cos of r + rlo, |r| <= pi/4 and a little */
+TP_HD void tp_sincos_reduced(double r, double rlo, double *sp, double *cp)
+{
+    double z = r * r;
+    /* sin(r) = r + r z Ps(z) */
+    double ps = 0x1.952c77030ad4ap-49;                      /*  1/17! */
+    ps = fma(ps, z, -0x1.ae7f3e733b81fp-41);                /* -1/15! */
+    ps = fma(ps, z, 0x1.6124613a86d09p-33);                 /*  1/13! */
+    ps = fma(ps, z, -0x1.ae64567f544e4p-26);                /* -1/11! */
+    ps = fma(ps, z, 0x1.71de3a556c734p-19);                 /*  1/9!  */
+    ps = fma(ps, z, -0x1.a01a01a01a01ap-13);                /* -1/7!  */
+    ps = fma(ps, z, 0x1.1111111111111p-7);                  /*  1/5!  */
+    ps = fma(ps, z, -0x1.5555555555555p-3);                 /* -1/3!  */
+    *sp = r + fma(r * z, ps, rlo);
+    /* cos(r) = 1 - z/2 + z^2 Pc(z) */
+    double pc = 0x1.6827863b97d97p-53;                      /*  1/18! */
+    pc = fma(pc, z, -0x1.ae7f3e733b81fp-45);                /* -1/16! */
+    pc = fma(pc, z, 0x1.93974a8c07c9dp-37);                 /*  1/14! */
+    pc = fma(pc, z, -0x1.1eed8eff8d898p-29);                /* -1/12! */
+    pc = fma(pc, z, 0x1.27e4fb7789f5cp-22);                 /*  1/10! */
+    pc = fma(pc, z, -0x1.a01a01a01a01ap-16);                /* -1/8!  */
+    pc = fma(pc, z, 0x1.6c16c16c16c17p-10);                 /*  1/6!  */
+    pc = fma(pc, z, -0x1.5555555555555p-5);                 /* -1/4!  */
+    pc = -pc;                                               /* z^2 * (1/4! - ...) */
+    double hz = 0.5 * z;
+    double wc = 1.0 - hz;
+    *cp = wc + (((1.0 - wc) - hz) + fma(z * z, pc, -r * rlo));
+}
+
 /* sin(x) and cos(x) together; NaN/Inf in give NaN out. */
 TP_HD void tp_sincos(double x, double *sp, double *cp)
 {
@@ -131,38 +160,25 @@ TP_HD void tp_sincos(double x, double *sp, double *cp)
     double rlo = (r1 - (r - bb)) + (-w - bb);
     rlo = rlo - werr;
     rlo = fma(-k, TP_PIO2_3, rlo);
-
-    double z = r * r;
-    /* sin(r) = r + r z Ps(z) */
-    double ps = 0x1.952c77030ad4ap-49;                      /*  1/17! */
-    ps = fma(ps, z, -0x1.ae7f3e733b81fp-41);                /* -1/15! */
-    ps = fma(ps, z, 0x1.6124613a86d09p-33);                 /*  1/13! */
-    ps = fma(ps, z, -0x1.ae64567f544e4p-26);                /* -1/11! */
-    ps = fma(ps, z, 0x1.71de3a556c734p-19);                 /*  1/9!  */
-    ps = fma(ps, z, -0x1.a01a01a01a01ap-13);                /* -1/7!  */
-    ps = fma(ps, z, 0x1.1111111111111p-7);                  /*  1/5!  */
-    ps = fma(ps, z, -0x1.5555555555555p-3);                 /* -1/3!  */
-    double s = r + fma(r * z, ps, rlo);
-    /* cos(r) = 1 - z/2 + z^2 Pc(z) */
-    double pc = 0x1.6827863b97d97p-53;                      /*  1/18! */
-    pc = fma(pc, z, -0x1.ae7f3e733b81fp-45);                /* -1/16! */
-    pc = fma(pc, z, 0x1.93974a8c07c9dp-37);                 /*  1/14! */
-    pc = fma(pc, z, -0x1.1eed8eff8d898p-29);                /* -1/12! */
-    pc = fma(pc, z, 0x1.27e4fb7789f5cp-22);                 /*  1/10! */
-    pc = fma(pc, z, -0x1.a01a01a01a01ap-16);                /* -1/8!  */
-    pc = fma(pc, z, 0x1.6c16c16c16c17p-10);                 /*  1/6!  */
-    pc = fma(pc, z, -0x1.5555555555555p-5);                 /* -1/4!  */
-    pc = -pc;                                               /* z^2 * (1/4! - ...) */
-    double hz = 0.5 * z;
-    double wc = 1.0 - hz;
-    double c = wc + (((1.0 - wc) - hz) + fma(z * z, pc, -r * rlo));
-
+    double s, c;
+    tp_sincos_reduced(r, rlo, &s, &c);
     /* (s, c), (c, -s), (-s, -c), (-c, s) in quadrants 0 to 3: a swap and two
      * sign bits */
     const double so = tp_flip_sign(q & 1u ? c : s, (q & 2u) << 30);
     const double co = tp_flip_sign(q & 1u ? s : c, ((q + 1u) & 2u) << 30);
     *sp = so;
     *cp = co;
+}
+
+/* tp_sincos for angles that are small as a rule (a step's rotation): below
+ * 0.75 the reduction gives k = 0, r = x and rlo = 0, and is left out with its
+ * quadrants (same bits).  Wirz, 33,000 particles x 200 steps, tp_sincos / this:
+ * MHD grid 748 / 723 us, PIC grid 712 / 684, its textbook gather on two slices
+ * 845 / 823; 140,000 in the ABC field 1188 / 1144. */
+TP_HD void tp_sincos_angle(double x, double *sp, double *cp)
+{
+    if (fabs(x) < 0.75) tp_sincos_reduced(x, 0.0, sp, cp);
+    else tp_sincos(x, sp, cp);
 }
 
 TP_HD double tp_sin(double x)

@@ -34,6 +34,21 @@ def test_tp_sincos_special_values(oracle_tp):
     assert np.isnan(s[4]) and np.isnan(c[5])
 
 
+def test_sincos_angle_is_sincos(oracle_tp):
+    """The form for small angles leaves the reduction out below 0.75: the same
+    bits, signed zeros included, on either side of the line."""
+    rng = np.random.default_rng(9)
+    x = np.concatenate([
+        [0.0, 5e-324, 1e-310, 2.0 ** -1022, 1e-160, 1e-17, 0.75, np.nextafter(0.75, 0),
+         np.nextafter(0.75, 1), np.pi / 4, np.pi / 2, np.pi, 1e9, 2.0 ** 50, 1e17, np.inf, np.nan],
+        rng.uniform(0, 0.75, 20000), 10.0 ** rng.uniform(-300, 0, 20000),
+        10.0 ** rng.uniform(-1, 16, 20000)])
+    x = np.concatenate([x, -x])
+    for a, b in zip(oracle_tp.sincos(x), oracle_tp.sincos(x, angle=True)):
+        assert np.array_equal(a, b, equal_nan=True)
+        assert np.array_equal(np.signbit(a[~np.isnan(a)]), np.signbit(b[~np.isnan(b)]))
+
+
 @pytest.mark.parametrize("lo,hi,tol", [(1.0, 1e9, 5e-16), (1e9, 7e15, 5e-16),
                                        (7e15, 2.0 ** 53, 1e-12), (2.0 ** 53, 2.0 ** 54, 1e-11)])
 def test_mode_cosine_of_large_phases(oracle_tp, lo, hi, tol):

@@ -1781,12 +1781,16 @@ int tp_gpu_load_particles(tp_ctx *c, int n, const tp_particle *ptl, const tp_par
 static int block_size_for(const tp_ctx *c, int n)
 {
     /* Blocks of four wavefronts, which go to the four SIMDs of a compute unit,
-     * unless that leaves compute units idle; then of one.  Blocks of two put
-     * both blocks of a compute unit on the same two SIMDs: 65,536 particles in
-     * the ABC field, one wavefront to a SIMD, 423 us per 100 Wirz steps in
-     * blocks of 128 lanes, 270 in blocks of 256. */
-    int cu = c->num_cu > 0 ? c->num_cu : 256;
-    return (n + 255) / 256 >= cu ? 256 : 64;
+     * where they fill the compute units twice or more, or exactly once: blocks
+     * of two put both blocks of a compute unit on the same two SIMDs (65,536
+     * particles in the ABC field, one wavefront to a SIMD, 423 us per 100 Wirz
+     * steps in blocks of 128 lanes, 270 in blocks of 256).  In between, blocks of
+     * two spread better (double grid, FP64 Boris, 70,000 particles x 200 steps:
+     * 1.26 ms in blocks of 128, 1.54 in blocks of 256; the other fields are within
+     * 8 % either way); with fewer particles, single wavefronts do. */
+    const int cu = c->num_cu > 0 ? c->num_cu : 256, n256 = (n + 255) / 256;
+    if (n256 >= 2 * cu || n256 == cu) return 256;
+    return (n + 127) / 128 >= 2 * cu ? 128 : 64;
 }
 
 /* Buffers of one fixed-step run: the context's own (tp_gpu_run_fixed) or the

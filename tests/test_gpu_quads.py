@@ -67,3 +67,13 @@ def test_unusual_states(gpu, oracle_tp, pusher):
     ref = oracle_tp.track_fixed(oracle_tp.Field.abc(1.0, 1.0, 1.0), prm, p, nthreads=1)
     assert np.array_equal(r["ptl"], ref["ptl"], equal_nan=True)
     assert np.array_equal(r["nsteps"], ref["nsteps"])
+
+
+@pytest.mark.parametrize("n", [65536, 65537, 70001, 130816, 130817])
+def test_block_sizes(gpu, oracle_tp, n):
+    """Blocks of 256, 128 and 64 lanes and the lines between them."""
+    p = init_particles(n, LO, HI, 0.7, seed=84)
+    prm = params(abi.TP_PUSH_BORIS, 0, 10, dcoeff_interval=5)
+    gpu.set_field_abc(1.0, 0.7, -0.4)
+    r = gpu.track_fixed(prm, p)
+    compare(r, oracle_tp.track_fixed(oracle_tp.Field.abc(1.0, 0.7, -0.4), prm, p, nthreads=1))

@@ -395,7 +395,10 @@ int tp_gpu_track_adaptive(tp_ctx *ctx, const tp_bs_params *p, int n, tp_particle
  * 65,536) resident particles over a short horizon for each candidate
  * (block, waves_per_cu), keeps the state unchanged, writes the choice to
  * *block and *waves_per_cu and, if cache_path is given, caches it there
- * keyed by field kind, mode count and tolerance (read back on later calls). */
+ * keyed by field kind, mode count, tolerance and the number of particles that
+ * an ensemble of this size gives a wavefront (read back on later calls; entries
+ * of other kernel versions are left alone).  Runs whose ensemble gives a
+ * wavefront another number of particles take the default shape. */
 int tp_gpu_tune_adaptive(tp_ctx *ctx, const tp_bs_params *p, const char *cache_path,
                          int *block, int *waves_per_cu);
 

@@ -1222,6 +1222,24 @@ static int bs_lanes(const tp_ctx *c, int wpc, int n)
     return lanes;
 }
 
+/* What the tuner's choice depends on besides field and tolerance: how many
+ * particles a wavefront takes in an ensemble of n. */
+static int bs_class(const tp_ctx *c, int n) { return bs_lanes(c, 4, n); }
+
+/* the launch shape: the caller's, else the tuner's for ensembles of this
+ * class, else the default */
+static void bs_shape(const tp_ctx *c, const tp_bs_params *p, int n, int *block, int *wpc)
+{
+    *block = c->f.kind == FK_MODES ? 256 : 64;
+    *wpc = 8;
+    if (c->bs_tuned[0] && c->bs_tuned[2] == bs_class(c, n)) {
+        *block = c->bs_tuned[0];
+        *wpc = c->bs_tuned[1];
+    }
+    if (p->block) *block = p->block;
+    if (p->waves_per_cu) *wpc = p->waves_per_cu;
+}
+
 static dim3 bs_grid(const tp_ctx *c, int block, int wpc, int n, int lanes)
 {
     int cu = c->num_cu > 0 ? c->num_cu : 256;
@@ -1280,13 +1298,8 @@ int tp_gpu_run_adaptive(tp_ctx *c, const tp_bs_params *p, tp_bs_stats *stats)
     HIPCHK(hipSetDevice(c->device));
     if ((rc = bs_ensure_ctr(c))) return rc;
     const int n = c->s.n;
-    int block = p->block, wpc = p->waves_per_cu;
-    if (block == 0 || wpc == 0) {
-        int tb = c->f.kind == FK_MODES ? 256 : 64, tw = 8;
-        if (c->bs_tune_block) { tb = c->bs_tune_block[0]; tw = c->bs_tune_block[1]; }
-        if (block == 0) block = tb;
-        if (wpc == 0) wpc = tw;
-    }
+    int block, wpc;
+    bs_shape(c, p, n, &block, &wpc);
     const int cap = p->max_attempts > 0 ? p->max_attempts : 10000000;
     BsArgs a;
     State &S = c->s;
@@ -1370,13 +1383,8 @@ int tp_gpu_run_adaptive_diag(tp_ctx *c, const tp_bs_params *p, const tp_track_pa
     const int nd = q->estep / q->dcoeff_interval + 1;
     int nframes = q->estep / q->einterval_t;
     if (nframes > q->nt_out) nframes = q->nt_out;
-    int block = p->block, wpc = p->waves_per_cu;
-    if (block == 0 || wpc == 0) {
-        int tb = c->f.kind == FK_MODES ? 256 : 64, tw = 8;
-        if (c->bs_tune_block) { tb = c->bs_tune_block[0]; tw = c->bs_tune_block[1]; }
-        if (block == 0) block = tb;
-        if (wpc == 0) wpc = tw;
-    }
+    int block, wpc;
+    bs_shape(c, p, n, &block, &wpc);
     const int lanes = bs_lanes(c, wpc, n);
     const dim3 grid = bs_grid(c, block, wpc, n, lanes);
     const long nl = (long)grid.x * (block / 64) * lanes;
@@ -1489,9 +1497,10 @@ int tp_gpu_tune_adaptive(tp_ctx *c, const tp_bs_params *p, const char *cache_pat
     bs_fn fn = pick_bs(c->f.kind);
     if (!fn) return TP_E_ARG;
     HIPCHK(hipSetDevice(c->device));
+    /* "k2": timed on the present kernels; entries of others do not count */
     char key[160];
-    snprintf(key, sizeof(key), "fk=%d modes=%d rtol=%.3g kmax=%d cu=%d", c->f.kind,
-             c->f.nmodes, p->rtol, p->kmax, c->num_cu);
+    snprintf(key, sizeof(key), "k2 fk=%d modes=%d lanes=%d rtol=%.3g kmax=%d cu=%d", c->f.kind,
+             c->f.nmodes, bs_class(c, c->s.n), p->rtol, p->kmax, c->num_cu);
     int best_b = 0, best_w = 0;
     if (cache_path) {
         FILE *fp = fopen(cache_path, "r");
@@ -1537,7 +1546,7 @@ int tp_gpu_tune_adaptive(tp_ctx *c, const tp_bs_params *p, const char *cache_pat
                 bs_fill_args(c, p, a, nt, buf, buf + nt, buf + 2 * (size_t)nt,
                              buf + 3 * (size_t)nt, buf + 4 * (size_t)nt, buf + 5 * (size_t)nt,
                              buf + 6 * (size_t)nt, ib, ib + nt, c->bs_ctr, 24);
-                a.lanes = bs_lanes(c, wpcs[wi], c->s.n);
+                a.lanes = bs_lanes(c, wpcs[wi], nt);
                 const size_t lds = bs_lds(c, blocks[bi], wpcs[wi], a);
                 hipLaunchKernelGGL(k_bs_reset, dim3(1), dim3(64), 0, c->stream, c->bs_ctr);
                 (void)hipEventRecord(c->ev0, c->stream);
@@ -1574,12 +1583,9 @@ int tp_gpu_tune_adaptive(tp_ctx *c, const tp_bs_params *p, const char *cache_pat
         }
     }
     if (!best_b) return TP_E_HIP;
-    if (!c->bs_tune_block) {
-        c->bs_tune_block = (int *)malloc(2 * sizeof(int));
-        if (!c->bs_tune_block) return TP_E_NOMEM;
-    }
-    c->bs_tune_block[0] = best_b;
-    c->bs_tune_block[1] = best_w;
+    c->bs_tuned[0] = best_b;
+    c->bs_tuned[1] = best_w;
+    c->bs_tuned[2] = bs_class(c, c->s.n);
     if (block) *block = best_b;
     if (waves_per_cu) *waves_per_cu = best_w;
     return TP_OK;

@@ -63,7 +63,7 @@ struct tp_ctx {
     unsigned long long *bs_ctr = nullptr;
     hipGraphExec_t bs_graph = nullptr;
     unsigned long long bs_graph_key = 0;
-    int *bs_tune_block = nullptr;
+    int bs_tuned[3] = {0, 0, 0};                   /* tuner: block, waves per CU, class */
     /* adaptive stepper with diagnostics: dense-output scratch per lane, D
      * terms per particle and row, counted-out histogram */
     double *bs_ds = nullptr, *bs_dbuf = nullptr;

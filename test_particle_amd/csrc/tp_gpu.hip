@@ -900,7 +900,6 @@ void tp_gpu_finalize(tp_ctx *c)
     (void)hipFree(c->traj);
     (void)hipFree(c->traj_accum);
     (void)hipFree(c->traj_pts);
-    free(c->bs_tune_block);
     staging_release(c);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);

@@ -102,3 +102,24 @@ def test_bs_autotuner_cache(gpu, tmp_path):
     # the tuner leaves the resident particles untouched
     q, _ = gpu.store()
     assert np.array_equal(q, p)
+
+
+def test_bs_autotuner_keys(gpu, tmp_path):
+    """A choice counts for the kernels and the ensemble class it was timed for:
+    entries without them (older files) and of another class are not taken."""
+    rows = mode_table(16, kmin=0.5, kmax=10.0, rms=0.5, seed=56)
+    gpu.set_field_modes(rows, 1.0)
+    prm = abi.make_bs_params(rtol=1e-8, atol=1e-10, t_end_gyro=1.0)
+    cu = gpu.device_info()[1]
+    cache = tmp_path / "tune.txt"
+    cache.write_text(f"192 1 1e9 fk=5 modes=16 rtol=1e-08 kmax={prm.kmax} cu={cu}\n")
+    gpu.load(init_particles(2048, (0, 0, 0), (5, 5, 5), 0.5, seed=57))
+    b, _ = gpu.tune_adaptive(prm, str(cache))
+    lines = cache.read_text().splitlines()
+    assert b != 192 and len(lines) == 2
+    gpu.load(init_particles(70000, (0, 0, 0), (5, 5, 5), 0.5, seed=57))
+    gpu.tune_adaptive(prm, str(cache))
+    lines = cache.read_text().splitlines()
+    assert len(lines) == 3 and lines[1].split(None, 3)[3] != lines[2].split(None, 3)[3]
+    gpu.tune_adaptive(prm, str(cache))
+    assert cache.read_text().splitlines() == lines

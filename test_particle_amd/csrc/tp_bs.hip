@@ -1252,18 +1252,21 @@ static dim3 bs_grid(const tp_ctx *c, int block, int wpc, int n, int lanes)
 }
 
 /* The mode table goes to LDS when the copies of the blocks that share a
- * compute unit fit beside their point buffers (up to 1008 modes): its reads
- * then take some 100 cycles instead of those of an L2 hit, which a wavefront
- * alone on its SIMD waits for (131,072 particles, 1000 modes, 0.3
- * gyroperiods: 22.9 -> 20.5 ms).  Returns the launch's dynamic LDS. */
+ * compute unit fit: its reads then take some 100 cycles instead of those of an
+ * L2 hit, which a wavefront alone on its SIMD waits for (131,072 particles, 1000
+ * modes, 0.3 gyroperiods: 22.9 -> 20.5 ms of kernels).  The kernels' registers
+ * leave room for four wavefronts a compute unit, whatever is launched, and a
+ * block has the constants and the points of four wavefronts beside its copy.  A
+ * block's copy is at most 64 KiB (1008 modes).  Returns the launch's dynamic
+ * LDS. */
 static size_t bs_lds(const tp_ctx *c, int block, int wpc, BsArgs &a)
 {
     a.lds_quads = 0;
     if (c->f.kind != FK_MODES) return 0;
     const int quads = c->f.nquads + MODES_PAD_QUADS;
     const size_t bytes = (size_t)32 * sizeof(double) * quads;
-    const size_t per_cu = (size_t)(wpc * 64 + block - 1) / block;
-    const size_t fixed = 4 * MODES_WAVE_LDS * sizeof(double);
+    const size_t per_cu = (size_t)((wpc < 4 ? wpc : 4) * 64 + block - 1) / block;
+    const size_t fixed = 4 * MODES_WAVE_LDS * sizeof(double) + sizeof(BsConsts);
     if (bytes > 64 * 1024 || (bytes + fixed) * per_cu > 160 * 1024) return 0;
     a.lds_quads = quads;
     return bytes;

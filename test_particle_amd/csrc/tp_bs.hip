@@ -15,8 +15,7 @@
  *    field) never diverges across a wavefront; the mode sum runs on the
  *    matrix cores over the active lanes' points only (modes_wave64).  Only
  *    the tableau and controller bookkeeping between evaluations is divergent;
- *    its parts are run once an iteration for all lanes that need them, from
- *    registers.
+ *    its parts are run once an iteration for all lanes that need them.
  *  - The kernel is persistent: a fixed number of waves per compute unit pull
  *    particles from a global work queue.  Lanes whose particle reached its
  *    end time are refilled together: one atomic per wavefront hands out as
@@ -55,16 +54,17 @@ enum { NX_NONE = 0, NX_ACCEPT = 1, NX_START = 2, NX_ATTEMPT = 3, NX_SEQ = 4, NX_
        NX_DONE = 6 };
 
 /* Dense form: a lane whose step was accepted waits (PH_PREP, evaluating no
- * point, like an idle lane) until a quarter of its wavefront's lanes wait, or
- * no other lane is busy, and then they form their interpolants together.
- * prepare_dense is a long chain of per-lane scratch accesses; run for one
- * lane at a time it stalled the whole wavefront at almost every iteration.
- * Each lane's arithmetic is unchanged (same results). */
+ * point, like an idle lane) until BS_PREP lanes of its wavefront wait, or a
+ * quarter of those that take particles where that is fewer, or no other lane is
+ * busy, and then their interpolants are formed together, a lane per component
+ * (bs_prepare_dense): the wavefront waits for the rows in memory and the chain
+ * of divisions once for all of them.  Each step's arithmetic is the same
+ * whichever others it shares the batch with. */
 enum { Q_HEAD = 0, Q_ACC = 1, Q_REJ = 2, Q_RHS = 3, Q_FAIL = 4, Q_N = 8 };
 
 struct BsConsts {
-    int kmax, ktarg0, dense;
-    int nseq[10], cost[10], ipoint[11];
+    int kmax, ktarg0;
+    int cost[10];
     double coeff[10][10];
     double errfac[19];
     double facmin[10];           /* STEPFAC3^(1 / (2k + 1)) */
@@ -73,8 +73,8 @@ struct BsConsts {
 /* largest kmax */
 #define BS_KMAX 8
 /* dense output: per lane, in HBM, rows of the six components: ysave (9
- * rows), fsave (162: every substep derivative of sequences 0..8, ipoint[9]
- * = 162) and the interpolation coefficients (23); row r of lane g at
+ * rows), fsave (162: every substep derivative of sequences 0..8, sequence k
+ * from row 2 k^2 on) and the interpolation coefficients (23); row r of lane g at
  * ds[(r * nl + g) * 6] */
 #define DS_YSAVE 0
 #define DS_FSAVE 9
@@ -114,17 +114,17 @@ struct BsArgs {
 };
 
 /* StepperBase (src/unused/StepperBS.c:103-149): the step-size sequence
- * (dense output: nseq = 4k+2, else 2(k+1)), costs, k_targ from rtol, the
- * extrapolation coefficients, the dense interpolation error factors and
- * ipoint, where each sequence's derivatives start in fsave */
+ * (dense output: 4k+2, else 2(k+1); bs_nseq in the kernels), costs, k_targ
+ * from rtol, the extrapolation coefficients and the dense interpolation error
+ * factors */
 static void bs_consts(int kmax, double rtol, int dense, BsConsts *c)
 {
     memset(c, 0, sizeof(*c));
     c->kmax = kmax;
-    c->dense = dense;
-    for (int i = 0; i <= kmax; i++) c->nseq[i] = dense ? 4 * i + 2 : 2 * (i + 1);
-    c->cost[0] = c->nseq[0] + 1;
-    for (int k = 0; k < kmax; k++) c->cost[k + 1] = c->cost[k] + c->nseq[k + 1];
+    int nseq[BS_KMAX + 1];
+    for (int i = 0; i <= kmax; i++) nseq[i] = dense ? 4 * i + 2 : 2 * (i + 1);
+    c->cost[0] = nseq[0] + 1;
+    for (int k = 0; k < kmax; k++) c->cost[k + 1] = c->cost[k] + nseq[k + 1];
     double logfact = -log10(rtol > 1.0e-12 ? rtol : 1.0e-12) * 0.6 + 0.5;
     int kt = (int)logfact;
     if (kt > kmax - 1) kt = kmax - 1;
@@ -132,7 +132,7 @@ static void bs_consts(int kmax, double rtol, int dense, BsConsts *c)
     c->ktarg0 = kt;
     for (int k = 0; k <= kmax; k++)
         for (int l = 0; l < k; l++) {
-            double ratio = (double)c->nseq[k] / c->nseq[l];
+            double ratio = (double)nseq[k] / nseq[l];
             c->coeff[k][l] = 1.0 / (ratio * ratio - 1.0);
         }
     for (int i = 0; i < 2 * (kmax + 1) + 1; i++) {
@@ -142,12 +142,6 @@ static void bs_consts(int kmax, double rtol, int dense, BsConsts *c)
         for (int j = 0; j <= i; j++) c->errfac[i] *= e / (j + 1);
     }
     for (int k = 0; k <= kmax; k++) c->facmin[k] = tp_pow(BS_STEPFAC3, 1.0 / (2 * k + 1));
-    c->ipoint[0] = 0;
-    for (int i = 1; i <= kmax + 1; i++) {
-        int njadd = 4 * i - 2;
-        if (c->nseq[i - 1] > njadd) njadd++;
-        c->ipoint[i] = c->ipoint[i - 1] + njadd;
-    }
 }
 
 /* the right-hand side from the field e at the point y */
@@ -162,15 +156,6 @@ __device__ __forceinline__ void bs_deriv(const Emf &e, double qm, const double *
     dy[3] = qm * (e.ex + (vy * e.bz - vz * e.by));
     dy[4] = qm * (e.ey + (vz * e.bx - vx * e.bz));
     dy[5] = qm * (e.ez + (vx * e.by - vy * e.bx));
-}
-
-template <int FK>
-__device__ __forceinline__ void bs_rhs(const FieldDev &f, double qm, double t, const double *y,
-                                       double *dy)
-{
-    Emf e;
-    get_emf64<FK>(f, y[0], y[1], y[2], t, e);
-    bs_deriv(e, qm, y, dy);
 }
 
 /* per-lane state of one particle's integration */
@@ -311,7 +296,7 @@ __device__ __forceinline__ void bs_finish(const BsArgs &a, BsLane &L, int failed
     L.pi = -1;
 }
 
-/* step number of row k: bs_consts' nseq */
+/* step number of row k */
 template <bool DENSE>
 __device__ __forceinline__ int bs_nseq(int k)
 {
@@ -569,7 +554,7 @@ constexpr double bs_const_pow(double x, int e)
 }
 
 /* sequence KK's derivative rows (offsets o in the sequence; row 0 of the
- * sequence is row 2 KK^2 of fsave, ipoint for nseq = 4k + 2), from order KMI
+ * sequence is row 2 KK^2 of fsave), from order KMI
  * on: the value order KMI takes, then the differences between orders
  * (src/unused/StepperBS.c:558-601) */
 template <int KK, int KMI>

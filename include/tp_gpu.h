@@ -286,6 +286,14 @@ int tp_gpu_track_fixed_traj(tp_ctx *ctx, const tp_track_params *p, int n,
 int tp_gpu_load_particles(tp_ctx *ctx, int n, const tp_particle *ptl,
                           const tp_particle *ptl_init);
 int tp_gpu_run_fixed(tp_ctx *ctx, const tp_track_params *p);
+/* Particles and step counts (may be NULL) back to the host; returns when they
+ * are there.  8 MiB of particles (95,326) and more into pageable memory go
+ * through pinned host memory that the context allocates at its first such call
+ * (4 MiB, or 8 MiB from 16 MiB of particles on) and keeps until
+ * tp_gpu_finalize, with three host threads that the call starts and joins.
+ * Into pinned, managed or device memory, and where the pinned memory cannot be
+ * had, the copy is a direct one, which allocates nothing here and starts no
+ * thread; where threads cannot be started, the caller's does their part. */
 int tp_gpu_store_particles(tp_ctx *ctx, tp_particle *ptl, int *nsteps);
 int tp_gpu_read_diagnostics(tp_ctx *ctx, double *espect,
                             double *espect_escape, double *dcoeff,

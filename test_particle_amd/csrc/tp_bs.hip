@@ -1195,8 +1195,8 @@ static int bs_ensure_ctr(tp_ctx *c)
  * wavefront's particles in steps of 16 (modes_wave64), so wavefronts take 32
  * or 16 as long as that still leaves at most one for each SIMD, which is what
  * the kernels' registers allow to run at a time: 30,000 particles, 200 modes,
- * dense form, 64 / 32 / 16 lanes: 32.0 / 23.1 / 28.8 ms (16 lanes take two
- * rounds).  The other fields cost a wavefront the same however many of its
+ * dense form, 64 / 32 / 16 lanes: 32.0 / 23.1 / 28.8 ms of kernels (16 lanes take
+ * two rounds).  The other fields cost a wavefront the same however many of its
  * lanes are in use. */
 static int bs_lanes(const tp_ctx *c, int wpc, int n)
 {
@@ -1239,7 +1239,7 @@ static dim3 bs_grid(const tp_ctx *c, int block, int wpc, int n, int lanes)
 /* The mode table goes to LDS when the copies of the blocks that share a
  * compute unit fit: its reads then take some 100 cycles instead of those of an
  * L2 hit, which a wavefront alone on its SIMD waits for (131,072 particles, 1000
- * modes, 0.3 gyroperiods: 22.9 -> 20.5 ms of kernels).  The kernels' registers
+ * modes, 0.3 gyroperiods: 11 % of the kernel's time).  The kernels' registers
  * leave room for four wavefronts a compute unit, whatever is launched, and a
  * block has the constants and the points of four wavefronts beside its copy.  A
  * block's copy is at most 64 KiB (1008 modes).  Returns the launch's dynamic

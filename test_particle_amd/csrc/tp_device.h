@@ -1025,8 +1025,8 @@ __device__ __forceinline__ void get_emf64(const FieldDev &f, double x, double y,
  * Bound: FP64 issue, 17 operations of the cosine and two 16-cycle products
  * per 4 modes x 16 points (FP64 products and vector FMAs share one unit).
  * Measured in k_bs, where many lanes of a wavefront are idle at any time:
- * 131,072 particles, 1000 modes, 0.3 gyroperiods 47.4 -> 22 ms together with
- * the cheaper cosine; in a loop over full wavefronts, four per SIMD, the
+ * kernel time of 131,072 particles, 1000 modes, 0.3 gyroperiods 47.4 -> 21.4 ms
+ * together with the cheaper cosine and the tableau's constant indices; in a loop over full wavefronts, four per SIMD, the
  * cosine alone gives 150 -> 119 cycles per 64 points and mode and the matrix
  * cores 114. */
 #define MODES_WAVE_LDS (64 * 4)      /* doubles of LDS per wavefront */
